@@ -25,8 +25,8 @@
 //    step (HBM-bound: read and write hidden * 2 bytes per token);
 //  * gather_rows_kernel: dst[i] = src[rows[i]] (the backward's vision rows;
 //    rows[i] < 0 gives a zero row);
-//  * emb_prep_kernel, emb_sum_kernel: the embedding table's gradient
-//    (below).
+//  * emb_prep_kernel, emb_sum_kernel, emb_hot_kernel: the embedding table's
+//    gradient (below).
 #include <algorithm>
 
 #include "splice.h"
@@ -286,8 +286,17 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const bf16* __restrict
 //  * emb_sum_kernel: one wave per sorted key; the wave of the first key of an
 //    id in the first chunk that holds the id sums the id's runs over that
 //    chunk and the later ones (chunks are in position order, so the
-//    concatenation is the stable order) and writes the row; every other wave
-//    returns at once.
+//    concatenation is the stable order) and writes the row, if they are one
+//    partial sum (at most kRowsPerPartial tokens); every other wave returns at
+//    once, and the wave of an id with more tokens puts it on the hot list;
+//  * emb_hot_kernel: the ids of the hot list, a workgroup per (id, column
+//    block).  The partial sums of an id are independent, so the sixteen waves
+//    form one each, all its rows in flight, and the workgroup adds them in
+//    order.  Token ids are Zipf-distributed (the commonest id of 12288 text
+//    tokens comes about 700 times), and one wave adding those rows one after
+//    the other waited for memory at each of them: 1065 us of the 1.24 ms that
+//    the splice's forward and backward took at 16384 tokens x 1536; with the
+//    hot list emb_sum takes 27 us and emb_hot 36 us.
 constexpr int kEmbChunk = 2048;  // two keys per thread of a 1024-thread workgroup
 constexpr int kRowsPerPartial = 10;
 
@@ -298,8 +307,9 @@ static_assert(kEmbChunk == 2 * 1024, "one compare-exchange pair per thread and s
 __global__ __launch_bounds__(1024) void emb_prep_kernel(const int64_t* __restrict__ ids, int64_t n, int64_t vocab,
                                                         int64_t skip0, int64_t skip1, uint64_t* __restrict__ keys,
                                                         int2* __restrict__ seg, int nch, u32x4* __restrict__ dw,
-                                                        int64_t dw16) {
+                                                        int64_t dw16, int* __restrict__ nhot) {
   __shared__ uint64_t sk[kEmbChunk];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *nhot = 0;
   const u32x4 z = {0u, 0u, 0u, 0u};
   if ((int)blockIdx.x >= nch) {
     const int64_t stride = (int64_t)(gridDim.x - nch) * 1024;
@@ -353,10 +363,10 @@ struct Vec16;
 template <>
 struct Vec16<bf16> {
   static constexpr int E = 8;
-  __device__ static void load(const bf16* p, float (&x)[8]) {
-    const bf16x8 v = ld_bf16x8(p);
+  typedef bf16x8 Raw;
+  __device__ static void add(float (&x)[8], const Raw& v) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = (float)v[i];
+    for (int i = 0; i < 8; ++i) x[i] += (float)v[i];
   }
   __device__ static void store(bf16* p, const float (&x)[8]) {
     bf16x8 v;
@@ -368,96 +378,194 @@ struct Vec16<bf16> {
 template <>
 struct Vec16<float> {
   static constexpr int E = 4;
-  __device__ static void load(const float* p, float (&x)[4]) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(p);
+  typedef f32x4 Raw;
+  __device__ static void add(float (&x)[4], const Raw& v) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = v[i];
+    for (int i = 0; i < 4; ++i) x[i] += v[i];
   }
   __device__ static void store(float* p, const float (&x)[4]) {
     *reinterpret_cast<f32x4*>(p) = f32x4{x[0], x[1], x[2], x[3]};
   }
 };
 
-// U 16-byte chunks of the row per lane and pass: every token's row is read
-// once per pass, its U loads in flight together.
+// An id whose tokens make more than one partial sum: first chunk c that holds it.
+struct HotId {
+  uint32_t v;
+  int c;
+};
+
+// The id's runs in chunks c .. c + 63 are read one per lane.  R rows x U
+// 16-byte chunks per lane are in flight together.
 template <typename T>
 __global__ __launch_bounds__(256) void emb_sum_kernel(const T* __restrict__ grad, const uint64_t* __restrict__ keys,
                                                       const int2* __restrict__ seg, int nchunks, int64_t vocab,
-                                                      int64_t hidden, T* __restrict__ dw) {
+                                                      int64_t hidden, T* __restrict__ dw, HotId* __restrict__ hot,
+                                                      int* __restrict__ nhot) {
   using V = Vec16<T>;
-  constexpr int E = V::E, U = 4;
-  const int lane = threadIdx.x & 63;
-  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int E = V::E, U = 4, R = 4;
+  __shared__ uint32_t tok_sh[4][kRowsPerPartial];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t item = (int64_t)blockIdx.x * 4 + wv;
   if (item >= (int64_t)nchunks * kEmbChunk) return;
   const int c = (int)(item / kEmbChunk), i = (int)(item % kEmbChunk);
   const uint64_t key = keys[item];
   if (key == ~0ull) return;
   const uint32_t v = (uint32_t)(key >> 32);
   if (i > 0 && (uint32_t)(keys[item - 1] >> 32) == v) return;  // not the first key of its id in this chunk
-  // the id's runs in chunks c .. c + 63 (lane l: chunk c + l), one load per lane; an earlier chunk holding the
-  // id means its wave writes the row
+  // an earlier chunk holding the id means its wave writes the row
   for (int c0 = 0; c0 < c; c0 += 64) {
     const int cc = c0 + lane;
     int2 r = make_int2(0, 0);
     if (cc < c) r = seg[(int64_t)cc * vocab + v];
     if (__ballot(r.y > r.x)) return;
   }
+  // the id's tokens (a wave's own LDS row: its writes and reads run in order)
+  int cnt = 0;
+  for (int g0 = c; g0 < nchunks && cnt <= kRowsPerPartial; g0 += 64) {
+    int2 mine = make_int2(0, 0);
+    if (g0 + lane < nchunks) mine = seg[(int64_t)(g0 + lane) * vocab + v];
+    const int len = mine.y - mine.x;
+    int incl = len;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    const int at = cnt + incl - len;
+    for (int t = 0; t < len && at + t < kRowsPerPartial; ++t)
+      tok_sh[wv][at + t] = (uint32_t)((g0 + lane) * kEmbChunk) + (uint32_t)keys[(int64_t)(g0 + lane) * kEmbChunk + mine.x + t];
+    cnt += __shfl(incl, 63);
+  }
+  if (cnt > kRowsPerPartial) {
+    if (lane == 0) hot[atomicAdd(nhot, 1)] = HotId{v, c};
+    return;
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // the token list is in LDS
   const int64_t nvec = hidden / E;
   for (int64_t p0 = 0; p0 < nvec; p0 += 64 * U) {
-    float tot[U][E], part[U][E];
+    float part[U][E];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int e = 0; e < E; ++e) tot[u][e] = part[u][e] = 0.f;
-    int cnt = 0;
-    for (int g0 = c; g0 < nchunks; g0 += 64) {
-      int2 mine = make_int2(0, 0);
-      if (g0 + lane < nchunks) mine = seg[(int64_t)(g0 + lane) * vocab + v];
-      const int ng = min(64, nchunks - g0);
-      for (int q = 0; q < ng; ++q) {
-        const int cc = g0 + q;
-        const int rb = __shfl(mine.x, q), re = __shfl(mine.y, q);
-        const uint64_t* kc = keys + (int64_t)cc * kEmbChunk;
-        for (int t = rb; t < re; ++t) {
-          const T* src = grad + ((int64_t)cc * kEmbChunk + (uint32_t)kc[t]) * hidden;
-          float x[U][E];
+      for (int e = 0; e < E; ++e) part[u][e] = 0.f;
+    for (int t0 = 0; t0 < cnt; t0 += R) {
+      typename V::Raw x[R][U];
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int64_t ch = p0 + 64 * u + lane;
-            if (ch < nvec) {
-              V::load(src + ch * E, x[u]);
-            } else {
+      for (int r = 0; r < R; ++r) {
+        if (t0 + r >= cnt) break;
+        const T* src = grad + (int64_t)tok_sh[wv][t0 + r] * hidden;
 #pragma unroll
-              for (int e = 0; e < E; ++e) x[u][e] = 0.f;
-            }
-          }
+        for (int u = 0; u < U; ++u) {
+          const int64_t ch = p0 + 64 * u + lane;
+          if (ch < nvec) x[r][u] = *reinterpret_cast<const typename V::Raw*>(src + ch * E);
+        }
+      }
 #pragma unroll
-          for (int u = 0; u < U; ++u)
+      for (int r = 0; r < R; ++r) {
+        if (t0 + r >= cnt) break;
 #pragma unroll
-            for (int e = 0; e < E; ++e) part[u][e] += x[u][e];
-          if (++cnt == kRowsPerPartial) {
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-              for (int e = 0; e < E; ++e) {
-                tot[u][e] += part[u][e];
-                part[u][e] = 0.f;
-              }
-            cnt = 0;
-          }
+        for (int u = 0; u < U; ++u) {
+          if (p0 + 64 * u + lane < nvec) V::add(part[u], x[r][u]);
         }
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t ch = p0 + 64 * u + lane;
-      if (ch >= nvec) continue;
-      if (cnt > 0) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) tot[u][e] += part[u][e];
-      }
-      V::store(dw + (int64_t)v * hidden + ch * E, tot[u]);
+      if (ch < nvec) V::store(dw + (int64_t)v * hidden + ch * E, part[u]);
     }
+  }
+}
+
+// One hot id and one block of 64 E columns per workgroup (ids strided over
+// gridDim.x).  Rounds of kHotWaves partial sums: the workgroup lists the
+// round's tokens in LDS (one thread per token), wave w sums rows
+// kRowsPerPartial w .. of the round in order, and thread j adds the round's
+// partial sums of column j in order to its running total.
+constexpr int kHotWaves = 16, kHotRound = kHotWaves * kRowsPerPartial;
+template <typename T>
+__global__ __launch_bounds__(64 * kHotWaves) void emb_hot_kernel(const T* __restrict__ grad,
+                                                                 const uint64_t* __restrict__ keys,
+                                                                 const int2* __restrict__ seg, int nchunks,
+                                                                 int64_t vocab, int64_t hidden, T* __restrict__ dw,
+                                                                 const HotId* __restrict__ hot,
+                                                                 const int* __restrict__ nhot) {
+  using V = Vec16<T>;
+  constexpr int E = V::E, COLS = 64 * E;
+  static_assert(COLS <= 64 * kHotWaves, "a thread per column");
+  __shared__ uint32_t tok_sh[kHotRound];
+  __shared__ float part_sh[kHotWaves][COLS];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t nvec = hidden / E, ch = (int64_t)blockIdx.y * 64 + lane;
+  const int64_t col = (int64_t)blockIdx.y * COLS + tid;
+  const int n = *nhot;
+  for (int k = blockIdx.x; k < n; k += gridDim.x) {
+    const uint32_t v = hot[k].v;
+    int g0 = hot[k].c;  // chunks g0 .. g0 + 63: lane l holds chunk g0 + l's run, every wave alike
+    int rank0 = 0;      // tokens of the group's runs listed so far
+    int first, incl, total;
+    auto group = [&]() {
+      int2 mine = make_int2(0, 0);
+      if (g0 + lane < nchunks) mine = seg[(int64_t)(g0 + lane) * vocab + v];
+      first = mine.x;
+      incl = mine.y - mine.x;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+      }
+      total = __shfl(incl, 63);
+    };
+    group();
+    float tot = 0.f;
+    for (;;) {
+      int have = 0;
+      for (;;) {
+        // token rank0 + tid of the group: in the first chunk whose inclusive count exceeds it
+        const int take = min(total - rank0, kHotRound - have);
+        const int rank = rank0 + tid;
+        int q = 0, base = 0;
+        for (int j = 0; j < 64 && g0 + j < nchunks; ++j) {
+          const int upto = __builtin_amdgcn_readlane(incl, j);
+          q = upto <= rank ? j + 1 : q;
+          base = upto <= rank ? upto : base;
+        }
+        const int at = __shfl(first, q & 63) + rank - base;
+        if (tid < take)
+          tok_sh[have + tid] = (uint32_t)((g0 + q) * kEmbChunk) + (uint32_t)keys[(int64_t)(g0 + q) * kEmbChunk + at];
+        have += take;
+        rank0 += take;
+        if (have == kHotRound || g0 + 64 >= nchunks) break;
+        g0 += 64;
+        rank0 = 0;
+        group();
+      }
+      __syncthreads();
+      if (have == 0) break;
+      const int r0 = wv * kRowsPerPartial, nr = min(kRowsPerPartial, have - r0);
+      if (nr > 0 && ch < nvec) {
+        typename V::Raw x[kRowsPerPartial];
+        float part[E];
+#pragma unroll
+        for (int r = 0; r < kRowsPerPartial; ++r)  // rows past the last one re-read it
+          x[r] = *reinterpret_cast<const typename V::Raw*>(grad + (int64_t)tok_sh[r0 + min(r, nr - 1)] * hidden + ch * E);
+#pragma unroll
+        for (int e = 0; e < E; ++e) part[e] = 0.f;
+#pragma unroll
+        for (int r = 0; r < kRowsPerPartial; ++r)
+          if (r < nr) V::add(part, x[r]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) part_sh[wv][lane * E + e] = part[e];
+      }
+      __syncthreads();
+      const int np = (have + kRowsPerPartial - 1) / kRowsPerPartial;
+      if (tid < COLS && col < hidden)
+        for (int w = 0; w < np; ++w) tot += part_sh[w][tid];
+      // the next round's list does not touch part_sh, and its barrier comes before the next partial sums
+    }
+    if (tid < COLS && col < hidden) dw[(int64_t)v * hidden + col] = (T)tot;
+    __syncthreads();  // part_sh and tok_sh are read no more
   }
 }
 
@@ -484,31 +592,60 @@ hipError_t splice_fwd(const SpliceArgs& a, int32_t* image_pos, int64_t* counts, 
   return hipGetLastError();
 }
 
-size_t embedding_bwd_workspace_bytes(int64_t n, int64_t vocab) {
-  const int64_t nch = n > 0 ? (n + kEmbChunk - 1) / kEmbChunk : 0;
-  const size_t keys = (size_t)nch * kEmbChunk * sizeof(uint64_t);
-  const size_t runs = ((size_t)nch * (size_t)vocab * sizeof(int2) + 15) & ~size_t(15);
-  return ((keys + 255) & ~size_t(255)) + runs + 256;
+namespace {
+// workspace of the table gradient: sorted keys, run table, hot list (ids with
+// more than kRowsPerPartial tokens: at most n / (kRowsPerPartial + 1)) and its length
+struct EmbLayout {
+  int64_t nch;
+  size_t runs, hot, nhot, total;
+};
+EmbLayout emb_layout(int64_t n, int64_t vocab) {
+  EmbLayout L;
+  L.nch = n > 0 ? (n + kEmbChunk - 1) / kEmbChunk : 0;
+  auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
+  L.runs = al((size_t)L.nch * kEmbChunk * sizeof(uint64_t));
+  L.hot = L.runs + al((size_t)L.nch * (size_t)vocab * sizeof(int2));
+  L.nhot = L.hot + al((size_t)(n > 0 ? n / (kRowsPerPartial + 1) + 1 : 1) * sizeof(HotId));
+  L.total = L.nhot + 256;
+  return L;
 }
+
+template <typename T>
+void launch_emb_sums(const void* grad, const uint64_t* keys, const int2* seg, int nch, int64_t vocab, int64_t hidden,
+                     void* dw, HotId* hot, int* nhot, hipStream_t stream) {
+  const T* g = static_cast<const T*>(grad);
+  T* out = static_cast<T*>(dw);
+  const unsigned blocks = (unsigned)(((int64_t)nch * kEmbChunk + 3) / 4);
+  hipLaunchKernelGGL(emb_sum_kernel<T>, dim3(blocks), dim3(256), 0, stream, g, keys, seg, nch, vocab, hidden, out, hot,
+                     nhot);
+  // an id needs more than kRowsPerPartial tokens to be hot
+  const unsigned ids = (unsigned)std::min<int64_t>((int64_t)nch * kEmbChunk / (kRowsPerPartial + 1), 128);
+  const unsigned cols = (unsigned)((hidden / Vec16<T>::E + 63) / 64);
+  hipLaunchKernelGGL(emb_hot_kernel<T>, dim3(ids, cols), dim3(64 * kHotWaves), 0, stream, g, keys, seg, nch, vocab, hidden,
+                     out, hot, nhot);
+}
+}  // namespace
+
+size_t embedding_bwd_workspace_bytes(int64_t n, int64_t vocab) { return emb_layout(n, vocab).total; }
 
 hipError_t embedding_bwd(const void* grad, const int64_t* ids, int64_t n, int64_t vocab, int64_t hidden, bool fp32,
                          int64_t skip0, int64_t skip1, void* dw, void* ws, hipStream_t stream) {
-  const int nch = n > 0 ? (int)((n + kEmbChunk - 1) / kEmbChunk) : 0;
-  const size_t keys_bytes = ((size_t)nch * kEmbChunk * sizeof(uint64_t) + 255) & ~size_t(255);
-  uint64_t* keys = static_cast<uint64_t*>(ws);
-  int2* seg = reinterpret_cast<int2*>(static_cast<char*>(ws) + keys_bytes);
+  const EmbLayout L = emb_layout(n, vocab);
+  const int nch = (int)L.nch;
+  char* base = static_cast<char*>(ws);
+  uint64_t* keys = reinterpret_cast<uint64_t*>(base);
+  int2* seg = reinterpret_cast<int2*>(base + L.runs);
+  HotId* hot = reinterpret_cast<HotId*>(base + L.hot);
+  int* nhot = reinterpret_cast<int*>(base + L.nhot);
   const int64_t dw16 = vocab * hidden * (fp32 ? 4 : 2) / 16;  // hidden % 8 == 0
   const int clear_blocks = (int)std::min<int64_t>((dw16 + 1023) / 1024, 512);
   hipLaunchKernelGGL(emb_prep_kernel, dim3((unsigned)(nch + std::max(clear_blocks, 1))), dim3(1024), 0, stream, ids, n,
-                     vocab, skip0, skip1, keys, seg, nch, static_cast<u32x4*>(dw), dw16);
+                     vocab, skip0, skip1, keys, seg, nch, static_cast<u32x4*>(dw), dw16, nhot);
   if (nch > 0) {
-    const unsigned blocks = (unsigned)(((int64_t)nch * kEmbChunk + 3) / 4);
     if (fp32)
-      hipLaunchKernelGGL(emb_sum_kernel<float>, dim3(blocks), dim3(256), 0, stream, static_cast<const float*>(grad),
-                         keys, seg, nch, vocab, hidden, static_cast<float*>(dw));
+      launch_emb_sums<float>(grad, keys, seg, nch, vocab, hidden, dw, hot, nhot, stream);
     else
-      hipLaunchKernelGGL(emb_sum_kernel<bf16>, dim3(blocks), dim3(256), 0, stream, static_cast<const bf16*>(grad), keys,
-                         seg, nch, vocab, hidden, static_cast<bf16*>(dw));
+      launch_emb_sums<bf16>(grad, keys, seg, nch, vocab, hidden, dw, hot, nhot, stream);
   }
   return hipGetLastError();
 }

@@ -307,3 +307,29 @@ def test_tiny_vlm_all_fused_vs_fp32():
         worst = max(worst, r)
         assert r <= 5e-2, (n, r)
     print(f"  worst parameter-gradient relative error {worst:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden", [8, 520, 1536])
+def test_table_gradient_of_frequent_ids_keeps_the_stated_order(hidden, dtype):
+    """Ids with 1 .. 2500 tokens (one partial sum of ten rows, one row more,
+    whole and broken rounds of sixteen partial sums, runs over several
+    2048-token chunks): bitwise the fp32 sums in the stated order (tokens in
+    position order, partial sums of at most ten rows added in order)."""
+    print(f"table gradient, frequent ids, hidden={hidden} {dtype}", flush=True)
+    counts = [1, 9, 10, 11, 20, 21, 159, 160, 161, 320, 331, 2500]
+    vocab = len(counts) + 3
+    ids = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)] + [torch.full((300,), len(counts) + 1)])
+    g = torch.Generator().manual_seed(hidden)
+    ids = ids[torch.randperm(ids.numel(), generator=g)]
+    grad = torch.randn(ids.numel(), hidden, generator=g).to(dtype)
+    got = S.embedding_bwd(grad.to(DEV), ids.to(DEV), vocab, (len(counts) + 1,)).cpu()
+    for v in range(vocab):
+        rows = grad[ids == v].float() if v != len(counts) + 1 else grad[:0].float()
+        tot = torch.zeros(hidden)
+        for a in range(0, rows.shape[0], 10):
+            part = torch.zeros(hidden)
+            for r in rows[a:a + 10]:
+                part = part + r
+            tot = tot + part
+        assert torch.equal(got[v], tot.to(dtype)), f"id {v}"
