@@ -63,20 +63,20 @@ struct LogitsArgs {
 };
 
 __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
-  __shared__ __align__(16) bf16 smem[4 * SLAB];
+  __shared__ __align__(16) bf16 smem[SMEM];
   int ti, tj;
   if (!tile_of(p.nI, p.nJ, 4, ti, tj)) return;
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
   if (j0 >= *p.nvalid - p.c0) return;  // token tile holds no valid row
   f32x16 acc[4][2];
-  gemm_core<true, true, true>(smem, p.W, p.H, i0, j0, 0, p.W.cols, acc);
+  gemm_core<true, true, false>(smem, p.W, p.H, i0, j0, 0, p.W.cols, acc);
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int wi = w & 1, wj = w >> 1;
   float* red = reinterpret_cast<float*>(smem);  // [2][256]
-  // accumulator (a, b, r) holds z for vocab row vbase + 32 a + 16 (r / 8) + (r % 8) and token column
+  // accumulator (a, b, r) holds z for vocab row vbase + wave_row(a, wi) + 16 (r / 8) + (r % 8) and token
   // j0 + 64 wj + 32 b + l32.  Only the last vocab tile has rows past V: masked there alone.
-  const int64_t vbase = i0 + 128 * wi + 8 * h;
+  const int64_t vbase = i0 + 8 * h;
   if (i0 + BI > p.V) {
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (vbase + 32 * a + 16 * (r >> 3) + (r & 7) >= p.V) acc[a][b][r] = -INFINITY;
+          if (vbase + wave_row(a, wi) + 16 * (r >> 3) + (r & 7) >= p.V) acc[a][b][r] = -INFINITY;
   }
   float mt[2];
 #pragma unroll
@@ -96,32 +96,32 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc[a][b][r]);
     // tile max in log2 units (scaling by log2 e > 0 commutes with the max)
     mx = wave_max_xor32(mx) * kLog2e;
-    if (h == 0) red[wi * 256 + 64 * wj + 32 * b + l32] = mx;
+    if (h == 0) red[wi * 256 + wave_col(b, wj) + l32] = mx;
   }
   __syncthreads();
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int col = 64 * wj + 32 * b + l32;
+    const int col = wave_col(b, wj) + l32;
     mt[b] = fmaxf(red[col], red[256 + col]);
   }
   __syncthreads();
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int col = 64 * wj + 32 * b + l32;
+    const int col = wave_col(b, wj) + l32;
     const int64_t tok = j0 + col;
     const bool tv = tok < p.nc;
     // the label logit: held by at most one lane of the workgroup, for one
     // vocab tile in ~600 -- located with one range test per token
     const int64_t rel64 = (tv ? p.y[tok] : -1) - vbase;
-    const bool hit = rel64 >= 0 && rel64 < 128 && ((rel64 >> 3) & 1) == 0;
+    const bool hit = rel64 >= 0 && rel64 < 256 && ((rel64 >> 6) & 1) == wi && ((rel64 >> 3) & 1) == 0;
     if (__any(hit)) {
-      const int rel = (int)rel64;
+      const int rel = (int)rel64 - 64 * wi;
       float zsel = 0.f;
 #pragma unroll
       for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (hit && rel == 32 * a + 16 * (r >> 3) + (r & 7)) zsel = acc[a][b][r];
+          if (hit && rel == wave_row(a, 0) + 16 * (r >> 3) + (r & 7)) zsel = acc[a][b][r];
       if (hit) p.zy[tok] = zsel;
     }
     const float m2 = mt[b];
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
     for (int a = 0; a < 4; ++a) {
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
-        const int64_t v0 = vbase + 32 * a + 16 * jj;
+        const int64_t v0 = vbase + wave_row(a, wi) + 16 * jj;
         bf16x8 e8;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
   if (wi == 0 && h == 0) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int col = 64 * wj + 32 * b + l32;
+      const int col = wave_col(b, wj) + l32;
       const int64_t tok = j0 + col;
       if (tok < p.nc) {
         p.mpart[tok * p.nvt + ti] = mt[b];
@@ -290,7 +290,7 @@ __device__ __forceinline__ bool dh_tile_of(int nI, int nJ, int splits, int& ti, 
 }
 
 __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
-  __shared__ __align__(16) bf16 smem[4 * SLAB];
+  __shared__ __align__(16) bf16 smem[SMEM];
   int ti, tj, split;
   if (!dh_tile_of(p.nI, p.nJ, p.splits, ti, tj, split)) return;
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
@@ -299,12 +299,12 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
   const int64_t kb = split * p.kper;
   const int64_t ke = min(p.E.cols, kb + p.kper);
   f32x16 acc[4][2];
-  gemm_core<false, true>(smem, p.Wt, p.E, i0, j0, kb, ke, acc);
+  gemm_core<false, true, true>(smem, p.Wt, p.E, i0, j0, kb, ke, acc);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int wi = w & 1, wj = w >> 1;
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int64_t tok = j0 + 64 * wj + 32 * b + l32;
+    const int64_t tok = j0 + wave_col(b, wj) + l32;
     if (tok >= p.nc) continue;
     if (p.splits == 1 && tok >= nv) continue;  // padding row
     const int64_t orow = p.splits == 1 ? p.rows[p.c0 + tok] : 0;
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
-        const int64_t hh = i0 + 128 * wi + 32 * a + 16 * jj + 8 * h;
+        const int64_t hh = i0 + wave_row(a, wi) + 16 * jj + 8 * h;
         if (hh >= p.hdim) continue;
         if (p.splits == 1) {
           bf16x8 o;
@@ -373,7 +373,7 @@ struct DwArgs {
 };
 
 __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
-  __shared__ __align__(16) bf16 smem[4 * SLAB];
+  __shared__ __align__(16) bf16 smem[SMEM];
   int ti, tj;
   if (!tile_of(p.nI, p.nJ, p.nI, ti, tj)) return;
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
@@ -396,18 +396,18 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
   const int64_t nv = nvt_all - p.c0;
   const int64_t ke = min(p.Ht.rows, nv > 0 ? ((nv + BK - 1) / BK) * BK : (int64_t)0);
   f32x16 acc[4][2];
-  gemm_core<false, false>(smem, p.Ht, p.Et, i0, j0, 0, ke, acc);
+  gemm_core<false, false, true>(smem, p.Ht, p.Et, i0, j0, 0, ke, acc);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int wi = w & 1, wj = w >> 1;
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int64_t v = j0 + 64 * wj + 32 * b + l32;
+    const int64_t v = j0 + wave_col(b, wj) + l32;
     if (v >= p.V) continue;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
-        const int64_t hh = i0 + 128 * wi + 32 * a + 16 * jj + 8 * h;
+        const int64_t hh = i0 + wave_row(a, wi) + 16 * jj + 8 * h;
         if (hh >= p.hdim) continue;
         f32x4 lo, hi;
 #pragma unroll

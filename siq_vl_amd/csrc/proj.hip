@@ -59,59 +59,66 @@ struct Shuffle {
   }
 };
 
-// Xs as a k-contiguous operand (slab rows = shuffled tokens j0 + row,
+// Xs as a k-contiguous operand (half rows = shuffled tokens j0 + 128 half + row,
 // 64 features per k-step, inside one (i, j) segment since dv % 64 == 0): the
-// layout of SlabLoad<true>, with each row's x address from the shuffle.
+// layout of OpLoad<true>, with each row's x address from the shuffle.
 struct GatherKC {
   const bf16* x;
   Shuffle sh;
-  uint32_t rowoff[4];  // per instruction: xrow(token) * dv + the lane's swizzled chunk
+  uint32_t off[2][2];  // [half][q]: byte offset of xrow(token) * dv + the lane's swizzled chunk
   __device__ __forceinline__ void init(const bf16* xp, const Shuffle& s, int64_t j0, int lane, int w) {
     x = xp;
     sh = s;
-    const int lrow = lane / 8, lpc = lane % 8;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = 32 * w + 8 * q + lrow;
-      const int tok = min((int)j0 + row, s.m - 1);  // rows past the end re-read the last token (never stored)
-      rowoff[q] = (uint32_t)(s.xrow(tok) * s.dv + 8 * (lpc ^ swz_kc(row)));
-    }
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int row = 16 * w + 8 * q + lane / 8;
+        const int tok = min((int)j0 + 128 * hf + row, s.m - 1);  // rows past the end re-read the last token (never stored)
+        off[hf][q] = 2 * (uint32_t)(s.xrow(tok) * s.dv + 8 * ((lane % 8) ^ swz_kc(row)));
+      }
   }
-  __device__ __forceinline__ void issue(int64_t k0, bf16* lds, int wu) const {
-    const uint32_t delta = (uint32_t)sh.featoff((int)k0);
+  __device__ __forceinline__ void issue(int hf, int64_t k0, bf16* lds, int wu) const {
+    const bf16* b = x + sh.featoff((int)k0);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) dma16(x, rowoff[q] + delta, lds + (wu * 4 + q) * 512);
+    for (int q = 0; q < 2; ++q) dma16(b, off[hf][q], lds + (2 * wu + q) * 512);
   }
 };
 
-// Xs^T as a k-major operand (slab rows = shuffled tokens k0 + row, 256
-// feature columns i0 .. i0 + 255): the layout of SlabLoad<false>.  A lane's
-// chunk columns are fixed per tile; its rows' x addresses are recomputed per
-// k-step.
+// Xs^T as a k-major operand (half rows = shuffled tokens k0 + row, 128 feature
+// columns from i0 + 128 half): the layout of OpLoad<false>.  A lane's chunk
+// columns are fixed per tile; its rows' x addresses are recomputed per k-step,
+// for the lower half, and kept for the upper one (the core issues the halves
+// of a k-step in this order, with no other step's between them).
 struct GatherNKC {
   const bf16* x;
   Shuffle sh;
-  int coloff[4];  // per instruction: offset of the lane's 8 features from the token's row
-  int rr[4];      // per instruction: the lane's slab row
+  uint32_t rowoff[2];  // [q]: the current k-step's row
+  int coloff[2][2];  // [half][q]: offset of the lane's 8 features from the token's row
   __device__ __forceinline__ void init(const bf16* xp, const Shuffle& s, int64_t i0, int lane, int w) {
     x = xp;
     sh = s;
-    const int lrow = lane / 32, lpc = lane % 32;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = 8 * w + 2 * q + lrow;
-      const int col = min((int)i0 + 8 * (lpc ^ swz_nkc(row)), s.k - 8);  // columns past k: never stored
-      coloff[q] = s.featoff(col);
-      rr[q] = row;
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int row = 8 * w + 4 * q + lane / 16;
+        const int col = min((int)i0 + 128 * hf + 8 * ((lane % 16) ^ swz_nkc(row)), s.k - 8);  // columns past k: never stored
+        coloff[hf][q] = s.featoff(col);
+      }
+  }
+  __device__ __forceinline__ void issue(int hf, int64_t k0, bf16* lds, int wu) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (hf == 0) {
+        const int tok = min((int)k0 + 8 * wu + 4 * q + lane / 16, sh.m - 1);  // past the end: multiplied by the zeroed dY tail
+        rowoff[q] = (uint32_t)(sh.xrow(tok) * sh.dv);
+      }
+      dma16(x, 2 * (rowoff[q] + (uint32_t)coloff[hf][q]), lds + (2 * wu + q) * 512);
     }
   }
-  __device__ __forceinline__ void issue(int64_t k0, bf16* lds, int wu) const {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int tok = min((int)k0 + rr[q], sh.m - 1);  // past the end: multiplied by the zeroed dY tail
-      dma16(x, (uint32_t)(sh.xrow(tok) * sh.dv + coloff[q]), lds + (wu * 4 + q) * 512);
-    }
-  }
+  __device__ __forceinline__ void issue_tail(int hf, int64_t k0, int, bf16* lds, int wu, int) { issue(hf, k0, lds, wu); }
 };
 
 struct FwdArgs {
@@ -125,7 +132,7 @@ struct FwdArgs {
 };
 
 __global__ __launch_bounds__(NT) void proj_fwd_kernel(const FwdArgs p) {
-  __shared__ __align__(16) bf16 smem[4 * SLAB];
+  __shared__ __align__(16) bf16 smem[SMEM];
   int ti, tj;
   if (!tile_of(p.nI, p.nJ, p.nI, ti, tj)) return;
   const int split = blockIdx.y;
@@ -137,17 +144,17 @@ __global__ __launch_bounds__(NT) void proj_fwd_kernel(const FwdArgs p) {
   GatherKC lb;
   lb.init(p.x, p.sh, j0, lane, w);
   f32x16 acc[4][2];
-  gemm_core_l<true, true>(smem, la, lb, kb, ke, acc);
+  gemm_core_l<true, true, false>(smem, la, lb, kb, ke, acc);
   const int wi = w & 1, wj = w >> 1;
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int64_t tok = j0 + 64 * wj + 32 * b + l32;
+    const int64_t tok = j0 + wave_col(b, wj) + l32;
     if (tok >= p.sh.m) continue;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
-        const int64_t nn = i0 + 128 * wi + 32 * a + 16 * jj + 8 * h;
+        const int64_t nn = i0 + wave_row(a, wi) + 16 * jj + 8 * h;
         if (nn >= p.n) continue;
         if (p.splits == 1) {
           bf16x8 o;
@@ -178,24 +185,24 @@ struct DxArgs {
 };
 
 __global__ __launch_bounds__(NT) void proj_dx_kernel(const DxArgs p) {
-  __shared__ __align__(16) bf16 smem[4 * SLAB];
+  __shared__ __align__(16) bf16 smem[SMEM];
   int ti, tj;
   if (!tile_of(p.nI, p.nJ, p.nI, ti, tj)) return;
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
   f32x16 acc[4][2];
-  gemm_core<false, true>(smem, p.Wt, p.dY, i0, j0, 0, p.dY.cols, acc);
+  gemm_core<false, true, true>(smem, p.Wt, p.dY, i0, j0, 0, p.dY.cols, acc);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int wi = w & 1, wj = w >> 1;
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int tok = (int)(j0 + 64 * wj + 32 * b + l32);
+    const int tok = (int)(j0 + wave_col(b, wj) + l32);
     if (tok >= p.sh.m) continue;
     bf16* row = p.dx + (int64_t)p.sh.xrow(tok) * p.sh.dv;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
-        const int kf = (int)(i0 + 128 * wi + 32 * a + 16 * jj + 8 * h);
+        const int kf = (int)(i0 + wave_row(a, wi) + 16 * jj + 8 * h);
         if (kf >= p.sh.k) continue;
         bf16x8 o;
 #pragma unroll
@@ -216,7 +223,7 @@ struct DwArgs {
 };
 
 __global__ __launch_bounds__(NT) void proj_dw_kernel(const DwArgs p) {
-  __shared__ __align__(16) bf16 smem[4 * SLAB];
+  __shared__ __align__(16) bf16 smem[SMEM];
   int ti, tj;
   if (!tile_of(p.nI, p.nJ, p.nI, ti, tj)) return;
   const int split = blockIdx.y;
@@ -228,17 +235,17 @@ __global__ __launch_bounds__(NT) void proj_dw_kernel(const DwArgs p) {
   OpLoad<false> lb;
   lb.init(p.dY, j0, lane, w);
   f32x16 acc[4][2];
-  gemm_core_l<false, false>(smem, la, lb, kb, ke, acc);
+  gemm_core_l<false, false, true>(smem, la, lb, kb, ke, acc);
   const int wi = w & 1, wj = w >> 1;
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int64_t nn = j0 + 64 * wj + 32 * b + l32;
+    const int64_t nn = j0 + wave_col(b, wj) + l32;
     if (nn >= p.n) continue;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
-        const int64_t kf = i0 + 128 * wi + 32 * a + 16 * jj + 8 * h;
+        const int64_t kf = i0 + wave_row(a, wi) + 16 * jj + 8 * h;
         if (kf >= p.sh.k) continue;
         if (p.splits == 1) {
           bf16x8 o;

@@ -65,6 +65,25 @@ def test_vs_oracle(case):
     assert ry <= TOL and rdx <= TOL and rdw <= TOL
 
 
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("tail", [0, 8, 56])
+def test_gemm_core_at_few_k_steps(steps, tail):
+    """The GEMM core's prologue, steady state and last steps: 1 .. 5 k-steps of
+    64, without and with a partial one, in each of its three operand
+    orientations (y: k = steps 64; dx: k = n = 64 (steps - 1) + tail; dweight: k
+    = tokens), at one tile and past its edges.  Per element: one bf16 rounding
+    of an fp32 sum, |got - exact| <= 2^-8 |exact| + k 2^-23 sum |a b|."""
+    dv, n, tokens = 64 * steps, 64 * (steps - 1) + (tail or 64), 64 * (steps - 1) + (tail or 64) + 1
+    print(f"projector k-steps {steps} tail {tail}", flush=True)
+    x, w, dy = make(tokens, 1, dv, 1, n, seed=steps)
+    y = P.proj_fwd(x.to(DEV), w.to(DEV), 1).double().cpu().view(tokens, n)
+    dx, dw = (t.double().cpu() for t in P.proj_bwd(x.to(DEV), w.to(DEV), dy.to(DEV), 1))
+    xf, wf, gf = x.double().view(tokens, dv), w.double(), dy.double().view(tokens, n)
+    for got, a, b in ((y, xf, wf.T), (dx.view(tokens, dv), gf, wf), (dw, gf.T, xf)):
+        exact, mag = a @ b, a.abs() @ b.abs()
+        assert bool(((got - exact).abs() <= 2**-8 * exact.abs() + a.shape[1] * 2**-23 * mag).all())
+
+
 def test_repeat_is_bitwise():
     x, w, dy = (t.to(DEV) for t in make(16, 16, 256, 2, 512, seed=1))
     a = (P.proj_fwd(x, w, 2), *P.proj_bwd(x, w, dy, 2))
