@@ -17,24 +17,24 @@
 //    of 64 rows are double-buffered row-major in LDS and taken 32 rows at a
 //    time (operand reads one k-step ahead of the MFMAs); dQ^T += K^T dS^T reads
 //    K^T with ds_read_b64_tr_b16.
-//  * dK/dV (D = 128, and the atomic backward): one workgroup = 8 waves =
-//    128 kv rows of one kv-head.  Wave
-//    (g, kq) owns kv rows 32 kq .. 32 kq + 31 and q rows 32 g .. 32 g + 31 of
-//    each 64-row step, so every staged Q / dO tile feeds all 128 kv rows and
-//    every SIMD runs two waves.  K and V of the tile sit in LDS as the B
-//    operands of S = Q K^T and dP = dO V^T.  A work item walks steps (q block,
-//    q-head of the GQA group) of its kv tile, with Q / dO / LSE2 / Delta
-//    double-buffered in LDS by direct global->LDS loads and the operand reads
-//    one k-step ahead of the MFMAs; dV^T += dO^T P and dK^T += Q^T dS read
-//    dO^T / Q^T with ds_read_b64_tr_b16.  The two q-group waves' partial
-//    dK/dV of each kv quarter are summed through LDS.  Tiles heavier than the
-//    scheduler's piece length run as several work items writing fp32 sums to
-//    workspace slots,
+//  * dK/dV (D = 128): one workgroup = 8 waves = 128 kv rows of one kv-head.
+//    Wave (g, kq) owns kv rows 32 kq .. 32 kq + 31 and q rows 32 g .. 32 g + 31
+//    of each 64-row step, so every staged Q / dO tile feeds all 128 kv rows and
+//    every SIMD runs two waves, half a step apart.  K of the tile in LDS and V
+//    in registers are the B operands of S = Q K^T and dP = dO V^T.  A work item
+//    walks steps (q block, q-head of the GQA group) of its kv tile, with Q / dO
+//    / LSE2 / Delta in a ring of three LDS stages by direct global->LDS loads
+//    and the operand reads two k-steps ahead of the MFMAs; dV^T += dO^T P and
+//    dK^T += Q^T dS read dO^T / Q^T with ds_read_b64_tr_b16.  The two q-group
+//    waves' partial dK/dV of each kv quarter are summed through LDS.  Tiles
+//    heavier than the scheduler's piece length run as several work items
+//    writing fp32 sums to workspace slots,
 //  * which the partial-sum kernel adds in piece order afterwards.
 // At D = 64 the deterministic backward's dK/dV kernel is
 // attn_bwd_dkdv_w4_kernel (one wave per SIMD, K and V in registers); the
 // atomic backward replaces the dQ kernel with a Delta / LSE2 pass, dQ formed
-// in the 8-wave dK/dV kernel, and a conversion of the fp32 sums.
+// in a dK/dV kernel of its own (attn_bwd_dkdv_atomic_kernel, all waves in
+// step), and a conversion of the fp32 sums.
 // With the rotary embedding fused, the dQ kernel reads the rotated q the
 // forward wrote and stores dq through the rotation's backward (the separate
 // RoPE backward pass's exact roundings); dK stays the gradient of the rotated
@@ -45,25 +45,105 @@ namespace siq {
 
 namespace {
 
-// Atomic dQ (DQ = true, the non-deterministic backward): the dK/dV kernel
-// also forms dQ = dS K, so no second kernel recomputes S and dP.  Each wave
-// writes its 32 x 32 block of dS (bf16) to an LDS exchange buffer [64 q][128
-// kv] (rows padded to 136 elements: consecutive rows start one 16-byte bank
-// group apart, so the row reads below are conflict free and every write of a
-// lane is its base plus a constant); after a barrier wave (g, kq) multiplies
-// the q rows of group g by K for d-tile kq % NDT over the kv quarters of part
-// kq / NDT (all four at D = 128, two at D = 64) and adds the fp32 result to a
-// dQ workspace with vector atomics, issued after the step's closing barrier so
-// that its load wait does not also wait for them.  kv offset o of each 16-kv
-// group is stored at slot o with bits 2 and 3 swapped, so that a row read
-// returns the kv order of a transposed K read (TrRead's krow).
+// Atomic dQ (the non-deterministic backward): its dK/dV kernel also forms dQ =
+// dS K, so no second kernel recomputes S and dP.  Each wave writes its 32 x 32
+// block of dS (bf16) to an LDS exchange buffer [64 q][128 kv] (rows padded to
+// 136 elements: consecutive rows start one 16-byte bank group apart, so the
+// row reads below are conflict free and every write of a lane is its base plus
+// a constant); after a barrier wave (g, kq) multiplies the q rows of group g
+// by K for d-tile kq % NDT over the kv quarters of part kq / NDT (all four at
+// D = 128, two at D = 64) and adds the fp32 result to a dQ workspace with
+// vector atomics, issued after the step's closing barrier so that its load
+// wait does not also wait for them.  kv offset o of each 16-kv group is stored
+// at slot o with bits 2 and 3 swapped, so that a row read returns the kv order
+// of a transposed K read (TrRead's krow).
 constexpr int kDsxLd = kBwdBN + 8;
 __device__ __forceinline__ int dsx_slot(int kv) {
   return (kv & ~15) | (kv & 3) | ((kv & 4) << 1) | ((kv & 8) >> 1);
 }
 
-template <int D, bool CAUSAL, bool DQ>
-__global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams p) {
+// Sum the two q-group waves' partial dK^T / dV^T of each kv quarter in one
+// exchange through LDS: wave g finishes d-tiles [g NDT / 2, (g + 1) NDT / 2)
+// of both tensors and hands the other half of its partials to its partner
+// (wave 1 - g of the quarter), with 16-byte LDS stores of 1 KB per
+// instruction.  Each sum is g = 0's partial plus g = 1's.  A whole tile
+// (np == 1) is scaled and written as bf16; a piece of a split tile writes
+// its fp32 sums to its slot ([dK | dV][kv row][d]) for
+// attn_bwd_dkv_sum_kernel.  `smem` holds at least
+// 8 x 2 x NDT / 2 x 4 KB that no wave reads any more.
+template <int D>
+__device__ __forceinline__ void dkdv_finish(const AttnParams& p, const KvItem& it, int hk, int g, int kq, int lane,
+                                            bf16* smem, const f32x16 (&dk)[D / 32], const f32x16 (&dv)[D / 32]) {
+  constexpr int BN = kBwdBN, NDT = D / 32;
+  const int h = lane >> 5, l32 = lane & 31;
+  const SeqInfo si = it.s;
+  const int kvrow = it.t * BN + 32 * kq + l32;
+  const bool kvvalid = kvrow < si.k_len;
+  const bool split = it.np > 1;
+  const bool slot_ok = split && it.slot0 >= 0 && (it.slot0 + it.np) * p.hkv <= kSplitSlots;
+  float* slot = p.dkv_part + (int64_t)((it.slot0 + it.piece) * p.hkv + hk) * (2 * BN * D);
+  const int64_t row = si.k_start + kvrow;
+  constexpr int HT = NDT / 2;             // d-tiles a wave finishes
+  constexpr int XR = 2 * HT * 16 * 64;    // floats a wave hands its partner: [dK | dV][HT][16][64 lanes]
+  float* inbox = reinterpret_cast<float*>(smem) + (2 * kq + g) * XR;
+  float* outbox = reinterpret_cast<float*>(smem) + (2 * kq + (1 - g)) * XR;
+  // d-tiles are indexed statically (a wave-uniform branch picks them), so
+  // the accumulators stay in registers
+#pragma unroll
+  for (int t = 0; t < NDT; ++t) {
+    if (t / HT == g) continue;  // this wave finishes tile t itself
+    const int u = t % HT;
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      *reinterpret_cast<f32x4*>(outbox + ((0 * HT + u) * 4 + q4) * 256 + 4 * lane) =
+          f32x4{dk[t][4 * q4], dk[t][4 * q4 + 1], dk[t][4 * q4 + 2], dk[t][4 * q4 + 3]};
+      *reinterpret_cast<f32x4*>(outbox + ((1 * HT + u) * 4 + q4) * 256 + 4 * lane) =
+          f32x4{dv[t][4 * q4], dv[t][4 * q4 + 1], dv[t][4 * q4 + 2], dv[t][4 * q4 + 3]};
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int which = 0; which < 2; ++which) {
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+      if (dt / HT != g) continue;  // the partner finishes tile dt
+      const int u = dt % HT;
+      const f32x16& mine = which == 0 ? dk[dt] : dv[dt];
+      float sum[16];
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 o = *reinterpret_cast<const f32x4*>(inbox + ((which * HT + u) * 4 + q4) * 256 + 4 * lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[4 * q4 + i] = g == 0 ? mine[4 * q4 + i] + o[i] : o[i] + mine[4 * q4 + i];
+      }
+      if (!split) {
+        if (kvvalid) {
+          bf16* dst = which == 0 ? p.dk + row * p.dk_tok + (int64_t)hk * p.dk_head
+                                 : p.dv + row * p.dv_tok + (int64_t)hk * p.dv_head;
+          const float sc = which == 0 ? p.scale : 1.f;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            bf16x8 o;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) o[q] = (bf16)(sum[8 * j + q] * sc);
+            st_bf16x8(dst + 32 * dt + 16 * j + 8 * h, o);
+          }
+        }
+      } else if (slot_ok) {
+        float* dst = slot + ((int64_t)which * BN + 32 * kq + l32) * D + 32 * dt + 8 * h;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          *reinterpret_cast<f32x4*>(dst + 16 * j) = f32x4{sum[8 * j], sum[8 * j + 1], sum[8 * j + 2], sum[8 * j + 3]};
+          *reinterpret_cast<f32x4*>(dst + 16 * j + 4) =
+              f32x4{sum[8 * j + 4], sum[8 * j + 5], sum[8 * j + 6], sum[8 * j + 7]};
+        }
+      }
+    }
+  }
+}
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_atomic_kernel(const AttnParams p) {
   constexpr int BN = kBwdBN, BM = kBwdBM, NT = 512, NW = NT / 64, NS = 2;
   static_assert(BN == 128 && BM == 64, "128 kv rows (4 x 32) by 64 q rows (2 x 32) per step");
   using StTile = LdsTile<BM, D, NW / 2>;  // Q staged by waves 0-3, dO by waves 4-7
@@ -72,10 +152,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
   constexpr int STAGE = 2 * TE;  // Q, dO (bf16 elements)
   constexpr int NDT = D / 32;
   constexpr int SMEM = NS * STAGE + 2 * KVTile::ELEMS;  // stages, K, V
-  static_assert(2 * 4 * NDT * 16 * 64 * 4 <= SMEM * 2, "one reduction round fits the LDS");
   __shared__ __align__(16) bf16 smem[SMEM];
   __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | delta][q] (raw, as loaded)
-  __shared__ __align__(16) bf16 dsx[DQ ? BM * kDsxLd : 8];  // dS exchange (atomic dQ)
+  __shared__ __align__(16) bf16 dsx[BM * kDsxLd];  // dS exchange (atomic dQ)
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
   const int wu = wave_uniform(tid >> 6);
@@ -284,7 +363,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
       pb[1] = pack8(s, 8);
       db[0] = pack8(dp, 0);
       db[1] = pack8(dp, 8);
-      if constexpr (DQ) {
+      {
         // this wave's dS block into the exchange buffer: q = 32 g + 4 h + 8 (r / 4) + r % 4, kv = 32 kq + l32.
         // kv rows past the sequence end hold the last row's K (their dK / dV rows are never written, but
         // dQ sums over kv): their dS is written as zero
@@ -307,118 +386,328 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
         dk[dt] = mfma32(tq[cur], db[j], dk[dt]);
       }
     }
-    if constexpr (DQ) {
-      // every wave's dS block is in the exchange buffer after this barrier
-      __syncthreads();
-      // dQ[q][d] = sum dS[q][kv] K[kv][d] for q rows 32 g .., d-tile qdt, this part's kv quarters
-      f32x16 dqa = zero16();
-      bool any = false;
+    // every wave's dS block is in the exchange buffer after this barrier
+    __syncthreads();
+    // dQ[q][d] = sum dS[q][kv] K[kv][d] for q rows 32 g .., d-tile qdt, this part's kv quarters
+    f32x16 dqa = zero16();
+    bool any = false;
 #pragma unroll
-      for (int u = 0; u < 4 / WPT; ++u) {
-        const int qq = qpart * (4 / WPT) + u;
-        if (!quarter_active(qq)) continue;
-        any = true;
+    for (int u = 0; u < 4 / WPT; ++u) {
+      const int qq = qpart * (4 / WPT) + u;
+      if (!quarter_active(qq)) continue;
+      any = true;
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const bf16x8 a = ld_bf16x8(dsx + (32 * g + l32) * kDsxLd + 8 * h + 16 * (2 * qq + kk));
-          const bf16x8 b = tr.read(Ks, 32 * qq + 16 * kk, qdt);
-          dqa = mfma32(a, b, dqa);
-        }
+      for (int kk = 0; kk < 2; ++kk) {
+        const bf16x8 a = ld_bf16x8(dsx + (32 * g + l32) * kDsxLd + 8 * h + 16 * (2 * qq + kk));
+        const bf16x8 b = tr.read(Ks, 32 * qq + 16 * kk, qdt);
+        dqa = mfma32(a, b, dqa);
       }
-      // the next stage's loads first (the atomics below also count in vmcnt), then the sums
-      wait_vmem();
-      if (any) {
-        // wave-uniform base (first row of the group, its q-head) plus a 32-bit lane offset
-        float* base = p.dq_acc + ((int64_t)(si.q_start + wq0) * p.hq + hk * p.n_rep + step % p.n_rep) * D;
-        uint32_t rs = (uint32_t)(p.hq * D);
-        uint32_t lo = (uint32_t)(32 * qdt + perm32(l32)) + (uint32_t)(4 * h) * rs;
-        // recomputed here each step: hoisted out of the loop, the 16 row offsets would hold 16 registers
-        asm volatile("" : "+s"(rs), "+v"(lo));
-        const int rows = qvalid - 32 * g;
+    }
+    // the next stage's loads first (the atomics below also count in vmcnt), then the sums
+    wait_vmem();
+    if (any) {
+      // wave-uniform base (first row of the group, its q-head) plus a 32-bit lane offset
+      float* base = p.dq_acc + ((int64_t)(si.q_start + wq0) * p.hq + hk * p.n_rep + step % p.n_rep) * D;
+      uint32_t rs = (uint32_t)(p.hq * D);
+      uint32_t lo = (uint32_t)(32 * qdt + perm32(l32)) + (uint32_t)(4 * h) * rs;
+      // recomputed here each step: hoisted out of the loop, the 16 row offsets would hold 16 registers
+      asm volatile("" : "+s"(rs), "+v"(lo));
+      const int rows = qvalid - 32 * g;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int i = 8 * (r >> 2) + (r & 3);
-          if (i + 4 * h < rows) __builtin_amdgcn_global_atomic_fadd_f32(base + lo + (uint32_t)i * rs, dqa[r]);
-        }
+      for (int r = 0; r < 16; ++r) {
+        const int i = 8 * (r >> 2) + (r & 3);
+        if (i + 4 * h < rows) __builtin_amdgcn_global_atomic_fadd_f32(base + lo + (uint32_t)i * rs, dqa[r]);
       }
-    } else {
-      wait_vmem();
     }
     __syncthreads();
   }
 
-  // Sum the two q-group waves' partial dK^T / dV^T of each kv quarter in one
-  // exchange through LDS: wave g finishes d-tiles [g NDT / 2, (g + 1) NDT / 2)
-  // of both tensors and hands the other half of its partials to its partner
-  // (wave 1 - g of the quarter), with 16-byte LDS stores of 1 KB per
-  // instruction.  Each sum is g = 0's partial plus g = 1's.  A whole tile
-  // (np == 1) is scaled and written as bf16; a piece of a split tile writes
-  // its fp32 sums to its slot ([dK | dV][kv row][d]) for
-  // attn_bwd_dkv_sum_kernel.
-  const bool split = it.np > 1;
-  const bool slot_ok = split && it.slot0 >= 0 && (it.slot0 + it.np) * p.hkv <= kSplitSlots;
-  float* slot = p.dkv_part + (int64_t)((it.slot0 + it.piece) * p.hkv + hk) * (2 * BN * D);
-  const int64_t row = si.k_start + kvrow;
-  constexpr int HT = NDT / 2;             // d-tiles a wave finishes
-  constexpr int XR = 2 * HT * 16 * 64;    // floats a wave hands its partner: [dK | dV][HT][16][64 lanes]
-  static_assert(8 * XR * 4 <= SMEM * 2, "the exchange fits the LDS");
-  float* inbox = reinterpret_cast<float*>(smem) + (2 * kq + g) * XR;
-  float* outbox = reinterpret_cast<float*>(smem) + (2 * kq + (1 - g)) * XR;
   // the step loop ends on a barrier; an item without steps has only read K / V (D = 64) since the last one
   if (ns == 0) __syncthreads();
-  // d-tiles are indexed statically (a wave-uniform branch picks them), so
-  // the accumulators stay in registers
+  dkdv_finish<D>(p, it, hk, g, kq, lane, smem, dk, dv);
+}
+
+// dK/dV at D = 128.  A step of a wave has three parts: M1, the S / dP
+// products (16 MFMAs); V, the softmax's VALU work; M2, the dV / dK products
+// (16 MFMAs).  Waves 4-7 run half a step behind waves 0-3 (waves w and w + 4
+// share a SIMD), with a barrier after M1 and one after V: while the one wave
+// of a SIMD does its V, the other does M2 of its step and M1 of the next.
+// With both in step (all M1, all V, all M2, one barrier) the matrix cores
+// stood idle through every V, which the matrix products' register traffic
+// stretches to some 900 cycles against 512 each for M1 and M2.
+// Q / dO / LSE2 / Delta stages are a ring of three: between its M1 and its M2
+// a wave group keeps a stage while the other group already reads the next
+// and a third is loaded.  Waves 4-7 load the stage of step i + 2 in their V of
+// step i (its buffer, step i - 1's, was last read in their own M2 before; a
+// load in an M part would hold up the products behind it) and wait for it at
+// the end of their M1 of step i + 1.  V of the kv rows stays in registers (a
+// third of M1's LDS reads, which one wave per SIMD could not otherwise take at
+// the products' pace), K in LDS.
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams p) {
+  constexpr int BN = kBwdBN, BM = kBwdBM, NT = 512, NW = NT / 64, NS = 3;
+  static_assert(D == 128 && BN == 128 && BM == 64, "128 kv rows (4 x 32) by 64 q rows (2 x 32) per step");
+  using StTile = LdsTile<BM, D, NW / 2>;
+  using KTile = LdsTile<BN, D, NW>;
+  constexpr int TE = StTile::ELEMS, STAGE = 2 * TE;  // Q, dO (bf16 elements)
+  constexpr int NDT = D / 32, KS = D / 16, U2 = 2 * NDT;
+  constexpr int SMEM = NS * STAGE + KTile::ELEMS;  // stages, K
+  static_assert(8 * 2 * (NDT / 2) * 16 * 64 * 4 <= SMEM * 2, "dkdv_finish's exchange fits the LDS");
+  __shared__ __align__(256) bf16 smem[SMEM];  // (whole rows aligned: operand addresses are formed by XOR)
+  __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | delta][q] (raw, as loaded)
+
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+  const int wu = wave_uniform(tid >> 6);
+  const int g = wu & 1, kq = wu >> 1;  // q group (32 rows of a step), kv quarter (32 rows of the tile)
+  const bool late = wu >= NW / 2;
+  const float c = p.scale_log2;
+  bf16* Ks = smem + NS * STAGE;
+
+  // 1-D grid over (item, kv-head), kv-head fastest; each XCD takes one item
+  // (all its kv-heads) per run, so the heaviest-first items go round the XCDs
+  const int e = xcd_order(blockIdx.x, gridDim.x, p.hkv);
+  const int ii = e / p.hkv, hk = e - ii * p.hkv;
+  const PlanHeader ph = plan_header(p);
+  const KvItem it = p.kvitems[ii];
+  // every field of the entry and the plan header loaded before the idle
+  // test (the compiler would otherwise fetch b alone, wait for it, then
+  // fetch the rest)
+  asm volatile("" : : "s"(it.s.q_start), "s"(it.s.q_len), "s"(it.s.k_start), "s"(it.s.k_len), "s"(it.t), "s"(it.s0),
+               "s"(it.s1), "v"(ph.magic));
+  if (!plan_header_ok(ph, p, CAUSAL, true) || it.b < 0) return;
+  const SeqInfo si = it.s;
+  const int k0 = it.t * BN;
+  const int kb = k0 + 32 * kq;  // first kv row of this wave
+  const int off = si.k_len - si.q_len;
+
+  // K of the tile in LDS, V of this wave's rows in registers in the
+  // row-operand layout (lane: row l32, d = 16 ks + 8 h .. +7); rows past the
+  // end repeat the last row: they only reach dK / dV rows that are never
+  // written
+  KTile kt;
+  kt.init(p.k_tok, lane);
+  kt.template issue<true>(p.k + (int64_t)(si.k_start + k0) * p.k_tok + (int64_t)hk * p.k_head, p.k_tok, si.k_len - k0,
+                          Ks, wu);
+  bf16x8 vreg[KS];
+  {
+    const int r = max(0, min(kb + l32, si.k_len - 1));
+    const bf16* vp = p.v + (int64_t)(si.k_start + r) * p.v_tok + (int64_t)hk * p.v_head + 8 * h;
 #pragma unroll
-  for (int t = 0; t < NDT; ++t) {
-    if (t / HT == g) continue;  // this wave finishes tile t itself
-    const int u = t % HT;
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      *reinterpret_cast<f32x4*>(outbox + ((0 * HT + u) * 4 + q4) * 256 + 4 * lane) =
-          f32x4{dk[t][4 * q4], dk[t][4 * q4 + 1], dk[t][4 * q4 + 2], dk[t][4 * q4 + 3]};
-      *reinterpret_cast<f32x4*>(outbox + ((1 * HT + u) * 4 + q4) * 256 + 4 * lane) =
-          f32x4{dv[t][4 * q4], dv[t][4 * q4 + 1], dv[t][4 * q4 + 2], dv[t][4 * q4 + 3]};
-    }
+    for (int ks = 0; ks < KS; ++ks) vreg[ks] = ld_bf16x8(vp + 16 * ks);
   }
+  f32x16 dk[NDT], dv[NDT];
+#pragma unroll
+  for (int i = 0; i < NDT; ++i) {
+    dk[i] = zero16();
+    dv[i] = zero16();
+  }
+
+  // The tile's steps are (q block, q-head j of the GQA group) for the q blocks
+  // that can see any of its rows, q blocks from the last one down, the n_rep
+  // heads inside; this item runs steps [s0, s1).
+  const int qb_last = (si.q_len - 1) / BM;
+  const int s0 = it.s0, ns = it.s1 - it.s0;
+  int q0 = (qb_last - s0 / p.n_rep) * BM, j = s0 % p.n_rep;  // the step's first q row and head
+  int i = 0, buf = 0;                                        // the step, its stage
+
+  // Loads of waves 4-7: step ln into its stage (untracked; 4 + 4 instructions
+  // a wave of 4 rows each, waves 4 / 5 also LSE2 / Delta).  Instructions k
+  // cover rows lrow0 + 4 k .. + 3 of the block, and their swizzle is the
+  // lane's chunk XOR k.
+  const bf16* qsrc = p.q + ((int64_t)si.q_start + q0) * p.q_tok + (int64_t)(hk * p.n_rep + j) * p.q_head;
+  const bf16* gsrc = p.dout + ((int64_t)si.q_start + q0) * p.do_tok + (int64_t)(hk * p.n_rep + j) * p.do_head;
+  const float* rsrc = ((wu & 1) == 0 ? p.lse2 : p.delta) + (int64_t)(hk * p.n_rep + j) * p.lse_head + si.q_start + q0;
+  // to the next head; to the next block's first head
+  int64_t qstep = p.q_head, qwrap = -(p.n_rep - 1) * p.q_head - BM * p.q_tok;
+  int64_t gstep = p.do_head, gwrap = -(p.n_rep - 1) * p.do_head - BM * p.do_tok;
+  int64_t rstep = p.lse_head, rwrap = -(p.n_rep - 1) * p.lse_head - BM;
+  uint32_t qtok2 = 2 * (uint32_t)p.q_tok, gtok2 = 2 * (uint32_t)p.do_tok;
+  int n_rep = p.n_rep;
+  pin_sgpr(qstep);
+  pin_sgpr(qwrap);
+  pin_sgpr(gstep);
+  pin_sgpr(gwrap);
+  pin_sgpr(rstep);
+  pin_sgpr(rwrap);
+  pin_sgpr(qtok2);
+  pin_sgpr(gtok2);
+  pin_sgpr(n_rep);
+  const int lrow0 = 16 * (wu & 3), lrow = lrow0 + lane / StTile::CH;
+  const uint32_t lchunk = 16 * (uint32_t)((lane % StTile::CH) ^ ((lane / StTile::CH) << 2));
+  int nrows = si.q_len - q0, lj = j, ln = 0, nbuf = 0;
+  static_assert(StTile::PERW == 4, "four loads a step, wave and tensor");
+  auto load_k = [&](int k) {
+    if (ln >= ns) return;
+    const uint32_t row = (uint32_t)min(lrow + 4 * k, nrows - 1);  // rows past the end re-read the last one
+    bf16* dst = smem + nbuf * STAGE + (lrow0 + 4 * k) * D;
+    dma16(qsrc, row * qtok2 + (lchunk ^ (16 * k)), dst);
+    dma16(gsrc, row * gtok2 + (lchunk ^ (16 * k)), dst + TE);
+  };
+  // the row values, after which the next step's loads are on
+  auto load_rows = [&]() {
+    if (ln >= ns) return;
+    if ((wu & 3) < 2) dma4_untracked(rsrc + min(lane, nrows - 1), &rowv[nbuf][wu & 1][0]);
+    const bool wrap = lj + 1 == n_rep;
+    lj = wrap ? 0 : lj + 1;
+    qsrc += wrap ? qwrap : qstep;
+    gsrc += wrap ? gwrap : gstep;
+    rsrc += wrap ? rwrap : rstep;
+    nrows += wrap ? BM : 0;
+    ++ln;
+    nbuf = nbuf == NS - 1 ? 0 : nbuf + 1;
+  };
+  auto load_next = [&]() {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) load_k(k);
+    load_rows();
+  };
+
+  // byte addresses of this lane's operands in stage 0 (dO follows Q by TE elements)
+  RowRead<D> rr;
+  rr.init(lane);
+  TrRead<D> tr;
+  tr.init(lane);
+  const uint32_t qa0 = lds_addr(smem) + 2 * (32 * g * D + rr.base);
+  const uint32_t ta0 = lds_addr(smem) + 2 * (32 * g * D + tr.base[0]);
+  const uint32_t ta1 = lds_addr(smem) + 2 * (32 * g * D + tr.base[1]);
+  uint32_t ka = lds_addr(Ks) + 2 * (32 * kq * D + rr.base);
+  bf16x8 fq[KS], fg[KS], fk[KS];  // at most three k-steps of them are live
+  auto fetch = [&](uint32_t qa, int ks) {
+    fq[ks] = lds_read16(qa ^ (32 * ks));
+    fk[ks] = lds_read16(ka ^ (32 * ks));
+    fg[ks] = lds_read16((qa ^ (32 * ks)) + 2 * TE);
+  };
+  auto advance = [&]() {
+    const bool wrap = j + 1 == n_rep;
+    j = wrap ? 0 : j + 1;
+    q0 = wrap ? q0 - BM : q0;
+    buf = buf == NS - 1 ? 0 : buf + 1;
+    ++i;
+  };
+  // A wave has no product in the steps of the last q block when its group of
+  // 32 rows is past the sequence end, nor (causal) in those of the first
+  // blocks, before its kv rows: idle steps, active steps, idle steps.  Three
+  // loops rather than a branch in one: the accumulators are only carried
+  // through the active one.
+  auto active = [&]() {
+    return 32 * g < si.q_len - q0 && kb < si.k_len && (!CAUSAL || q0 + 32 * g + 31 + off >= kb);
+  };
+  auto idle_step = [&]() {
+    if (late) wait_vmem();
+    phase_barrier();
+    if (late) load_next();
+    phase_barrier();
+    advance();
+  };
+
+  if (late) {
+    load_next();
+    load_next();
+  }
+  wait_vmem();
   __syncthreads();
+  if (late) phase_barrier();
+  for (; i < ns && !active();) idle_step();
+  fetch(qa0 + 2 * STAGE * buf, 0);  // (in bounds, and unused, when there is no step left)
+  fetch(qa0 + 2 * STAGE * buf, 1);
+  for (; i < ns && active();) {
+    uint32_t qa = qa0 + 2 * STAGE * buf, a0 = ta0 + 2 * STAGE * buf, a1 = ta1 + 2 * STAGE * buf;
+    const int wq0 = q0 + 32 * g;
+    const int qvalid = si.q_len - q0;  // rows of this block that exist
+    // M1; accumulator r (= 8j + i) holds q = wq0 + 16j + 8(i / 4) + 4h + i % 4, kv = kb + l32.  Operands are read two
+    // k-steps ahead of the products.
+    f32x16 s = zero16(), dp = zero16();
+    opaque(qa);
+    opaque(ka);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-  for (int which = 0; which < 2; ++which) {
+    for (int ks = 0; ks < KS; ++ks) {
+      if (ks + 2 < KS) fetch(qa, ks + 2);
+      s = mfma32(fq[ks], fk[ks], s);
+      dp = mfma32(fg[ks], vreg[ks], dp);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if (late) wait_vmem();  // this wave's share of the next step
+    phase_barrier();
+    // V: P = exp2(S scale log2e - LSE2), dS = P (dP - Delta), in place; on the causal diagonal and past the
+    // end of the sequence the exponent is -inf (P = 0, hence dS = 0)
+    {
+      const float* lse2 = &rowv[buf][0][32 * g + 4 * h];
+      const float* delta = lse2 + BM;
+      f32x4 lv[4], dl[4];
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      if (dt / HT != g) continue;  // the partner finishes tile dt
-      const int u = dt % HT;
-      const f32x16& mine = which == 0 ? dk[dt] : dv[dt];
-      float sum[16];
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 o = *reinterpret_cast<const f32x4*>(inbox + ((which * HT + u) * 4 + q4) * 256 + 4 * lane);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sum[4 * q4 + i] = g == 0 ? mine[4 * q4 + i] + o[i] : o[i] + mine[4 * q4 + i];
+      for (int u = 0; u < 4; ++u) {
+        lv[u] = *reinterpret_cast<const f32x4*>(lse2 + 8 * u);
+        dl[u] = *reinterpret_cast<const f32x4*>(delta + 8 * u);
       }
-      if (!split) {
-        if (kvvalid) {
-          bf16* dst = which == 0 ? p.dk + row * p.dk_tok + (int64_t)hk * p.dk_head
-                                 : p.dv + row * p.dv_tok + (int64_t)hk * p.dv_head;
-          const float sc = which == 0 ? p.scale : 1.f;
+      if (late) load_k(0);
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            bf16x8 o;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) o[q] = (bf16)(sum[8 * j + q] * sc);
-            st_bf16x8(dst + 32 * dt + 16 * j + 8 * h, o);
-          }
-        }
-      } else if (slot_ok) {
-        float* dst = slot + ((int64_t)which * BN + 32 * kq + l32) * D + 32 * dt + 8 * h;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          *reinterpret_cast<f32x4*>(dst + 16 * j) = f32x4{sum[8 * j], sum[8 * j + 1], sum[8 * j + 2], sum[8 * j + 3]};
-          *reinterpret_cast<f32x4*>(dst + 16 * j + 4) =
-              f32x4{sum[8 * j + 4], sum[8 * j + 5], sum[8 * j + 6], sum[8 * j + 7]};
-        }
+      for (int r = 0; r < 16; ++r) {
+        s[r] = __builtin_fmaf(s[r], c, -lv[r >> 2][r & 3]);
+        dp[r] -= dl[r >> 2][r & 3];
       }
     }
+    pin_vgpr(s);
+    pin_vgpr(dp);
+    if (late) load_k(1);
+    if (CAUSAL && wq0 + off < kb + 31) {
+      const int rel = l32 - 4 * h + (kb - off - wq0);  // keep q offsets >= rel
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) >= rel ? s[r] : -INFINITY;
+    }
+    if (32 * g + 32 > qvalid) {
+      const int lim = qvalid - 32 * g - 4 * h;  // keep q offsets < lim
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) < lim ? s[r] : -INFINITY;
+    }
+    bf16x8 pb[2], db[2], tg[U2], tq[U2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int r = 8 * half; r < 8 * half + 8; ++r) {
+        s[r] = exp2f_fast(s[r]);
+        dp[r] *= s[r];
+      }
+      pb[half] = pack8(s, 8 * half);
+      db[half] = pack8(dp, 8 * half);
+      pin_vgpr(pb[half]);
+      pin_vgpr(db[half]);
+      if (late) load_k(2 + half);
+    }
+    if (late) load_rows();
+    opaque(a0);
+    opaque(a1);
+    auto fetch_t = [&](int u) {
+      const int dt = u % NDT, o = 2 * 16 * D * (u / NDT);
+      tg[u] = lds_read_tr((a0 ^ (64 * dt)) + o + 2 * TE, (a1 ^ (64 * dt)) + o + 2 * TE);
+      tq[u] = lds_read_tr((a0 ^ (64 * dt)) + o, (a1 ^ (64 * dt)) + o);
+    };
+    fetch_t(0);
+    fetch_t(1);
+    phase_barrier();
+    // M2, and the first operands of the next step (whatever its stage holds, if there is none)
+    advance();
+    uint32_t qn = qa0 + 2 * STAGE * buf;
+    opaque(qn);
+    opaque(ka);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int u = 0; u < U2; ++u) {
+      if (u + 2 < U2)
+        fetch_t(u + 2);
+      else
+        fetch(qn, u + 2 - U2);
+      dv[u % NDT] = mfma32(tg[u], pb[u / NDT], dv[u % NDT]);
+      dk[u % NDT] = mfma32(tq[u], db[u / NDT], dk[u % NDT]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
   }
+  for (; i < ns;) idle_step();
+  if (!late) phase_barrier();  // both groups have met the same number of barriers
+  __syncthreads();             // every wave's last stage reads are done
+  dkdv_finish<D>(p, it, hk, g, kq, lane, smem, dk, dv);
 }
 
 // dK/dV with one wave per SIMD (the deterministic backward's kernel at D =
@@ -1054,7 +1343,7 @@ hipError_t launch_bwd_t(const AttnParams& p, int qcap, int kvcap, hipStream_t st
     const int64_t pblocks = std::min<int64_t>((pairs + ppb - 1) / ppb, 8192);
     const int64_t blocks = std::min<int64_t>((pairs + 256 / (D / 8) - 1) / (256 / (D / 8)), 8192);
     if (pblocks > 0) hipLaunchKernelGGL((attn_bwd_prep_kernel<D>), dim3((unsigned)pblocks), dim3(256), 0, stream, p);
-    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, CAUSAL, true>), kvgrid, dim3(512), 0, stream, p);
+    hipLaunchKernelGGL((attn_bwd_dkdv_atomic_kernel<D, CAUSAL>), kvgrid, dim3(512), 0, stream, p);
     hipLaunchKernelGGL((attn_bwd_dkv_sum_kernel<D, CAUSAL>), dim3(min(kMaxSplitTiles * DkvSum<D>::NCH, 512), p.hkv), dim3(256),
                        0, stream, p);
     if (blocks > 0)
@@ -1073,7 +1362,7 @@ hipError_t launch_bwd_t(const AttnParams& p, int qcap, int kvcap, hipStream_t st
   if constexpr (D == 64)
     hipLaunchKernelGGL((attn_bwd_dkdv_w4_kernel<D, CAUSAL>), kvgrid, dim3(256), 0, stream, p);
   else
-    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, CAUSAL, false>), kvgrid, dim3(512), 0, stream, p);
+    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, CAUSAL>), kvgrid, dim3(512), 0, stream, p);
   hipLaunchKernelGGL((attn_bwd_dkv_sum_kernel<D, CAUSAL>), dim3(min(kMaxSplitTiles * DkvSum<D>::NCH, 512), p.hkv), dim3(256), 0, stream,
                      p);
   return hipGetLastError();

@@ -138,6 +138,23 @@ struct RowRead {
   }
 };
 
+// LDS reads at a byte address, for loops that keep the lane's address in one
+// register: a row operand's chunk 2 ks + h is at lane address ^ 32 ks (RowRead),
+// a transposed operand's column block dt at lane address ^ 64 dt (TrRead).
+typedef __attribute__((address_space(3))) const bf16x8 lds_cbf16x8;
+__device__ __forceinline__ bf16x8 lds_read16(uint32_t a) { return *(lds_cbf16x8*)a; }
+__device__ __forceinline__ bf16x8 lds_read_tr(uint32_t a0, uint32_t a1) {
+  const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)a0);
+  const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)a1);
+  return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(lds_void*)p; }
+
+// Makes a value opaque where it stands, so that what is derived from it in a
+// loop is computed there (the compiler would otherwise keep every derived
+// address in a register of its own).
+__device__ __forceinline__ void opaque(uint32_t& x) { asm volatile("" : "+v"(x)); }
+
 // Writes in the staging layout from the MFMA row layout: lane l owns tile row
 // rb + l % 32 (rb a multiple of 32) and writes its 16-byte logical chunks c,
 // so that whole rows can then be read out 256 bytes at a time (RowSpan).
@@ -208,6 +225,13 @@ struct TrRead {
   }
 };
 
+// One wave instruction of direct loading from a uniform base and this lane's
+// byte offset, untracked (as LdsTile::issue<true>, whose s_nop it shares).
+__device__ __forceinline__ void dma16(const bf16* gbase, uint32_t byte_off, const bf16* lds) {
+  const uint32_t la = (uint32_t)(uintptr_t)(lds_void*)lds;
+  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(byte_off), "s"(gbase), "{m0}"(la) : "memory");
+}
+
 // One dword per lane from gptr straight into LDS (lane l's 4 bytes land at LDS
 // byte lds + 4 l), untracked like LdsTile::issue<true>: the caller orders it
 // with wait_vmem and a barrier.  s_nop 0: m0 needs one wait state after its
@@ -224,6 +248,14 @@ __device__ __forceinline__ void pin_sgpr(T& x) {
   asm volatile("" : "+s"(x));
 }
 
+// Keeps the computation of a vector before this point (and what uses it
+// after): the compiler otherwise sinks VALU work to its first use, across
+// barriers.
+template <typename T>
+__device__ __forceinline__ void pin_vgpr(T& x) {
+  asm volatile("" : "+v"(x));
+}
+
 // Wait for this wave's outstanding global (and direct-to-LDS) loads.
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
@@ -236,6 +268,16 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
+}
+
+// A workgroup barrier that waits for no memory: the compiler neither moves
+// code across it nor drains the load queue at it.
+__device__ __forceinline__ void phase_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
 }
 
 // Per-sequence extents, clamped on the device to [0, total).

@@ -128,3 +128,29 @@ def test_more_sequences_than_the_scheduler_lds_holds(d, causal):
 def test_larger_qwen_head_layouts(hq, hkv):
     # Qwen2.5-7B (28 / 4 heads) and -14B (40 / 8) at d 128: GQA groups of 7 and 5, several kv-heads
     check([257, 40, 611, 128], [257, 40, 611, 128], hq, hkv, 128, True, seed=8)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("heads", [(1, 1), (3, 1), (4, 2)])
+def test_dkdv_stage_ring_at_few_steps(heads, causal):
+    """The D = 128 dK/dV kernel's two wave groups run half a step apart over a
+    ring of three stages: kv tiles with 1 .. 8 steps, ending in idle steps (a
+    last q block of up to 32 rows, q rows before a kv quarter), beside one
+    sequence long enough to be cut into pieces.  dK and dV are bitwise the
+    atomic backward's, whose kernel keeps all waves in step, and match the
+    oracle."""
+    print(f"dkdv ring heads={heads} causal={causal}", flush=True)
+    hq, hkv = heads
+    lens = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 193, 255, 256, 257, 1500]
+    g = torch.Generator().manual_seed(hq)
+    t, cu = sum(lens), offsets(lens)
+    q, do = (torch.randn(t, hq, 128, generator=g).to(torch.bfloat16) for _ in range(2))
+    k, v = (torch.randn(t, hkv, 128, generator=g).to(torch.bfloat16) for _ in range(2))
+    ref = oa.attention_bwd(do, q, k, v, cu, cu, 128**-0.5, causal)
+    q, k, v, do, cu = (x.to(DEV) for x in (q, k, v, do, cu))
+    out, lse = A.varlen_attn_fwd(q, k, v, cu, cu, 1500, 1500, 128**-0.5, causal)
+    got, atomic = (A.varlen_attn_bwd(do, q, k, v, out, lse, cu, cu, 1500, 1500, 128**-0.5, causal, deterministic=d)
+                   for d in (True, False))
+    for name, a, b, r in zip(("dk", "dv"), got[1:], atomic[1:], ref[1:]):
+        assert torch.equal(a, b), name
+        assert rel(a.float().cpu().numpy(), r) <= TOL, name
