@@ -216,8 +216,9 @@ int siq_attn_rope_bwd_plan(const void* q_embed, const void* k, const void* v, co
  * exactly 0.
  *
  * The logits are produced chunk_tokens rows at a time: only the softmax
- * numerators of one chunk (chunk_tokens x vocab bf16, each relative to the max
- * of its 256-column tile) ever exist, in the workspace; chunks count rows
+ * numerators of one chunk (chunk_tokens x vocab bf16, each relative to its
+ * row's label logit, or to a larger one where that is more than 2^60 too low)
+ * ever exist, in the workspace; chunks count rows
  * whose label counts (ignored rows are compacted away first).  Over two
  * chunks dweight is summed in dweight itself (the first chunk's sum rounded to
  * bf16 once); over more it is summed in an fp32 [vocab, hdim] workspace

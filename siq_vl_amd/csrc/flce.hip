@@ -15,19 +15,37 @@
 // only (each workgroup reads the valid count on the device and returns early
 // past it), and dH rows are scattered back to their positions.
 //
+// Each row has a reference: its label logit in log2 units, from a dot product
+// of its own (any value not far below the row's maximum does; every logit it
+// can be exceeded by is caught below).  Softmax numerators are taken relative
+// to it, so one factor per row turns them into probabilities, and the
+// gradient products take them as they are.
+//
 // Pipeline per chunk of C compacted rows (the only logits-sized buffer is one
 // chunk's softmax numerators):
 //  1. logits GEMM  Z^T = W H_c^T (MFMA, 256x256 tiles, K = hdim).  The epilogue
-//     never writes z: per (token, 256-column vocab tile) it keeps the tile
-//     max m and the sum s of exp(z - m) (the chunked-vocab logsumexp), the
-//     label logit z_y, and E = exp(z - m) in bf16 (a value in (0, 1], so bf16
-//     keeps full relative precision however large the logits are).
-//  2. row pass: lse = M + log(sum_t s_t exp(m_t - M)), the row's loss, and E
-//     rewritten in place as dZ = E * f_t - g * [v == y] with f_t = exp(m_t -
-//     lse) * g (g = inv_den, or 0 for an ignored row): one multiply per element,
-//     once for both gradient GEMMs.
-//  3. dH GEMM  dH_c^T = W^T dZ_c^T (split over the vocab) and
-//  4. dW GEMM  dW^T = H_c^T dZ_c.
+//     never writes z: it writes E = exp2(z2 - ref) in bf16 (whose exponent
+//     range is fp32's: full relative precision) and keeps, per (token,
+//     256-column vocab tile), the sum of E (the chunked-vocab logsumexp), and
+//     the label logit z_y.  A tile whose sum says that the reference is more
+//     than 2^60 below some logit is redone relative to its own maximum, which
+//     is recorded.
+//  2. row pass over those sums: lse = ref + log2(sum), the row's loss, its
+//     factor f = 2^(ref - lse) inv_den and its label weight w = (p_y - 1)
+//     inv_den; E at the label is set to zero (the label's term is added in
+//     fp32 instead); rows with redone tiles have their E brought to one
+//     reference; for dW, H's rows are scaled by f and the rows sorted by
+//     label.
+//  3. dH GEMM  dH_c^T = W^T E_c^T (split over the vocab), dH = f (sum over the
+//     splits) + w W[y], and
+//  4. dW GEMM  dW^T = (f H_c)^T E_c, plus the sums of w H over the rows of
+//     each label.
+// So dZ = (softmax - onehot) inv_den never exists: E is written once and read
+// twice, where a pass between the products read it and wrote dZ (1.5 of 14.8
+// ms at 16384 rows x 1536, V = 151936, 340 of 1970 us at 4099 x 896).  E is
+// rounded once on its way into dH (dZ was twice); in dW one rounding of E and
+// one of f H replace E's two; the label terms, which dominate both gradients,
+// are exact.
 // With several chunks dW accumulates over them: in dW itself (bf16) when the
 // valid rows span two chunks, in an fp32 workspace when they span more;
 // whether a chunk starts, continues or finishes that sum is decided on the
@@ -35,10 +53,11 @@
 // reduction has a fixed order, so results are bitwise reproducible.
 //
 // Loss only (no gradient wanted, e.g. evaluation under torch.no_grad): the
-// logits epilogue keeps its tile max / sum and z_y but stores no E, the row
-// pass stops at the loss, and neither gradient GEMM runs.
+// logits epilogue keeps its tile sums and z_y but stores no E, the row pass
+// stops at the loss, and neither gradient GEMM runs.
 #include "flce.h"
 #include "gemm.h"
+#include "ids.h"
 
 namespace siq {
 
@@ -49,15 +68,20 @@ using namespace gemm;
 constexpr int kVT = BI;  // vocab columns per logits tile
 
 // ---------------------------------------------------------------- logits
+// A tile sum at or above this (or not a number) means the row's reference is
+// too low for the tile.
+constexpr float kRefLimit = 0x1p60f;
+
 struct LogitsArgs {
   GOp W, H;               // W [V, hdim], H = hidden rows of the chunk [nc, hdim]
   const int64_t* y;       // chunk labels
+  const float* ref;       // [nc] row references (log2 units)
   bf16* E;                // [nc, V]
-  float* mpart;           // [nc, nvt] tile max (log2 units)
-  float* spart;           // [nc, nvt] tile sum of exp2(z2 - m)
+  float* spart;           // [nvt, ldp] tile sum of exp2(z2 - ref); negated for a redone tile
+  float* mpart;           // [nvt, ldp] a redone tile's own reference
   float* zy;              // [nc] label logit (natural units)
   const int64_t* nvalid;  // valid (compacted) rows in all chunks
-  int64_t V, nc, nvt, c0;
+  int64_t V, nc, c0, ldp;
   int nI, nJ;
   int store_e;            // 0: loss only, E is not needed
 };
@@ -68,15 +92,26 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
   if (!tile_of(p.nI, p.nJ, 4, ti, tj)) return;
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
   if (j0 >= *p.nvalid - p.c0) return;  // token tile holds no valid row
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
+  const int wi = w & 1, wj = w >> 1;
+  // accumulator (a, b, r) holds z for vocab row vbase + wave_row(a, wi) + 16 (r / 8) + (r % 8) and token
+  // column j0 + wave_col(b, wj) + l32
+  const int64_t vbase = i0 + 8 * h;
+  // the tokens' references, and their labels' offsets from the tile (-1: elsewhere)
+  float ref[2];
+  int rel[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int64_t tok = min(j0 + wave_col(b, wj) + l32, p.nc - 1);
+    ref[b] = p.ref[tok];
+    const int64_t d = p.y[tok] - vbase;
+    rel[b] = d >= 0 && d < 256 ? (int)d : -1;
+  }
   f32x16 acc[4][2];
   gemm_core<true, true, false>(smem, p.W, p.H, i0, j0, 0, p.W.cols, acc);
 
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
-  const int wi = w & 1, wj = w >> 1;
   float* red = reinterpret_cast<float*>(smem);  // [2][256]
-  // accumulator (a, b, r) holds z for vocab row vbase + wave_row(a, wi) + 16 (r / 8) + (r % 8) and token
-  // j0 + 64 wj + 32 b + l32.  Only the last vocab tile has rows past V: masked there alone.
-  const int64_t vbase = i0 + 8 * h;
+  // only the last vocab tile has rows past V: masked there alone
   if (i0 + BI > p.V) {
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -86,45 +121,9 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
         for (int r = 0; r < 16; ++r)
           if (vbase + wave_row(a, wi) + 16 * (r >> 3) + (r & 7) >= p.V) acc[a][b][r] = -INFINITY;
   }
-  float mt[2];
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    float mx = -INFINITY;
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc[a][b][r]);
-    // tile max in log2 units (scaling by log2 e > 0 commutes with the max)
-    mx = wave_max_xor32(mx) * kLog2e;
-    if (h == 0) red[wi * 256 + wave_col(b, wj) + l32] = mx;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int col = wave_col(b, wj) + l32;
-    mt[b] = fmaxf(red[col], red[256 + col]);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int col = wave_col(b, wj) + l32;
-    const int64_t tok = j0 + col;
-    const bool tv = tok < p.nc;
-    // the label logit: held by at most one lane of the workgroup, for one
-    // vocab tile in ~600 -- located with one range test per token
-    const int64_t rel64 = (tv ? p.y[tok] : -1) - vbase;
-    const bool hit = rel64 >= 0 && rel64 < 256 && ((rel64 >> 6) & 1) == wi && ((rel64 >> 3) & 1) == 0;
-    if (__any(hit)) {
-      const int rel = (int)rel64 - 64 * wi;
-      float zsel = 0.f;
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (hit && rel == wave_row(a, 0) + 16 * (r >> 3) + (r & 7)) zsel = acc[a][b][r];
-      if (hit) p.zy[tok] = zsel;
-    }
-    const float m2 = mt[b];
+  // E of column b relative to m2 (stored where `store`), and its sum over the tile's rows of this wave
+  auto numerators = [&](int b, float m2, bool store) {
+    const int64_t tok = j0 + wave_col(b, wj) + l32;
     float sum = 0.f;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
@@ -138,10 +137,66 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
           sum += e;
           e8[i] = (bf16)e;
         }
-        if (p.store_e && tv && v0 < p.V) st_bf16x8(p.E + tok * p.V + v0, e8);
+        if (store && v0 < p.V) st_bf16x8(p.E + tok * p.V + v0, e8);
       }
     }
-    sum = wave_sum_xor32(sum);
+    return half_sum(sum);
+  };
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int col = wave_col(b, wj) + l32;
+    const int64_t tok = j0 + col;
+    const bool tv = tok < p.nc;
+    // the label logit: held by at most one lane of the workgroup, for one
+    // vocab tile in ~600 -- located with one range test per token
+    const bool hit = tv && rel[b] >= 0 && ((rel[b] >> 6) & 1) == wi && ((rel[b] >> 3) & 1) == 0;
+    if (__any(hit)) {
+      const int r0 = rel[b] - 64 * wi;
+      float zsel = 0.f;
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (hit && r0 == wave_row(a, 0) + 16 * (r >> 3) + (r & 7)) zsel = acc[a][b][r];
+      if (hit) p.zy[tok] = zsel;
+    }
+    const float sum = numerators(b, ref[b], p.store_e && tv);
+    if (h == 0) red[wi * 256 + col] = sum;
+  }
+  __syncthreads();
+  float tot[2];
+  bool redo = false;
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int col = wave_col(b, wj) + l32;
+    const int64_t tok = j0 + col;
+    tot[b] = red[col] + red[256 + col];
+    redo |= tok < p.nc && !(tot[b] < kRefLimit);
+    if (wi == 0 && h == 0 && tok < p.nc) p.spart[(int64_t)ti * p.ldp + tok] = tot[b];
+  }
+  if (!__syncthreads_or(redo)) return;
+  // columns whose reference is too low: the same relative to the tile's maximum
+  float mt[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc[a][b][r]);
+    // log2 units (scaling by log2 e > 0 commutes with the max)
+    mx = half_max(mx) * kLog2e;
+    if (h == 0) red[wi * 256 + wave_col(b, wj) + l32] = mx;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < 2; ++b) mt[b] = fmaxf(red[wave_col(b, wj) + l32], red[256 + wave_col(b, wj) + l32]);
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int col = wave_col(b, wj) + l32;
+    const bool bad = j0 + col < p.nc && !(tot[b] < kRefLimit);
+    const float sum = numerators(b, mt[b], p.store_e && bad);
     if (h == 0) red[wi * 256 + col] = sum;
   }
   __syncthreads();
@@ -150,9 +205,9 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
     for (int b = 0; b < 2; ++b) {
       const int col = wave_col(b, wj) + l32;
       const int64_t tok = j0 + col;
-      if (tok < p.nc) {
-        p.mpart[tok * p.nvt + ti] = mt[b];
-        p.spart[tok * p.nvt + ti] = red[col] + red[256 + col];
+      if (tok < p.nc && !(tot[b] < kRefLimit)) {
+        p.spart[(int64_t)ti * p.ldp + tok] = -(red[col] + red[256 + col]);
+        p.mpart[(int64_t)ti * p.ldp + tok] = mt[b];
       }
     }
   }
@@ -160,113 +215,279 @@ __global__ __launch_bounds__(NT) void flce_logits_kernel(const LogitsArgs p) {
 
 // ---------------------------------------------------------------- row pass
 struct RowArgs {
-  const float* mpart;    // [nc, nvt] tile max (log2 units)
-  const float* spart;    // [nc, nvt] tile sum of exp2(z2 - m)
+  const float* spart;    // [nvt, ldp] tile sums (negative: redone, relative to mpart)
+  const float* mpart;
+  const float* ref;      // [nc] row references (log2 units)
   const float* zy;
   const int64_t* y;      // chunk labels
-  bf16* E;               // [nc, V]: E on entry, dZ on exit
+  bf16* E;               // [nc, V]
+  bf16* H;               // [nc, hdim] compacted rows: scaled by f (need_dw)
+  float* f;              // [nc] factors of E
+  float* wt;             // [nc] weights of the label terms
   float* loss_row;       // [nc] (chunk slice)
   const float* invden;
   const int64_t* nvalid;
-  int64_t nc, nvt, V, ignore_index, c0;
-  int rewrite;           // 0: loss only (E was never stored)
+  uint64_t* keys;        // [nsort, kIdChunk] rows sorted by label
+  int32_t* slot;         // [V] cleared
+  int64_t nc, nvt, V, hdim, ignore_index, c0, ldp;
+  int nsort;             // sorting workgroups (0 without dW)
+  int grads;             // 0: loss only (E was never stored)
 };
 
-// One workgroup (four waves) per token row.  lse2 = M + log2(sum_t s_t
-// 2^(m_t - M)); then the row of E becomes dZ = E * f_t - g [v == y], f_t =
-// 2^(m_t - lse2) * g, in fp32 and rounded to bf16 once (zero for an ignored
-// row: g = 0).  The factors f_t are computed once per tile into LDS, in
-// segments of kRowSegTiles tiles, so the streaming loop does one LDS read and
-// eight multiplies per 16 bytes.  Four waves per row (rather than one) split
-// the per-row reductions over the tile statistics, which precede the
-// streaming, four ways.
-constexpr int kRowSegTiles = 1024, kRowThreads = 256;
+// Workgroups [0, nsort) sort the chunk's labels; each of the others takes 64
+// rows.  Sixteen waves read the rows' tile sums (lane = row, so each read is
+// 256 contiguous bytes), added in a fixed order; the rest of the work is per
+// row.
+constexpr int kRowThreads = 1024, kRowRows = 64;
 __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) {
-  constexpr int RT = kRowThreads, NWR = RT / 64;
-  __shared__ float fsh[kRowSegTiles];
-  __shared__ float red[NWR];
+  constexpr int NWR = kRowThreads / 64;
+  __shared__ union {
+    uint64_t sk[kIdChunk];
+    struct {
+      float sum[NWR][kRowRows], mx[NWR][kRowRows], f[kRowRows], top[kRowRows];
+    } r;
+  } sh;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int64_t row = blockIdx.x;
-  // rows past the last token tile with a valid row are read by no GEMM
-  if (row >= p.nc || row >= ((*p.nvalid - p.c0 + BJ - 1) / BJ) * BJ) return;
-  const float* m = p.mpart + row * p.nvt;
-  const float* s = p.spart + row * p.nvt;
-  float mx = -INFINITY;
-  for (int64_t t = tid; t < p.nvt; t += RT) mx = fmaxf(mx, m[t]);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-  if (lane == 0) red[w] = mx;
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NWR; ++i) mx = fmaxf(mx, red[i]);
-  __syncthreads();  // red is reused below
-  float sum = 0.f;
-  for (int64_t t = tid; t < p.nvt; t += RT) sum += s[t] * exp2f_fast(m[t] - mx);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
-  if (lane == 0) red[w] = sum;
-  __syncthreads();
-  sum = 0.f;
-#pragma unroll
-  for (int i = 0; i < NWR; ++i) sum += red[i];  // fixed order: every thread gets the same sum
-  const float lse2 = mx + __log2f(sum);
-  const int64_t yv = p.y[row];
-  const bool valid = yv != p.ignore_index && yv >= 0 && yv < p.V;
-  const float gv = valid ? *p.invden : 0.f;
-  if (tid == 0) p.loss_row[row] = valid ? lse2 * kLn2 - p.zy[row] : 0.f;
-  if (!p.rewrite) return;
-  // dZ, 8 columns per thread per chunk (V is a multiple of 8, so a chunk never
-  // straddles the row end; 8 aligned columns never straddle a 256-column
-  // tile: chunk c lies in tile c / 32).  An ignored row's dZ is zero: written
-  // without reading E.
-  bf16* e = p.E + row * p.V;
-  const int64_t nchunk = p.V / 8;
-  if (gv == 0.f) {
-    for (int64_t c = tid; c < nchunk; c += RT) st_bf16x8(e + 8 * c, zero_bf16x8());
+  const int64_t nv = min(p.nc, *p.nvalid - p.c0);  // valid rows of the chunk
+  if ((int)blockIdx.x < p.nsort) {
+    const int64_t base = (int64_t)blockIdx.x * kIdChunk;
+    const int len = (int)max((int64_t)0, min((int64_t)kIdChunk, nv - base));
+    int np2 = 64;
+    while (np2 < len) np2 <<= 1;
+    for (int i = tid; i < np2; i += kRowThreads)
+      sh.sk[i] = i < len ? ((uint64_t)p.y[base + i] << 32) | (uint32_t)i : kNoKey;
+    __syncthreads();
+    sort_keys(sh.sk, np2);
+    for (int i = tid; i < kIdChunk; i += kRowThreads) p.keys[base + i] = i < np2 ? sh.sk[i] : kNoKey;
     return;
   }
-  auto chunk = [&](const bf16x8& x, float fv, int64_t c) {
-    const int64_t v0 = 8 * c;
-    bf16x8 o;
+  const int blk = (int)blockIdx.x - p.nsort, nblk = (int)gridDim.x - p.nsort;
+  if (p.nsort > 0)
+    for (int64_t v = (int64_t)blk * kRowThreads + tid; v < p.V; v += (int64_t)nblk * kRowThreads) p.slot[v] = 0;
+  const int64_t r0 = (int64_t)blk * kRowRows;
+  if (r0 >= nv) return;
+  {
+    const int64_t row = min(r0 + lane, nv - 1);
+    const float rf = p.ref[row];
+    float sum = 0.f, mx = -INFINITY;  // of the tiles relative to ref; the redone tiles' largest reference
+    constexpr int U = 8;
+    for (int64_t t0 = w; t0 < p.nvt; t0 += NWR * U) {
+      float s[U];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = (bf16)((float)x[i] * fv);
-    const int64_t yrel = yv - v0;
-    if (yrel >= 0 && yrel < 8) {
+      for (int u = 0; u < U; ++u) s[u] = t0 + NWR * u < p.nvt ? p.spart[(t0 + NWR * u) * p.ldp + row] : 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = (i == yrel) ? (bf16)((float)x[i] * fv - gv) : o[i];
+      for (int u = 0; u < U; ++u) {
+        if (s[u] < 0.f)
+          mx = fmaxf(mx, p.mpart[(t0 + NWR * u) * p.ldp + row]);
+        else
+          sum += s[u];  // (a NaN too)
+      }
     }
-    st_bf16x8(e + v0, o);
-  };
-  // U chunks per thread in flight: thread chunks c + RT u sit in tiles
-  // c / 32 + (RT / 32) u (the pass streams E in and dZ out at the device's
-  // mixed read / write rate; deeper unrolling, loading the next chunks before
-  // this U's stores, and non-temporal accesses measured no faster)
-  constexpr int U = 8;
-  for (int64_t t0 = 0; t0 < p.nvt; t0 += kRowSegTiles) {
-    const int nt = (int)min((int64_t)kRowSegTiles, p.nvt - t0);
-    __syncthreads();  // the previous segment's factors are no longer read
-    for (int t = tid; t < nt; t += RT) fsh[t] = exp2f_fast(m[t0 + t] - lse2) * gv;
+    sh.r.sum[w][lane] = sum;
+    sh.r.mx[w][lane] = mx;
     __syncthreads();
-    const int64_t cb = 32 * t0, ce = min(nchunk, 32 * (t0 + nt));
-    int64_t c = cb + tid;
-    for (; c + RT * (U - 1) < ce; c += RT * U) {
-      bf16x8 x[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) x[u] = ld_bf16x8(e + 8 * (c + RT * u));
-      const int tb = (int)((c - cb) >> 5);
-#pragma unroll
-      for (int u = 0; u < U; ++u) chunk(x[u], fsh[tb + (RT / 32) * u], c + RT * u);
+    if (w == 0) {
+      sum = sh.r.sum[0][lane];
+      mx = sh.r.mx[0][lane];
+      for (int i = 1; i < NWR; ++i) {
+        sum += sh.r.sum[i][lane];
+        mx = fmaxf(mx, sh.r.mx[i][lane]);
+      }
+      float top = rf;  // the reference that E has after this pass
+      if (mx > -INFINITY) {
+        // redone tiles: everything relative to the largest reference
+        top = fmaxf(rf, mx);
+        sum *= exp2f_fast(rf - top);
+        for (int64_t t = 0; t < p.nvt; ++t) {
+          const float s = p.spart[t * p.ldp + row];
+          if (s < 0.f) sum -= s * exp2f_fast(p.mpart[t * p.ldp + row] - top);
+        }
+      }
+      const float lse2 = top + __log2f(sum);
+      const bool mine = r0 + lane < nv;
+      const int64_t y = p.y[row];
+      if (mine) p.loss_row[row] = lse2 * kLn2 - p.zy[row];
+      if (p.grads) {
+        const float g = *p.invden, f = exp2f_fast(top - lse2) * g;
+        if (mine) {
+          p.f[row] = f;
+          p.wt[row] = (exp2f_fast(__builtin_fmaf(p.zy[row], kLog2e, -lse2)) - 1.f) * g;
+          if (!(mx > -INFINITY)) p.E[row * p.V + y] = (bf16)0.f;
+        }
+        sh.r.f[lane] = f;
+        sh.r.top[lane] = mx > -INFINITY ? top : INFINITY;  // INFINITY: E is already relative to one reference
+      }
     }
-    for (; c < ce; c += RT) chunk(ld_bf16x8(e + 8 * c), fsh[(c - cb) >> 5], c);
+  }
+  if (!p.grads) return;
+  __syncthreads();
+  const int rows = (int)min((int64_t)kRowRows, nv - r0);
+  // rows with redone tiles: E of every tile brought to the common reference (8 columns never straddle a tile)
+  for (int r = 0; r < rows; ++r) {
+    const float top = sh.r.top[r];
+    if (top == INFINITY) continue;
+    const int64_t row = r0 + r, y = p.y[row];
+    const float rf = p.ref[row];
+    for (int64_t c = tid; c < p.V / 8; c += kRowThreads) {
+      const int64_t t = c / (kVT / 8);
+      const float fv = exp2f_fast((p.spart[t * p.ldp + row] < 0.f ? p.mpart[t * p.ldp + row] : rf) - top);
+      bf16x8 x = ld_bf16x8(p.E + row * p.V + 8 * c);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = 8 * c + i == y ? (bf16)0.f : (bf16)((float)x[i] * fv);
+      st_bf16x8(p.E + row * p.V + 8 * c, x);
+    }
+  }
+  if (p.nsort == 0) return;
+  const int gpr = (int)(p.hdim / 8);
+  for (int i = tid; i < rows * gpr; i += kRowThreads) {
+    const float f = sh.r.f[i / gpr];
+    bf16* hp = p.H + r0 * p.hdim + 8 * (int64_t)i;
+    bf16x8 x = ld_bf16x8(hp);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = (bf16)((float)x[k] * f);
+    st_bf16x8(hp, x);
+  }
+}
+
+// Label terms of dW: for each label of the chunk, the sum of w H over its
+// rows in fp32, in the slot of the label's first sorted key (lsum[slot],
+// slot[label] = that slot + 1).  One workgroup per key; the keys of a label
+// but its first one return at once.  Rounds of kLabelRound rows, listed one
+// per thread: wave k adds rows k, k + 4, ... of the round, eight in flight; the
+// waves' sums are added in order at the end.  Bound by the commonest label
+// (400 of 6912 rows where labels are Zipf-distributed): 77 us for 6912 rows x 1536.
+constexpr int kLabelRound = 256;
+struct LabelArgs {
+  const uint64_t* keys;  // [nsort, kIdChunk]
+  const bf16* H;         // [n, hdim] all rows, unscaled
+  const int32_t* rows;   // chunk's compacted row -> row of H
+  const float* wt;       // [nc]
+  float* lsum;           // [nsort * kIdChunk (rows that exist), hdim]
+  int32_t* slot;         // [V]
+  int64_t hdim;
+  int nsort;
+};
+__global__ __launch_bounds__(256) void flce_label_kernel(const LabelArgs p) {
+  constexpr int U = 3, R = 8, NWL = 4;
+  static_assert(kLabelRound == 64 * NWL, "a thread per listed row");
+  __shared__ int32_t row_sh[kLabelRound];
+  __shared__ float wt_sh[kLabelRound];
+  __shared__ __align__(16) float part_sh[NWL - 1][U * 64 * 8];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int64_t item = blockIdx.x;
+  const int c = (int)(item / kIdChunk), i = (int)(item % kIdChunk);
+  const uint64_t key = p.keys[item];
+  if (key == kNoKey) return;
+  const uint32_t v = (uint32_t)(key >> 32);
+  if (i > 0 && (uint32_t)(p.keys[item - 1] >> 32) == v) return;  // not the label's first key in this chunk
+  // lane l: the label's run [first, first + len) in chunk g0 + l
+  int first = 0, incl = 0, total = 0;
+  auto runs = [&](int g0) {
+    int len = 0;
+    if (g0 + lane < p.nsort) {
+      const int2 r = id_run(p.keys + (int64_t)(g0 + lane) * kIdChunk, v);
+      first = r.x;
+      len = r.y - r.x;
+    }
+    incl = len;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    total = __shfl(incl, 63);
+    return len;
+  };
+  for (int g0 = 0; g0 < c; g0 += 64) {
+    const int len = runs(g0);
+    if (__ballot(len > 0 && g0 + lane < c)) return;  // an earlier chunk holds the label
+  }
+  if (tid == 0) p.slot[v] = (int32_t)item + 1;
+  const int64_t nvec = p.hdim / 8;
+  for (int64_t p0 = 0; p0 < nvec; p0 += 64 * U) {
+    float acc[U][8];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[u][e] = 0.f;
+    for (int g0 = c; g0 < p.nsort; g0 += 64) {
+      runs(g0);
+      for (int rank0 = 0; rank0 < total; rank0 += kLabelRound) {
+        const int have = min(kLabelRound, total - rank0);
+        __syncthreads();  // the last round's list is read no more
+        // row rank0 + tid of the group's runs: in the first chunk whose inclusive count exceeds it
+        int q = 0, base = 0;
+        for (int j = 0; j < 64 && g0 + j < p.nsort; ++j) {
+          const int upto = __builtin_amdgcn_readlane(incl, j);
+          q = upto <= rank0 + tid ? j + 1 : q;
+          base = upto <= rank0 + tid ? upto : base;
+        }
+        const int at = __shfl(first, q & 63) + rank0 + tid - base;
+        if (tid < have) {
+          const uint32_t k = (uint32_t)((g0 + q) * kIdChunk) + (uint32_t)p.keys[(int64_t)(g0 + q) * kIdChunk + at];
+          row_sh[tid] = p.rows[k];
+          wt_sh[tid] = p.wt[k];
+        }
+        __syncthreads();
+        for (int t0 = w; t0 < have; t0 += NWL * R) {
+          bf16x8 x[R][U];
+          float wr[R];
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const int t = min(t0 + NWL * r, have - 1);
+            wr[r] = wt_sh[t];
+            const bf16* src = p.H + (int64_t)row_sh[t] * p.hdim;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int64_t ch = min(p0 + 64 * u + lane, nvec - 1);
+              x[r][u] = ld_bf16x8(src + 8 * ch);
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            if (t0 + NWL * r >= have) break;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+              for (int e = 0; e < 8; ++e) acc[u][e] = __builtin_fmaf(wr[r], (float)x[r][u][e], acc[u][e]);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    if (w > 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part_sh[w - 1][(u * 64 + lane) * 8 + e] = acc[u][e];
+    }
+    __syncthreads();
+    if (w == 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t ch = p0 + 64 * u + lane;
+        if (ch >= nvec) continue;
+#pragma unroll
+        for (int k = 0; k < NWL - 1; ++k)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[u][e] += part_sh[k][(u * 64 + lane) * 8 + e];
+        float* dst = p.lsum + item * p.hdim + 8 * ch;
+        *reinterpret_cast<f32x4*>(dst) = f32x4{acc[u][0], acc[u][1], acc[u][2], acc[u][3]};
+        *reinterpret_cast<f32x4*>(dst + 4) = f32x4{acc[u][4], acc[u][5], acc[u][6], acc[u][7]};
+      }
+    }
   }
 }
 
 // ---------------------------------------------------------------- dH
 struct DhArgs {
   GOp Wt;        // W [V, hdim] read as A[i = h][k = v]
-  GOp E;         // dZ [nc, V] read as B[j = tok][k = v]
-  bf16* dh;      // dhidden rows of the chunk [nc, hdim] (used when splits == 1)
+  GOp E;         // [nc, V] read as B[j = tok][k = v]
+  bf16* dh;      // dhidden [n, hdim] (used when splits == 1)
   float* part;   // [splits, nc, hdim]
+  const float* f;         // [nc] row factors, label weights, labels (used when splits == 1)
+  const float* wt;
+  const int64_t* y;
   const int32_t* rows;    // compacted row -> original row (whole batch)
   const int64_t* nvalid;
   int64_t hdim, nc, kper, c0;
@@ -274,7 +495,7 @@ struct DhArgs {
 };
 
 // dH work: a unit is one (token tile, vocab split); its nI hdim tiles share
-// the unit's dZ slab, so they run as consecutive blocks on one XCD (block b
+// the unit's E slab, so they run as consecutive blocks on one XCD (block b
 // runs on XCD b % 8).  Units are dealt out over the XCDs in turn, splits of a
 // token tile on different XCDs: every XCD gets the same number of units, also
 // when the token tiles past the valid rows (which return at once) are many --
@@ -308,6 +529,8 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
     if (tok >= p.nc) continue;
     if (p.splits == 1 && tok >= nv) continue;  // padding row
     const int64_t orow = p.splits == 1 ? p.rows[p.c0 + tok] : 0;
+    const float f = p.splits == 1 ? p.f[tok] : 0.f, wt = p.splits == 1 ? p.wt[tok] : 0.f;
+    const bf16* wy = p.Wt.base + (p.splits == 1 ? p.y[tok] : 0) * p.hdim;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -315,9 +538,10 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
         const int64_t hh = i0 + wave_row(a, wi) + 16 * jj + 8 * h;
         if (hh >= p.hdim) continue;
         if (p.splits == 1) {
+          const bf16x8 l = ld_bf16x8(wy + hh);
           bf16x8 o;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) o[i] = (bf16)acc[a][b][8 * jj + i];
+          for (int i = 0; i < 8; ++i) o[i] = (bf16)__builtin_fmaf(f, acc[a][b][8 * jj + i], wt * (float)l[i]);
           st_bf16x8(p.dh + orow * p.hdim + hh, o);
         } else {
           float* dst = p.part + ((int64_t)split * p.nc + tok) * p.hdim + hh;
@@ -334,37 +558,39 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
   }
 }
 
-// dH rows of the chunk: the splits' fp32 partial sums added in split order,
-// each compacted row written to its original row.
-__global__ __launch_bounds__(256) void flce_dh_sum_kernel(const float* __restrict__ part, bf16* __restrict__ dh,
-                                                          const int32_t* __restrict__ rows,
-                                                          const int64_t* __restrict__ nvalid, int64_t c0, int64_t nc,
-                                                          int64_t hdim, int splits) {
+// dH rows of the chunk: f times the splits' fp32 partial sums, added in split
+// order, plus the label term w W[y]; each compacted row written to its
+// original row.
+__global__ __launch_bounds__(256) void flce_dh_sum_kernel(const DhArgs p) {
   // part is [splits][nc * hdim]; groups of 8 elements, hdim / 8 per row
-  const int64_t nv = min(nc, *nvalid - c0);
-  const int64_t gpr = hdim / 8, stride = nc * hdim;
+  const int64_t nv = min(p.nc, *p.nvalid - p.c0);
+  const int64_t gpr = p.hdim / 8, stride = p.nc * p.hdim;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nv * gpr; i += (int64_t)gridDim.x * 256) {
-    f32x4 a = *reinterpret_cast<const f32x4*>(part + 8 * i);
-    f32x4 b = *reinterpret_cast<const f32x4*>(part + 8 * i + 4);
-    for (int s = 1; s < splits; ++s) {
-      a += *reinterpret_cast<const f32x4*>(part + s * stride + 8 * i);
-      b += *reinterpret_cast<const f32x4*>(part + s * stride + 8 * i + 4);
+    const int64_t r = i / gpr, col = 8 * (i - r * gpr);
+    const bf16x8 l = ld_bf16x8(p.Wt.base + p.y[r] * p.hdim + col);
+    f32x4 a = *reinterpret_cast<const f32x4*>(p.part + 8 * i);
+    f32x4 b = *reinterpret_cast<const f32x4*>(p.part + 8 * i + 4);
+    for (int s = 1; s < p.splits; ++s) {
+      a += *reinterpret_cast<const f32x4*>(p.part + s * stride + 8 * i);
+      b += *reinterpret_cast<const f32x4*>(p.part + s * stride + 8 * i + 4);
     }
+    const float f = p.f[r], wt = p.wt[r];
     bf16x8 o;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      o[k] = (bf16)a[k];
-      o[4 + k] = (bf16)b[k];
+      o[k] = (bf16)__builtin_fmaf(f, a[k], wt * (float)l[k]);
+      o[4 + k] = (bf16)__builtin_fmaf(f, b[k], wt * (float)l[4 + k]);
     }
-    const int64_t r = i / gpr;
-    st_bf16x8(dh + (int64_t)rows[c0 + r] * hdim + 8 * (i - r * gpr), o);
+    st_bf16x8(p.dh + (int64_t)p.rows[p.c0 + r] * p.hdim + col, o);
   }
 }
 
 // ---------------------------------------------------------------- dW
 struct DwArgs {
-  GOp Ht;        // hidden rows of the chunk [nc, hdim] read as A[i = h][k = tok]
-  GOp Et;        // dZ [nc, V] read as B[j = v][k = tok]
+  GOp Ht;        // hidden rows of the chunk [nc, hdim], scaled by f, read as A[i = h][k = tok]
+  GOp Et;        // E [nc, V] read as B[j = v][k = tok]
+  const int32_t* slot;   // [V] label terms: row of lsum + 1, or 0
+  const float* lsum;     // [rows, hdim]
   bf16* dw;      // [V, hdim]
   float* acc32;  // [V, hdim] fp32 accumulator across chunks
   const int64_t* nvalid;
@@ -403,6 +629,8 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
   for (int b = 0; b < 2; ++b) {
     const int64_t v = j0 + wave_col(b, wj) + l32;
     if (v >= p.V) continue;
+    const int sl = nv > 0 ? p.slot[v] : 0;
+    const float* lt = p.lsum + (int64_t)(sl - 1) * p.hdim;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -414,6 +642,10 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
         for (int i = 0; i < 4; ++i) {
           lo[i] = acc[a][b][8 * jj + i];
           hi[i] = acc[a][b][8 * jj + 4 + i];
+        }
+        if (sl > 0) {
+          lo += *reinterpret_cast<const f32x4*>(lt + hh);
+          hi += *reinterpret_cast<const f32x4*>(lt + hh + 4);
         }
         float* a32 = p.acc32 + v * p.hdim + hh;
         if (mode == 2 || mode == 3) {
@@ -528,24 +760,41 @@ __global__ __launch_bounds__(1024) void flce_compact_kernel(const int64_t* __res
   if (tid == 0) *nvalid = carry_sh;
 }
 
-// The compacted operands: Hc[k] = H[rows[k]], yc[k] = y[rows[k]] for k < nvalid,
-// zero rows and ignore_index up to the next multiple of 256 (the padding the
-// GEMM tiles read); and dH = 0 on every row whose label does not count.  One
-// wave per row, 16 bytes per lane per step.
-__global__ __launch_bounds__(256) void flce_gather_kernel(const bf16* __restrict__ H, const int64_t* __restrict__ y,
+// The compacted operands: Hc[k] = H[rows[k]], yc[k] = y[rows[k]] and the row's
+// reference, its label logit in log2 units, for k < nvalid; zero rows,
+// ignore_index and 0 up to the next multiple of 256 (the padding the GEMM
+// tiles read); and dH = 0 on every row whose label does not count.  One wave
+// per row, 16 bytes per lane per step.
+__global__ __launch_bounds__(256) void flce_gather_kernel(const bf16* __restrict__ H, const bf16* __restrict__ W,
+                                                          const int64_t* __restrict__ y,
                                                           const int32_t* __restrict__ rows,
                                                           const int64_t* __restrict__ nvalid, int64_t n, int64_t hdim,
                                                           int64_t V, int64_t ignore_index, bf16* __restrict__ Hc,
-                                                          int64_t* __restrict__ yc, bf16* __restrict__ dh) {
+                                                          int64_t* __restrict__ yc, float* __restrict__ ref,
+                                                          bf16* __restrict__ dh) {
   const int lane = threadIdx.x & 63;
   const int64_t nvec = hdim / 8, nv = *nvalid, npad = ((nv + 255) / 256) * 256;
   const int64_t wstep = (int64_t)gridDim.x * 4;
   for (int64_t k = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); k < npad; k += wstep) {
     const bool real = k < nv;
     const int64_t src = real ? rows[k] : 0;
-    if (lane == 0) yc[k] = real ? y[src] : ignore_index;
-    for (int64_t c = lane; c < nvec; c += 64)
-      st_bf16x8(Hc + k * hdim + 8 * c, real ? ld_bf16x8(H + src * hdim + 8 * c) : zero_bf16x8());
+    const int64_t yk = real ? y[src] : ignore_index;
+    float dot = 0.f;
+    for (int64_t c = lane; c < nvec; c += 64) {
+      const bf16x8 x = real ? ld_bf16x8(H + src * hdim + 8 * c) : zero_bf16x8();
+      if (real) {
+        const bf16x8 wy = ld_bf16x8(W + yk * hdim + 8 * c);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dot = __builtin_fmaf((float)x[i], (float)wy[i], dot);
+      }
+      st_bf16x8(Hc + k * hdim + 8 * c, x);
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) dot += __shfl_xor(dot, o);
+    if (lane == 0) {
+      yc[k] = yk;
+      ref[k] = dot * kLog2e;
+    }
   }
   if (dh == nullptr) return;  // loss only
   for (int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < n; t += wstep) {
@@ -596,8 +845,9 @@ __global__ __launch_bounds__(256) void zero_bf16_kernel(bf16* __restrict__ x, in
 
 // ---------------------------------------------------------------- workspace
 struct Layout {
-  size_t invden, loss_row, mpart, spart, zy, E, part, acc32, rows, hc, yc, total;
+  size_t invden, loss_row, mpart, spart, zy, f, wt, E, part, acc32, rows, hc, yc, ref, keys, slot, lsum, total;
   int64_t chunk, nvt, splits;
+  int nsort;  // sorted runs of a chunk's labels (dW only)
 };
 
 size_t al(size_t x) { return (x + 255) & ~size_t(255); }
@@ -611,7 +861,7 @@ int dh_splits(int64_t hdim, int64_t chunk) {
 }
 
 // need_dh false: loss only (no E, no gradient buffers); its chunks only bound
-// the per-(row, vocab tile) max / sum buffers, so they are large.
+// the per-(row, vocab tile) sum buffers, so they are large.
 constexpr int64_t kLossChunk = 32768;
 
 Layout layout(int64_t n, int64_t hdim, int64_t V, int64_t chunk, bool need_dh, bool need_dw) {
@@ -635,6 +885,10 @@ Layout layout(int64_t n, int64_t hdim, int64_t V, int64_t chunk, bool need_dh, b
   off += al(sizeof(float) * (size_t)(L.chunk * L.nvt));
   L.zy = off;
   off += al(sizeof(float) * (size_t)L.chunk);
+  L.f = off;
+  if (need_dh) off += al(sizeof(float) * (size_t)L.chunk);
+  L.wt = off;
+  if (need_dh) off += al(sizeof(float) * (size_t)L.chunk);
   L.E = off;
   if (need_dh) off += al(sizeof(bf16) * (size_t)(L.chunk * V));
   L.part = off;
@@ -650,6 +904,16 @@ Layout layout(int64_t n, int64_t hdim, int64_t V, int64_t chunk, bool need_dh, b
   off += al(sizeof(bf16) * (size_t)(npad * hdim));
   L.yc = off;
   off += al(sizeof(int64_t) * (size_t)npad);
+  L.ref = off;
+  off += al(sizeof(float) * (size_t)npad);
+  L.nsort = need_dw ? (int)((L.chunk + kIdChunk - 1) / kIdChunk) : 0;
+  L.keys = off;
+  off += al(sizeof(uint64_t) * (size_t)L.nsort * kIdChunk);
+  L.slot = off;
+  if (need_dw) off += al(sizeof(int32_t) * (size_t)V);
+  // the label terms' sums, one row for each row of the chunk: in dH's partial sums, which are read by then
+  L.lsum = L.splits > 1 ? L.part : off;
+  if (need_dw && L.splits <= 1) off += al(sizeof(float) * (size_t)(L.chunk * hdim));
   L.total = off;
   return L;
 }
@@ -677,6 +941,12 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
   int32_t* rows = reinterpret_cast<int32_t*>(ws + L.rows);
   bf16* hcomp = reinterpret_cast<bf16*>(ws + L.hc);
   int64_t* ycomp = reinterpret_cast<int64_t*>(ws + L.yc);
+  float* ref = reinterpret_cast<float*>(ws + L.ref);
+  float* frow = reinterpret_cast<float*>(ws + L.f);
+  float* wrow = reinterpret_cast<float*>(ws + L.wt);
+  uint64_t* keys = reinterpret_cast<uint64_t*>(ws + L.keys);
+  int32_t* slot = reinterpret_cast<int32_t*>(ws + L.slot);
+  float* lsum = reinterpret_cast<float*>(ws + L.lsum);
   const int64_t V = a.vocab, Hd = a.hdim;
 
   hipLaunchKernelGGL(flce_count_kernel, dim3(1), dim3(1024), 0, stream, a.labels, a.n, V, a.ignore_index,
@@ -686,8 +956,8 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
   if (a.n > 0) {
     int64_t blocks = (a.n + 3) / 4;
     if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(flce_gather_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a.hidden, a.labels, rows,
-                       nvalid, a.n, Hd, V, a.ignore_index, hcomp, ycomp, grads ? a.dhidden : nullptr);
+    hipLaunchKernelGGL(flce_gather_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a.hidden, a.weight, a.labels, rows,
+                       nvalid, a.n, Hd, V, a.ignore_index, hcomp, ycomp, ref, grads ? a.dhidden : nullptr);
   }
   // chunks of compacted rows: the host sizes them for n rows; those past the
   // valid count return at once
@@ -695,13 +965,14 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
   for (int64_t ci = 0; ci < nchunks; ++ci) {
     const int64_t c0 = ci * L.chunk;
     const int64_t nc = (a.n - c0) < L.chunk ? (a.n - c0) : L.chunk;
-    const bf16* Hc = hcomp + c0 * Hd;
+    bf16* Hc = hcomp + c0 * Hd;
     const int64_t* yc = ycomp + c0;
 
     LogitsArgs lg{};
     lg.W = GOp{a.weight, Hd, V, Hd};
     lg.H = GOp{Hc, Hd, nc, Hd};
     lg.y = yc;
+    lg.ref = ref + c0;
     lg.E = E;
     lg.mpart = mpart;
     lg.spart = spart;
@@ -710,7 +981,7 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
     lg.c0 = c0;
     lg.V = V;
     lg.nc = nc;
-    lg.nvt = L.nvt;
+    lg.ldp = L.chunk;
     lg.nI = (int)L.nvt;
     lg.nJ = (int)((nc + BJ - 1) / BJ);
     lg.store_e = grads ? 1 : 0;
@@ -723,19 +994,29 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
     RowArgs rw{};
     rw.mpart = mpart;
     rw.spart = spart;
+    rw.ref = ref + c0;
     rw.zy = zy;
     rw.y = yc;
     rw.E = E;
+    rw.H = Hc;
+    rw.f = frow;
+    rw.wt = wrow;
     rw.loss_row = loss_row + c0;
     rw.invden = invden;
     rw.nvalid = nvalid;
+    rw.keys = keys;
+    rw.slot = slot;
     rw.c0 = c0;
     rw.nc = nc;
     rw.nvt = L.nvt;
     rw.V = V;
+    rw.hdim = Hd;
+    rw.ldp = L.chunk;
     rw.ignore_index = a.ignore_index;
-    rw.rewrite = grads ? 1 : 0;
-    hipLaunchKernelGGL(flce_row_kernel, dim3((unsigned)nc), dim3(kRowThreads), 0, stream, rw);
+    rw.nsort = L.nsort;
+    rw.grads = grads ? 1 : 0;
+    hipLaunchKernelGGL(flce_row_kernel, dim3((unsigned)(L.nsort + (nc + kRowRows - 1) / kRowRows)), dim3(kRowThreads), 0,
+                       stream, rw);
     if (!grads) continue;
 
     DhArgs dh{};
@@ -743,6 +1024,9 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
     dh.E = GOp{E, V, nc, V};
     dh.dh = a.dhidden;
     dh.part = part;
+    dh.f = frow;
+    dh.wt = wrow;
+    dh.y = yc;
     dh.rows = rows;
     dh.nvalid = nvalid;
     dh.c0 = c0;
@@ -764,14 +1048,26 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
       const int64_t nvec = nc * Hd / 8;
       int64_t blocks = (nvec + 255) / 256;
       if (blocks > 4096) blocks = 4096;
-      hipLaunchKernelGGL(flce_dh_sum_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, part, a.dhidden, rows,
-                         nvalid, c0, nc, Hd, (int)L.splits);
+      hipLaunchKernelGGL(flce_dh_sum_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, dh);
     }
 
-    if (grads && a.dweight != nullptr) {
+    if (a.dweight != nullptr) {
+      LabelArgs la{};
+      la.keys = keys;
+      la.H = a.hidden;
+      la.rows = rows + c0;
+      la.wt = wrow;
+      la.lsum = lsum;
+      la.slot = slot;
+      la.hdim = Hd;
+      la.nsort = L.nsort;
+      hipLaunchKernelGGL(flce_label_kernel, dim3((unsigned)nc), dim3(256), 0, stream, la);
+
       DwArgs dw{};
       dw.Ht = GOp{Hc, Hd, nc, Hd};
       dw.Et = GOp{E, V, nc, V};
+      dw.slot = slot;
+      dw.lsum = lsum;
       dw.dw = a.dweight;
       dw.acc32 = acc32;
       dw.nvalid = nvalid;

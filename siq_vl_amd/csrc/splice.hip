@@ -29,6 +29,7 @@
 //    gradient (below).
 #include <algorithm>
 
+#include "ids.h"
 #include "splice.h"
 
 namespace siq {
@@ -297,13 +298,12 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const bf16* __restrict
 //    the other waited for memory at each of them: 1065 us of the 1.24 ms that
 //    the splice's forward and backward took at 16384 tokens x 1536; with the
 //    hot list emb_sum takes 27 us and emb_hot 36 us.
-constexpr int kEmbChunk = 2048;  // two keys per thread of a 1024-thread workgroup
+constexpr int kEmbChunk = kIdChunk;
 constexpr int kRowsPerPartial = 10;
 
 // Blocks [0, nch) sort one chunk each (after clearing that chunk's run
 // table); the other blocks zero the table gradient meanwhile, so that the
 // sort, which keeps only nch CUs busy, hides under the HBM-bound clear.
-static_assert(kEmbChunk == 2 * 1024, "one compare-exchange pair per thread and stage");
 __global__ __launch_bounds__(1024) void emb_prep_kernel(const int64_t* __restrict__ ids, int64_t n, int64_t vocab,
                                                         int64_t skip0, int64_t skip1, uint64_t* __restrict__ keys,
                                                         int2* __restrict__ seg, int nch, u32x4* __restrict__ dw,
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(1024) void emb_prep_kernel(const int64_t* __restric
   int np2 = 64;
   while (np2 < len) np2 <<= 1;
   for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-    uint64_t k = ~0ull;
+    uint64_t k = kNoKey;
     if (i < len) {
       const int64_t v = ids[base + i];
       if (v >= 0 && v < vocab && v != skip0 && v != skip1) k = ((uint64_t)v << 32) | (uint32_t)i;
@@ -331,27 +331,13 @@ __global__ __launch_bounds__(1024) void emb_prep_kernel(const int64_t* __restric
     sk[i] = k;
   }
   __syncthreads();  // also orders the run table's clearing before its writes below
-  // bitonic network: in each stage thread t owns the pair (i, i + j), i = t with a zero bit inserted at j
-  const int t = threadIdx.x;
-  for (int k = 2; k <= np2; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const int i = 2 * t - (t & (j - 1));
-      if (i + j < np2) {
-        const uint64_t a = sk[i], b = sk[i + j];
-        if ((a > b) == ((i & k) == 0)) {
-          sk[i] = b;
-          sk[i + j] = a;
-        }
-      }
-      __syncthreads();
-    }
-  }
+  sort_keys(sk, np2);
   // every key slot of the chunk is written (all-ones past the tokens), so the sum kernel reads no stale key
   uint64_t* kout = keys + base;
   for (int i = threadIdx.x; i < kEmbChunk; i += blockDim.x) {
-    const uint64_t key = i < np2 ? sk[i] : ~0ull;
+    const uint64_t key = i < np2 ? sk[i] : kNoKey;
     kout[i] = key;
-    if (key == ~0ull) continue;
+    if (key == kNoKey) continue;
     const uint32_t v = (uint32_t)(key >> 32);
     if (i == 0 || (uint32_t)(sk[i - 1] >> 32) != v) sg[v].x = i;
     if (i == len - 1 || (uint32_t)(sk[i + 1] >> 32) != v) sg[v].y = i + 1;
@@ -409,7 +395,7 @@ __global__ __launch_bounds__(256) void emb_sum_kernel(const T* __restrict__ grad
   if (item >= (int64_t)nchunks * kEmbChunk) return;
   const int c = (int)(item / kEmbChunk), i = (int)(item % kEmbChunk);
   const uint64_t key = keys[item];
-  if (key == ~0ull) return;
+  if (key == kNoKey) return;
   const uint32_t v = (uint32_t)(key >> 32);
   if (i > 0 && (uint32_t)(keys[item - 1] >> 32) == v) return;  // not the first key of its id in this chunk
   // an earlier chunk holding the id means its wave writes the row

@@ -248,3 +248,41 @@ def test_full_size_vs_torch_fp32():
           flush=True)
     assert r_loss <= TOL and r_dh <= TOL and r_dw <= TOL
     assert bool((dh[~valid] == 0).all())
+
+
+@pytest.mark.parametrize("n,hdim,vocab,chunk", [(70, 64, 1032, 4096), (4500, 128, 1032, 4096), (700, 192, 520, 300)])
+def test_row_references_and_label_terms(n, hdim, vocab, chunk):
+    """Rows whose label logit is near the maximum, 2^60 below it in every tile
+    or in some (their tiles are redone relative to their own maximum), labels
+    that come once, often, in several sorted runs of 2048 rows, and rows whose
+    label holds all the mass.  Per element: dH one rounding of each softmax
+    numerator (a second one in redone rows) and of the result, dW one of f H
+    besides; the label terms are exact."""
+    print(f"flce references n={n} hdim={hdim} V={vocab} chunk={chunk}", flush=True)
+    h, w, y = make(n, hdim, vocab, seed=n, ignore_frac=0.2, wscale=1.0)
+    g = torch.Generator().manual_seed(n + 1)
+    valid = torch.nonzero((y >= 0)).flatten()
+    y[valid[torch.rand(valid.numel(), generator=g) < 0.4]] = 7  # a frequent label
+    scale = torch.tensor([0.01, 0.2, 3.0, 12.0])[torch.randint(0, 4, (n,), generator=g)]
+    h = (h.float() * scale[:, None]).to(torch.bfloat16)
+    for r in valid[::5].tolist():  # the label far above the rest
+        h[r] = w[y[r]] * 2.0
+    for r in valid[1::7].tolist():  # one vocab tile far above the label's, the others not
+        h[r] = (0.02 * h[r].float() + 3.0 * w[300 + r % 100].float()).to(torch.bfloat16)
+    loss, count, bad, dh, dw = run(h, w, y, chunk)
+    ref = oc.linear_ce(h, w, y)
+    assert count == ref["count"] and bad == 0
+    assert abs(loss - ref["loss"]) <= 1e-5 * abs(ref["loss"])
+    hf, wf = h.double().numpy()[valid], w.double().numpy()
+    z = hf @ wf.T
+    p = np.exp(z - z.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True) * count
+    # fp32 logits: p's relative error is the logit's absolute one
+    slack = 2.0**-8 + hdim * 2.0**-22 * float((np.abs(hf) @ np.abs(wf).T).max())
+    mag_h, mag_w = p @ np.abs(wf), p.T @ np.abs(hf)
+    assert np.all(np.abs(dh[valid] - ref["dh"][valid]) <= 2**-8 * np.abs(ref["dh"][valid]) + slack * mag_h + 1e-30)
+    steps = -(-count // chunk)
+    assert np.all(np.abs(dw - ref["dw"]) <= (2**-8 if steps == 1 else 2**-7) * np.abs(ref["dw"]) + 2 * slack * mag_w
+                  + (0 if steps == 1 else 2**-8 * 2 * np.abs(mag_w).max()) + 1e-30)
+    alone, c2, _ = C.flce_loss(h.to(DEV), w.to(DEV), y.to(DEV))
+    assert float(alone) == loss and int(c2) == count
