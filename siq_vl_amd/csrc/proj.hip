@@ -21,7 +21,7 @@
 //   dX       dXs^T [k][m] = W^T . dY^T (A = W read k-major, B = dY rows)
 //   dW       dW^T [k][n]  = Xs^T . dY  (A = gathered Xs read k-major, B = dY read k-major)
 // The forward and dW have few tiles at projector sizes (96 at m = 4096,
-// n = 1536, k = 4096), so their reduction is split over up to 8 workgroups
+// n = 1536, k = 4096), so their reduction is split over up to 48 workgroups
 // per tile with fp32 partial sums added afterwards in split order
 // (deterministic).
 #include "gemm.h"
@@ -267,13 +267,28 @@ __global__ __launch_bounds__(NT) void proj_dw_kernel(const DwArgs p) {
   }
 }
 
-// out[e] = bf16(sum over s of part[s][e]), s in order; nvec groups of 8.
+// out[e] = bf16(sum over s of part[s][e]), s in order, four splits' loads in
+// flight; nvec groups of 8.
 __global__ __launch_bounds__(256) void proj_sum_kernel(const float* __restrict__ part, bf16* __restrict__ out,
                                                        int64_t nvec, int64_t stride, int splits) {
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nvec; i += (int64_t)gridDim.x * 256) {
     f32x4 a = *reinterpret_cast<const f32x4*>(part + 8 * i);
     f32x4 b = *reinterpret_cast<const f32x4*>(part + 8 * i + 4);
-    for (int s = 1; s < splits; ++s) {
+    int s = 1;
+    for (; s + 4 <= splits; s += 4) {
+      f32x4 x[4], y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        x[u] = *reinterpret_cast<const f32x4*>(part + (s + u) * stride + 8 * i);
+        y[u] = *reinterpret_cast<const f32x4*>(part + (s + u) * stride + 8 * i + 4);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a += x[u];
+        b += y[u];
+      }
+    }
+    for (; s < splits; ++s) {
       a += *reinterpret_cast<const f32x4*>(part + s * stride + 8 * i);
       b += *reinterpret_cast<const f32x4*>(part + s * stride + 8 * i + 4);
     }
@@ -320,12 +335,16 @@ Shuffle shuffle_of(const ProjArgs& a) {
 }
 
 // Split-K factor: enough workgroups to cover the CUs once, each keeping at
-// least 8 k-steps, at most 8 splits.
+// least 4 k-steps, at most 48 splits.  A call of few tiles is bound by the
+// length of a workgroup's k loop (one 27 x 27 image, 4 tiles of 162 k-steps:
+// forward 32 us at 8 splits, 25 at 40); a call of many tiles has few splits either way.  kMaxSplits bounds
+// the partial sums (48 m n fp32 for at most 5 tiles).
+constexpr int kMaxSplits = 48;
 int splits_for(int64_t tiles, int64_t kdim, int cus) {
   int64_t s = tiles > 0 ? cus / tiles : 1;
   const int64_t ksteps = (kdim + BK - 1) / BK;
-  if (s > ksteps / 8) s = ksteps / 8;
-  if (s > 8) s = 8;
+  if (s > ksteps / 4) s = ksteps / 4;
+  if (s > kMaxSplits) s = kMaxSplits;
   return s < 1 ? 1 : (int)s;
 }
 

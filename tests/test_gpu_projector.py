@@ -84,6 +84,22 @@ def test_gemm_core_at_few_k_steps(steps, tail):
         assert bool(((got - exact).abs() <= 2**-8 * exact.abs() + a.shape[1] * 2**-23 * mag).all())
 
 
+@pytest.mark.parametrize("side,dv,n", [(6, 1152, 40), (6, 448, 264), (30, 64, 8)])
+def test_many_splits_of_few_tiles(side, dv, n):
+    """Few tiles, long k: the forward's reduction over up to 48 workgroups
+    (40, 15 and 2 here), dweight's over tokens likewise.  One bf16 rounding of
+    fp32 sums, as in test_gemm_core_at_few_k_steps."""
+    print(f"projector splits side={side} dv={dv} n={n}", flush=True)
+    x, w, dy = make(1, side, dv, 3, n, seed=n)
+    y = P.proj_fwd(x.to(DEV), w.to(DEV), 3).double().cpu()[0]
+    _, dw = P.proj_bwd(x.to(DEV), w.to(DEV), dy.to(DEV), 3, need_dx=False)
+    t = side // 3
+    xs = x.double().view(t, 3, t, 3, dv).permute(0, 2, 1, 3, 4).reshape(t * t, 9 * dv)
+    for got, a, b in ((y, xs, w.double().T), (dw.double().cpu(), dy.double()[0].T, xs)):
+        exact, mag = a @ b, a.abs() @ b.abs()
+        assert bool(((got - exact).abs() <= 2**-8 * exact.abs() + a.shape[1] * 2**-23 * mag).all())
+
+
 def test_repeat_is_bitwise():
     x, w, dy = (t.to(DEV) for t in make(16, 16, 256, 2, 512, seed=1))
     a = (P.proj_fwd(x, w, 2), *P.proj_bwd(x, w, dy, 2))
