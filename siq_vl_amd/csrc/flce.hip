@@ -55,6 +55,8 @@
 // Loss only (no gradient wanted, e.g. evaluation under torch.no_grad): the
 // logits epilogue keeps its tile sums and z_y but stores no E, the row pass
 // stops at the loss, and neither gradient GEMM runs.
+#include <algorithm>
+
 #include "flce.h"
 #include "gemm.h"
 #include "ids.h"
@@ -483,51 +485,89 @@ __global__ __launch_bounds__(256) void flce_label_kernel(const LabelArgs p) {
 struct DhArgs {
   GOp Wt;        // W [V, hdim] read as A[i = h][k = v]
   GOp E;         // [nc, V] read as B[j = tok][k = v]
-  bf16* dh;      // dhidden [n, hdim] (used when splits == 1)
-  float* part;   // [splits, nc, hdim]
-  const float* f;         // [nc] row factors, label weights, labels (used when splits == 1)
+  bf16* dh;      // dhidden [n, hdim]
+  float* part;   // [slots][prow][hdim] partial sums (dh_layout; none when splits == 1)
+  const float* f;         // [nc] row factors, label weights, labels
   const float* wt;
   const int64_t* y;
   const int32_t* rows;    // compacted row -> original row (whole batch)
   const int64_t* nvalid;
-  int64_t hdim, nc, kper, c0;
-  int nI, nJ, splits;
+  int64_t hdim, nc, c0;
+  int nI, splits, prow;  // hdim tiles; vocab ranges; rows of a slot
 };
 
-// dH work: a unit is one (token tile, vocab split); its nI hdim tiles share
+// dH work: a unit is one (token tile, vocab range); its nI hdim tiles share
 // the unit's E slab, so they run as consecutive blocks on one XCD (block b
-// runs on XCD b % 8).  Units are dealt out over the XCDs in turn, splits of a
-// token tile on different XCDs: every XCD gets the same number of units, also
-// when the token tiles past the valid rows (which return at once) are many --
-// a whole token tile per XCD left some XCDs half as loaded as others.  The
-// grid is 8 nI ceil(nJ splits / 8) blocks.
-__device__ __forceinline__ bool dh_tile_of(int nI, int nJ, int splits, int& ti, int& tj, int& split) {
-  const int x = (int)(blockIdx.x % kXcds), k = (int)(blockIdx.x / kXcds);
-  ti = k % nI;
-  const int unit = x + kXcds * (k / nI);
-  tj = unit / splits;
-  split = unit - tj * splits;
-  return tj < nJ;
+// runs on XCD b % 8).  Units are dealt out over the XCDs in turn, ranges of a
+// token tile on different XCDs.  With 8 ranges an XCD has one range of every
+// token tile, and a last round of a few of its workgroups (32 run at a time)
+// would leave the others idle: 27 token tiles x 6 hdim tiles are 5 rounds and
+// 2 workgroups.  So the token tiles past the last whole round have their ranges
+// cut into kDhSub parts.  The cut is made on the device, from the valid rows;
+// partial sums lie in slots, splits of them for a token tile with whole ranges,
+// then kDhSub times 8 for each of the others.  With fewer ranges (more than 292
+// tiles: eight rounds or more) nothing is cut.  Measured, whole calls on one
+// card: loss, dH and dW of 16384 rows, 11455 valid, x 1536 13.31 -> 13.05 ms;
+// loss and dH of 4099 rows, 2870 valid, x 896 1.57 -> 1.50 ms.
+constexpr int kDhSub = 4, kXcdSlots = 32;
+// Splits of the dH vocab reduction: enough WGs to fill the chip several
+// rounds over, bounded by the size of the fp32 partial sums.
+int dh_splits(int64_t hdim, int64_t chunk) {
+  const int64_t tiles = ((hdim + BI - 1) / BI) * ((chunk + BJ - 1) / BJ);
+  int64_t s = (2048 + tiles - 1) / tiles;
+  if (s < 1) s = 1;
+  if (s > kXcds) s = kXcds;
+  return (int)s;
+}
+struct DhLayout {
+  int nj, nfull;  // token tiles with a valid row, those with whole ranges
+};
+__device__ __forceinline__ DhLayout dh_layout(int64_t nv, int nI, int splits) {
+  DhLayout L;
+  L.nj = nv > 0 ? (int)((nv + BJ - 1) / BJ) : 0;
+  const int rem = (int)(((int64_t)L.nj * nI) % kXcdSlots);
+  L.nfull = splits == kXcds ? L.nj - min(L.nj, (rem + nI - 1) / nI) : L.nj;
+  return L;
+}
+// Slots, also units, for any number of valid rows in nj token tiles.
+int64_t dh_slots(int nj, int nI, int splits) {
+  if (splits < kXcds) return (int64_t)nj * splits;
+  return (int64_t)kXcds * (nj + (int64_t)(kDhSub - 1) * std::min(nj, (kXcdSlots - 1 + nI - 1) / nI));
 }
 
 __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
   __shared__ __align__(16) bf16 smem[SMEM];
-  int ti, tj, split;
-  if (!dh_tile_of(p.nI, p.nJ, p.splits, ti, tj, split)) return;
+  const int64_t nv = min(p.nc, *p.nvalid - p.c0);
+  const DhLayout L = dh_layout(nv, p.nI, p.splits);
+  const int x = (int)(blockIdx.x % kXcds), k = (int)(blockIdx.x / kXcds);
+  const int ti = k % p.nI, unit = x + kXcds * (k / p.nI), slot = unit;
+  // k-steps of the unit's range, or part of one
+  const int64_t S = (p.E.cols + BK - 1) / BK, per = (S + p.splits - 1) / p.splits;
+  int tj;
+  int64_t sb, se;
+  if (unit < L.nfull * p.splits) {
+    tj = unit / p.splits;
+    sb = (unit - tj * p.splits) * per;
+    se = min(S, sb + per);
+  } else {
+    const int q = k / p.nI - L.nfull;
+    tj = L.nfull + q / kDhSub;
+    if (p.splits < kXcds || tj >= L.nj) return;
+    const int64_t sub = (per + kDhSub - 1) / kDhSub, s0 = x * per;
+    sb = s0 + (q % kDhSub) * sub;
+    se = min(min(S, s0 + per), sb + sub);
+  }
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
-  const int64_t nv = *p.nvalid - p.c0;
-  if (j0 >= nv) return;
-  const int64_t kb = split * p.kper;
-  const int64_t ke = min(p.E.cols, kb + p.kper);
   f32x16 acc[4][2];
-  gemm_core<false, true, true>(smem, p.Wt, p.E, i0, j0, kb, ke, acc);
+  // (an empty range, of a vocabulary of few steps, leaves zeros)
+  gemm_core<false, true, true>(smem, p.Wt, p.E, i0, j0, sb * BK, min(p.E.cols, se * BK), acc);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int wi = w & 1, wj = w >> 1;
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
-    const int64_t tok = j0 + wave_col(b, wj) + l32;
-    if (tok >= p.nc) continue;
-    if (p.splits == 1 && tok >= nv) continue;  // padding row
+    const int r = wave_col(b, wj) + l32;
+    const int64_t tok = j0 + r;
+    if (tok >= nv) continue;
     const int64_t orow = p.splits == 1 ? p.rows[p.c0 + tok] : 0;
     const float f = p.splits == 1 ? p.f[tok] : 0.f, wt = p.splits == 1 ? p.wt[tok] : 0.f;
     const bf16* wy = p.Wt.base + (p.splits == 1 ? p.y[tok] : 0) * p.hdim;
@@ -544,7 +584,7 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
           for (int i = 0; i < 8; ++i) o[i] = (bf16)__builtin_fmaf(f, acc[a][b][8 * jj + i], wt * (float)l[i]);
           st_bf16x8(p.dh + orow * p.hdim + hh, o);
         } else {
-          float* dst = p.part + ((int64_t)split * p.nc + tok) * p.hdim + hh;
+          float* dst = p.part + ((int64_t)slot * p.prow + r) * p.hdim + hh;
           f32x4 lo, hi;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -558,21 +598,36 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
   }
 }
 
-// dH rows of the chunk: f times the splits' fp32 partial sums, added in split
-// order, plus the label term w W[y]; each compacted row written to its
-// original row.
+// dH rows of the chunk: f times the fp32 partial sums of the row's token tile,
+// added in slot order, plus the label term w W[y]; each compacted row written
+// to its original row.
 __global__ __launch_bounds__(256) void flce_dh_sum_kernel(const DhArgs p) {
-  // part is [splits][nc * hdim]; groups of 8 elements, hdim / 8 per row
+  constexpr int U = 4;  // partial sums in flight
   const int64_t nv = min(p.nc, *p.nvalid - p.c0);
-  const int64_t gpr = p.hdim / 8, stride = p.nc * p.hdim;
+  const DhLayout L = dh_layout(nv, p.nI, p.splits);
+  const int64_t gpr = p.hdim / 8, stride = p.prow * p.hdim;  // groups of 8 elements, hdim / 8 per row
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nv * gpr; i += (int64_t)gridDim.x * 256) {
     const int64_t r = i / gpr, col = 8 * (i - r * gpr);
+    const int tj = (int)(r / BJ), tail = tj - L.nfull;
+    const int nslots = tail < 0 ? p.splits : kDhSub * kXcds;
+    const float* src = p.part + (r - (int64_t)tj * BJ) * p.hdim + col +
+                       stride * (tail < 0 ? tj * p.splits : kXcds * (L.nfull + kDhSub * tail));
     const bf16x8 l = ld_bf16x8(p.Wt.base + p.y[r] * p.hdim + col);
-    f32x4 a = *reinterpret_cast<const f32x4*>(p.part + 8 * i);
-    f32x4 b = *reinterpret_cast<const f32x4*>(p.part + 8 * i + 4);
-    for (int s = 1; s < p.splits; ++s) {
-      a += *reinterpret_cast<const f32x4*>(p.part + s * stride + 8 * i);
-      b += *reinterpret_cast<const f32x4*>(p.part + s * stride + 8 * i + 4);
+    f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    for (int s = 0; s < nslots; s += U, src += U * stride) {
+      f32x4 lo[U], hi[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s + u < nslots) {
+          lo[u] = *reinterpret_cast<const f32x4*>(src + u * stride);
+          hi[u] = *reinterpret_cast<const f32x4*>(src + u * stride + 4);
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s + u < nslots) {
+          a += lo[u];
+          b += hi[u];
+        }
     }
     const float f = p.f[r], wt = p.wt[r];
     bf16x8 o;
@@ -846,19 +901,12 @@ __global__ __launch_bounds__(256) void zero_bf16_kernel(bf16* __restrict__ x, in
 // ---------------------------------------------------------------- workspace
 struct Layout {
   size_t invden, loss_row, mpart, spart, zy, f, wt, E, part, acc32, rows, hc, yc, ref, keys, slot, lsum, total;
-  int64_t chunk, nvt, splits;
+  int64_t chunk, nvt;
+  int splits, prow;  // of dH: vocab ranges, rows of a slot
   int nsort;  // sorted runs of a chunk's labels (dW only)
 };
 
 size_t al(size_t x) { return (x + 255) & ~size_t(255); }
-
-int dh_splits(int64_t hdim, int64_t chunk) {
-  const int64_t tiles = ((hdim + BI - 1) / BI) * ((chunk + BJ - 1) / BJ);
-  int64_t s = (2048 + tiles - 1) / tiles;
-  if (s < 1) s = 1;
-  if (s > 8) s = 8;
-  return (int)s;
-}
 
 // need_dh false: loss only (no E, no gradient buffers); its chunks only bound
 // the per-(row, vocab tile) sum buffers, so they are large.
@@ -872,7 +920,6 @@ Layout layout(int64_t n, int64_t hdim, int64_t V, int64_t chunk, bool need_dh, b
   }
   L.chunk = chunk < n ? chunk : (n > 0 ? n : 1);
   L.nvt = (V + kVT - 1) / kVT;
-  L.splits = dh_splits(hdim, L.chunk);
   const int64_t nchunks = n > 0 ? (n + L.chunk - 1) / L.chunk : 0;
   size_t off = 0;
   L.invden = off;
@@ -892,7 +939,11 @@ Layout layout(int64_t n, int64_t hdim, int64_t V, int64_t chunk, bool need_dh, b
   L.E = off;
   if (need_dh) off += al(sizeof(bf16) * (size_t)(L.chunk * V));
   L.part = off;
-  if (need_dh && L.splits > 1) off += al(sizeof(float) * (size_t)(L.splits * L.chunk * hdim));
+  L.splits = dh_splits(hdim, L.chunk);
+  L.prow = (int)std::min<int64_t>(L.chunk, BJ);
+  if (need_dh && L.splits > 1)
+    off += al(sizeof(float) * (size_t)(dh_slots((int)((L.chunk + BJ - 1) / BJ), (int)((hdim + BI - 1) / BI), L.splits) *
+                                       L.prow * hdim));
   L.acc32 = off;
   // the fp32 dW sum: only when the valid rows may span more than two chunks
   // (over two, the first chunk's sum is kept in dW itself)
@@ -1032,17 +1083,13 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
     dh.c0 = c0;
     dh.hdim = Hd;
     dh.nc = nc;
-    dh.splits = (int)L.splits;
-    {
-      const int64_t kblocks = (V + BK - 1) / BK;
-      dh.kper = ((kblocks + L.splits - 1) / L.splits) * BK;
-    }
     dh.nI = (int)((Hd + BI - 1) / BI);
-    dh.nJ = (int)((nc + BJ - 1) / BJ);
+    dh.splits = L.splits;
+    dh.prow = L.prow;
     {
-      const int units = dh.nJ * (int)L.splits;
-      const int grid = kXcds * dh.nI * ((units + kXcds - 1) / kXcds);
-      hipLaunchKernelGGL(flce_dh_kernel, dim3(grid), dim3(NT), 0, stream, dh);
+      const int64_t units = dh_slots((int)((nc + BJ - 1) / BJ), dh.nI, L.splits);
+      const int64_t grid = kXcds * dh.nI * ((units + kXcds - 1) / kXcds);
+      hipLaunchKernelGGL(flce_dh_kernel, dim3((unsigned)grid), dim3(NT), 0, stream, dh);
     }
     if (L.splits > 1) {
       const int64_t nvec = nc * Hd / 8;

@@ -337,8 +337,9 @@ Shuffle shuffle_of(const ProjArgs& a) {
 // Split-K factor: enough workgroups to cover the CUs once, each keeping at
 // least 4 k-steps, at most 48 splits.  A call of few tiles is bound by the
 // length of a workgroup's k loop (one 27 x 27 image, 4 tiles of 162 k-steps:
-// forward 32 us at 8 splits, 25 at 40); a call of many tiles has few splits either way.  kMaxSplits bounds
-// the partial sums (48 m n fp32 for at most 5 tiles).
+// forward 32 us at 8 splits, 25 at 40); a call of many tiles has few splits
+// either way.  kMaxSplits bounds the partial sums (48 m n fp32 for at most 5
+// tiles).
 constexpr int kMaxSplits = 48;
 int splits_for(int64_t tiles, int64_t kdim, int cus) {
   int64_t s = tiles > 0 ? cus / tiles : 1;

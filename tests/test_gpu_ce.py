@@ -286,3 +286,33 @@ def test_row_references_and_label_terms(n, hdim, vocab, chunk):
                   + (0 if steps == 1 else 2**-8 * 2 * np.abs(mag_w).max()) + 1e-30)
     alone, c2, _ = C.flce_loss(h.to(DEV), w.to(DEV), y.to(DEV))
     assert float(alone) == loss and int(c2) == count
+
+
+@pytest.mark.parametrize("n,hdim,vocab", [(300, 64, 8), (2100, 1024, 712), (1800, 1280, 5000), (20000, 1024, 520),
+                                          (32600, 4096, 264)])
+def test_dh_ranges_and_parts(n, hdim, vocab):
+    """dH's vocab ranges: fewer k-steps than ranges and parts, token tiles with
+    whole ranges and with cut ones in one call, a valid-row count well below
+    the chunk, 7 ranges, and 1.  Per element: one rounding of each softmax
+    numerator, one of the result, and the fp32 logit's error."""
+    print(f"flce dH ranges n={n} hdim={hdim} V={vocab}", flush=True)
+    h, w, y = make(n, hdim, vocab, seed=n, ignore_frac=0.6 if n == 1800 else 0.05, wscale=2.0 / hdim**0.5)
+    hd, wd, yd = h.to(DEV), w.to(DEV), y.to(DEV)
+    loss, count, bad, dh, _ = C.flce_fwd_bwd(hd, wd, yd, -100, None, False, n)
+    wf, total = wd.double(), 0.0
+    valid = yd >= 0
+    assert int(count) == int(valid.sum()) and int(bad) == 0
+    assert bool((dh[~valid] == 0).all())
+    for r0 in range(0, n, 4096):
+        hb, yb, vb = hd[r0:r0 + 4096].double(), yd[r0:r0 + 4096], valid[r0:r0 + 4096]
+        z = hb @ wf.t()
+        rows = torch.arange(hb.shape[0], device=DEV)
+        zy = z[rows, yb.clamp(min=0)]
+        total += float((torch.logsumexp(z, 1) - zy)[vb].sum())
+        p = torch.softmax(z, 1) / int(count)
+        slack = 2.0**-8 + hdim * 2.0**-22 * float((hb.abs() @ wf.abs().t()).max())
+        mag = p @ wf.abs()
+        ref = p @ wf - wf[yb.clamp(min=0)] / int(count)
+        err = (dh[r0:r0 + 4096].double() - ref).abs()
+        assert bool((err <= 2.0**-8 * ref.abs() + slack * mag + 1e-30)[vb].all())
+    assert abs(float(loss) - total / int(count)) <= 1e-5 * abs(total / int(count))
