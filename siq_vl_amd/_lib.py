@@ -11,6 +11,8 @@ import os
 import threading
 from pathlib import Path
 
+import torch
+
 from . import build as _build
 
 _LOCK = threading.Lock()
@@ -168,3 +170,14 @@ def check(rc: int, what: str) -> None:
 def int64_array(values) -> ctypes.Array:
     arr = (_i64 * len(values))(*[int(v) for v in values])
     return arr
+
+
+def strides(*values: int) -> ctypes.Array:
+    """``int64_array`` of what ``Tensor.stride()`` returned (ints already)."""
+    return (_i64 * len(values))(*values)
+
+
+def stream(device) -> int:
+    """The current stream's handle on a GPU device with an index, without the
+    ``torch.cuda.Stream`` object around it."""
+    return torch._C._cuda_getCurrentRawStream(device.index)

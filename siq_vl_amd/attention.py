@@ -38,7 +38,21 @@ SUPPORTED_HEAD_DIMS = (64, 128)
 
 
 # --------------------------------------------------------------------------- validation
+# The host's share of a call is what bounds the small ones (a prompt of 197
+# tokens: 8 us of kernel; the forward and backward of 5003: six kernels), so the
+# checks ask for a tensor's shape and strides once; what fails them goes on to
+# the function that names the fault.  Whole calls, before and
+# after: 22.1 -> 16.3 us and 245 -> 189 us.
 def _check_token_major(name: str, t: torch.Tensor, heads: int | None = None, dim: int | None = None) -> None:
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.bfloat16:
+        shape, stride = t.shape, t.stride()
+        if (len(shape) == 3 and stride[2] == 1 and not (stride[0] | stride[1]) & 7 and not t.data_ptr() & 15
+                and (heads is None or shape[1] == heads) and (dim is None or shape[2] == dim)):
+            return
+    _name_token_major_fault(name, t, heads, dim)
+
+
+def _name_token_major_fault(name: str, t: torch.Tensor, heads: int | None, dim: int | None) -> None:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.dim() != 3:
@@ -59,7 +73,8 @@ def _check_token_major(name: str, t: torch.Tensor, heads: int | None = None, dim
 
 def _ensure_token_major(t: torch.Tensor) -> torch.Tensor:
     """Returns ``t`` if the kernels can read it in place, else a contiguous copy."""
-    if t.stride(2) == 1 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0:
+    stride = t.stride()
+    if stride[2] == 1 and not (stride[0] | stride[1]) & 7 and not t.data_ptr() & 15:
         return t
     return t.contiguous()
 
@@ -88,6 +103,8 @@ def validate_cu_seqlens(cu: torch.Tensor, total: int, name: str = "cu_seqlens") 
 
 def _norm_device(device) -> torch.device:
     """``cuda`` -> ``cuda:<current index>`` (so that equal devices compare equal)."""
+    if isinstance(device, torch.device) and device.index is not None:
+        return device
     device = torch.device(device)
     if device.type == "cuda" and device.index is None:
         return torch.device("cuda", torch.cuda.current_device())
@@ -105,22 +122,22 @@ def _device_cu(cu: torch.Tensor, device: torch.device, total: int, name: str) ->
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch.cuda.current_stream(device).cuda_stream if device.index is None else _lib.stream(device)
 
 
 def _check_common(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> tuple[int, int, int]:
     _check_token_major("q", q)
-    hq, d = q.shape[1], q.shape[2]
+    _, hq, d = q.shape
     _check_token_major("k", k, dim=d)
-    hkv = k.shape[1]
+    total_k, hkv, _ = k.shape
     _check_token_major("v", v, heads=hkv, dim=d)
-    if v.shape[0] != k.shape[0]:
+    if v.shape[0] != total_k:
         raise ValueError(f"k and v token counts differ ({k.shape[0]} vs {v.shape[0]})")
     if d not in SUPPORTED_HEAD_DIMS:
         raise ValueError(f"head_dim {d} unsupported (supported: {SUPPORTED_HEAD_DIMS})")
     if hq % hkv:
         raise ValueError(f"num q heads ({hq}) must be a multiple of num kv heads ({hkv})")
-    if not (q.device == k.device == v.device):
+    if not (q.get_device() == k.get_device() == v.get_device()):
         raise ValueError("q, k, v must be on the same device")
     return hq, hkv, d
 
@@ -148,13 +165,15 @@ class AttnPlan:
         self.src = src
 
     def matches(self, batch: int, total_q: int, total_k: int, hq: int, hkv: int, causal: bool) -> bool:
-        return (self.batch, self.total_q, self.total_k, self.hq // self.hkv, self.hkv, self.causal) == (
-            batch, total_q, total_k, hq // hkv, hkv, bool(causal))
+        return (self.total_q == total_q and self.total_k == total_k and self.batch == batch and self.hkv == hkv
+                and self.hq // self.hkv == hq // hkv and self.causal == bool(causal))
 
     def describes(self, cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor) -> bool:
         """True when the plan was built from these offsets: the plan's own
         copies, the unchanged tensors it was built from, or tensors holding
         the same values (compared on the device: one device-to-host read)."""
+        if cu_seqlens_q is self.cu_q and cu_seqlens_k is self.cu_k:
+            return True
         for given, own, i in ((cu_seqlens_q, self.cu_q, 0), (cu_seqlens_k, self.cu_k, 1)):
             if given is own:
                 continue
@@ -218,7 +237,7 @@ def cached_attn_plan(cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor, tot
     ``_version``) or other totals / heads / causality build a new one."""
     device = _norm_device(device)
     key = (cu_seqlens_q._version, cu_seqlens_k._version, int(total_q), int(total_k), int(hq) // int(hkv), int(hkv),
-           bool(causal), str(device))
+           bool(causal), device)
     cache = getattr(cu_seqlens_q, _PLAN_ATTR, None)
     if cache is not None:
         hit = cache.get(key)
@@ -259,8 +278,7 @@ def varlen_attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlen
     out = torch.empty((total_q, hq, d), dtype=q.dtype, device=q.device)
     lse = torch.empty((hq, total_q), dtype=torch.float32, device=q.device)
     L = _lib.lib()
-    strides = _lib.int64_array([q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                                out.stride(0), out.stride(1)])
+    strides = _lib.strides(*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2])
     rc = L.siq_attn_varlen_fwd_plan(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                     pl.batch, total_q, total_k, hq, hkv, d, strides, float(softmax_scale),
                                     int(bool(causal)), pl.buf.data_ptr(), pl.buf.numel(), _stream(q.device))
@@ -306,9 +324,8 @@ def varlen_attn_bwd(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: tor
     L = _lib.lib()
     ws_bytes = L.siq_attn_bwd_plan_workspace_bytes(pl.batch, total_q, total_k, hq, hkv, d, int(det))
     ws = torch.empty((max(ws_bytes, 16),), dtype=torch.uint8, device=q.device)
-    strides = _lib.int64_array([q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                                out.stride(0), out.stride(1), dout.stride(0), dout.stride(1), dq.stride(0),
-                                dq.stride(1), dk.stride(0), dk.stride(1), dv.stride(0), dv.stride(1)])
+    strides = _lib.strides(*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2], *dout.stride()[:2],
+                           *dq.stride()[:2], *dk.stride()[:2], *dv.stride()[:2])
     rc = L.siq_attn_varlen_bwd_plan(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                     dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), pl.batch, total_q,
                                     total_k, hq, hkv, d, strides, float(softmax_scale), int(bool(causal)), int(det),
@@ -341,6 +358,11 @@ class _VarlenAttnFn(torch.autograd.Function):
 
 
 def _check_rope_rows(cos: torch.Tensor, sin: torch.Tensor, total_q: int, d: int) -> None:
+    want, s0, s1 = (total_q, d), cos.stride(), sin.stride()
+    if (cos.shape == want and sin.shape == want and cos.dtype == sin.dtype == torch.bfloat16 and cos.is_cuda
+            and sin.is_cuda and s0[1] == s1[1] == 1 and not (s0[0] | s1[0]) & 7
+            and not (cos.data_ptr() | sin.data_ptr()) & 15):
+        return
     for name, t in (("cos", cos), ("sin", sin)):
         if t.dim() != 2 or t.shape[0] != total_q or t.shape[1] != d:
             raise ValueError(f"{name} must be [total_q, head_dim] = [{total_q}, {d}], got {tuple(t.shape)}")
@@ -366,9 +388,8 @@ def varlen_attn_rope_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos:
     out = torch.empty((total_q, hq, d), dtype=q.dtype, device=q.device)
     lse = torch.empty((hq, total_q), dtype=torch.float32, device=q.device)
     qe = torch.empty((total_q, hq, d), dtype=q.dtype, device=q.device)
-    strides = _lib.int64_array([q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                                out.stride(0), out.stride(1), qe.stride(0), qe.stride(1), cos.stride(0),
-                                sin.stride(0)])
+    strides = _lib.strides(*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2], *qe.stride()[:2],
+                           cos.stride(0), sin.stride(0))
     rc = _lib.lib().siq_attn_rope_fwd_plan(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                            qe.data_ptr(), cos.data_ptr(), sin.data_ptr(), pl.batch, total_q, total_k,
                                            hq, hkv, d, strides, float(softmax_scale), int(bool(causal)),
@@ -402,10 +423,8 @@ def varlen_attn_rope_bwd(dout: torch.Tensor, q_embed: torch.Tensor, k: torch.Ten
     ws_bytes = L.siq_attn_bwd_plan_workspace_bytes(pl.batch, total_q, total_k, hq, hkv, d, 1)
     ws = torch.empty((max(ws_bytes, 16),), dtype=torch.uint8, device=q_embed.device)
     q = q_embed
-    strides = _lib.int64_array([q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                                out.stride(0), out.stride(1), dout.stride(0), dout.stride(1), dq.stride(0),
-                                dq.stride(1), dk.stride(0), dk.stride(1), dv.stride(0), dv.stride(1), cos.stride(0),
-                                sin.stride(0)])
+    strides = _lib.strides(*q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2], *dout.stride()[:2],
+                           *dq.stride()[:2], *dk.stride()[:2], *dv.stride()[:2], cos.stride(0), sin.stride(0))
     rc = L.siq_attn_rope_bwd_plan(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                   dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), cos.data_ptr(),
                                   sin.data_ptr(), pl.batch, total_q, total_k, hq, hkv, d, strides,
@@ -433,8 +452,7 @@ class _VarlenRopeAttnFn(torch.autograd.Function):
         from . import rope as _rope
 
         cos, sin = cos.contiguous(), sin.contiguous()
-        qe, ke = _rope.rope_fwd(q[None], k[None], cos[None], sin[None])
-        qe, ke = qe[0], ke[0]
+        qe, ke = _rope.rope_rows_fwd(q, k, cos, sin)
         v = _ensure_token_major(v)
         hq, hkv = qe.shape[1], ke.shape[1]
         plan = cached_attn_plan(cu_q, cu_k, qe.shape[0], ke.shape[0], hq, hkv, causal, qe.device)
@@ -471,8 +489,7 @@ class _VarlenRopeF32Attn(torch.autograd.Function):
         from . import rope as _rope
 
         cos, sin = cos.contiguous(), sin.contiguous()
-        qe, ke = _rope.rope_fwd(q[None], k[None], cos[None], sin[None])
-        qe, ke = qe[0], ke[0]
+        qe, ke = _rope.rope_rows_fwd(q, k, cos, sin)
         v = _ensure_token_major(v)
         plan = cached_attn_plan(cu_q, cu_k, qe.shape[0], ke.shape[0], qe.shape[1], ke.shape[1], causal, qe.device)
         out, lse = varlen_attn_fwd(qe, ke, v, cu_q, cu_k, max_q, max_k, scale, causal, plan=plan)
@@ -490,8 +507,8 @@ class _VarlenRopeF32Attn(torch.autograd.Function):
         plan = ctx.plan
         dqe, dke, dv = varlen_attn_bwd(_ensure_token_major(dout), qe, ke, v, out, lse, plan.cu_q, plan.cu_k, max_q,
                                        max_k, scale, causal, plan=plan)
-        dq, dk = _rope.rope_bwd(dqe[None], dke[None], cos[None], sin[None])
-        return dq[0], dk[0], dv, None, None, None, None, None, None, None, None
+        dq, dk = _rope.rope_rows_bwd(dqe, dke, cos, sin)
+        return dq, dk, dv, None, None, None, None, None, None, None, None
 
 
 def flash_attn_varlen_rope_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor,

@@ -63,7 +63,7 @@ def _launch(fn_name: str, x0, x1, cos, sin, y0, y1) -> None:
     hkv = x1.shape[2]
     strides = [*x0.stride()[:3], *x1.stride()[:3], *cos.stride()[:2], *sin.stride()[:2], *y0.stride()[:3],
                *y1.stride()[:3]]
-    stream = torch.cuda.current_stream(x0.device).cuda_stream
+    stream = _lib.stream(x0.device)
     rc = getattr(_lib.lib(), fn_name + "_ex")(x0.data_ptr(), x1.data_ptr(), cos.data_ptr(), sin.data_ptr(),
                                               y0.data_ptr(), y1.data_ptr(), b, s, hq, hkv, d,
                                               _lib.int64_array(strides), _CS_DTYPE[cos.dtype], stream)
@@ -117,6 +117,51 @@ def rope_bwd(dq_embed: torch.Tensor, dk_embed: torch.Tensor, cos: torch.Tensor, 
     if g0.numel() and g1.numel():
         _launch("siq_rope_bwd", g0, g1, cos, sin, dq, dk)
     return dq, dk
+
+
+def _rows_usable(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
+    """Token-major ``[T, H, D]`` q and k with ``[T, D]`` rows that the kernels
+    read in place: everything ``_check`` and ``_usable`` ask of their views
+    with a batch dimension (which cost the small calls six more torch ops)."""
+    if not (q.is_cuda and k.is_cuda and cos.is_cuda and sin.is_cuda and q.dtype == k.dtype == torch.bfloat16
+            and cos.dtype == sin.dtype and cos.dtype in _CS_DTYPE):
+        return False
+    (n0, n1, n2, n3), (s0, s1, s2, s3) = zip(*((t.shape, t.stride()) for t in (q, k, cos, sin)))
+    return (len(n0) == 3 and len(n1) == 3 and len(n2) == 2 and n1[0] == n0[0] and n1[2] == n0[2] and n2 == n3
+            and n2 == (n0[0], n0[2]) and n0[0] > 0 and n0[1] > 0 and n1[1] > 0 and n0[2] > 0
+            and s0[2] == s1[2] == s2[1] == s3[1] == 1
+            and not (s0[0] | s0[1] | s1[0] | s1[1] | s2[0] | s3[0]) & 7
+            and not (q.data_ptr() | k.data_ptr() | cos.data_ptr() | sin.data_ptr()) & 15)
+
+
+def _rows_launch(fn_name: str, q: torch.Tensor | None, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor):
+    """One pass over rows that ``_rows_usable`` accepts (q None: k only)."""
+    t, hkv, d = k.shape
+    y0, y1 = None if q is None else torch.empty_like(q), torch.empty_like(k)
+    p0, hq, s0, o0 = (None, 0, (0, 0), (0, 0)) if q is None else (q.data_ptr(), q.shape[1], q.stride()[:2],
+                                                                  y0.stride()[:2])
+    strides = _lib.strides(0, *s0, 0, *k.stride()[:2], 0, cos.stride(0), 0, sin.stride(0), 0, *o0, 0, *y1.stride()[:2])
+    rc = getattr(_lib.lib(), fn_name + "_ex")(p0, k.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+                                              None if q is None else y0.data_ptr(), y1.data_ptr(), 1, t, hq, hkv, d,
+                                              strides, _CS_DTYPE[cos.dtype], _lib.stream(k.device))
+    _lib.check(rc, fn_name)
+    return y0, y1
+
+
+def rope_rows_fwd(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor):
+    """``rope_fwd`` on token-major ``[T, H, D]`` with ``cos`` / ``sin [T, D]``."""
+    if _rows_usable(q, k, cos, sin):
+        return _rows_launch("siq_rope_fwd", q, k, cos, sin)
+    qe, ke = rope_fwd(q[None], k[None], cos[None], sin[None])
+    return qe[0], ke[0]
+
+
+def rope_rows_bwd(dq_embed: torch.Tensor, dk_embed: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor):
+    """``rope_bwd`` on token-major ``[T, H, D]`` with ``cos`` / ``sin [T, D]``."""
+    if _rows_usable(dq_embed, dk_embed, cos, sin):
+        return _rows_launch("siq_rope_bwd", dq_embed, dk_embed, cos, sin)
+    dq, dk = rope_bwd(dq_embed[None], dk_embed[None], cos[None], sin[None])
+    return dq[0], dk[0]
 
 
 class _Rope(torch.autograd.Function):
@@ -174,7 +219,7 @@ def _launch_k(fn_name: str, x1, cos, sin, y1) -> None:
     """k-only pass (hq = 0): q and its output are not touched."""
     b, s, hkv, d = x1.shape
     strides = [0, 0, 0, *x1.stride()[:3], *cos.stride()[:2], *sin.stride()[:2], 0, 0, 0, *y1.stride()[:3]]
-    stream = torch.cuda.current_stream(x1.device).cuda_stream
+    stream = _lib.stream(x1.device)
     rc = getattr(_lib.lib(), fn_name + "_ex")(None, x1.data_ptr(), cos.data_ptr(), sin.data_ptr(), None,
                                               y1.data_ptr(), b, s, 0, hkv, d, _lib.int64_array(strides),
                                               _CS_DTYPE[cos.dtype], stream)
@@ -206,6 +251,8 @@ class _RopeK(torch.autograd.Function):
 def rotate_k_backward(dk_embed: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
     """The rotation's backward for k alone on token-major ``[T, Hkv, D]`` with
     ``cos`` / ``sin [T, D]`` (one k-only pass of ``siq_rope_bwd``)."""
+    if _rows_usable(dk_embed, dk_embed, cos, sin):
+        return _rows_launch("siq_rope_bwd", None, dk_embed, cos, sin)[1]
     return _k_only("siq_rope_bwd", dk_embed[None], cos[None], sin[None])[0]
 
 

@@ -247,3 +247,43 @@ def test_fp32_cos_sin_is_the_promoted_rotation_rounded_once(d):
     torch.autograd.backward([oq.to(torch.bfloat16), ok.to(torch.bfloat16)], [gq, gk])
     dq, dk = R.rope_bwd(gq.transpose(1, 2), gk.transpose(1, 2), cos, sin)
     assert same(dq.transpose(1, 2), xq.grad) and same(dk.transpose(1, 2), xk.grad)
+
+
+@pytest.mark.parametrize("cs", [torch.bfloat16, torch.float32])
+def test_token_major_rows_equal_the_batched_call(cs):
+    """rope_rows_fwd / rope_rows_bwd / rotate_k_backward, which read token-major
+    rows without a batch dimension, against the batched calls: contiguous rows,
+    slices of one projection, permuted heads, rows off 16-byte alignment or
+    with strides the kernels cannot read (copied), broadcast and strided cos /
+    sin, no tokens, and operands that are refused."""
+    g = torch.Generator().manual_seed(5)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)
+
+    t, hq, hkv, d = 37, 4, 2, 64
+    qkv = rnd(t, (hq + 2 * hkv) * d)
+    odd = rnd(t, hq * d + 1)
+    pairs = [(rnd(t, hq, d), rnd(t, hkv, d)),
+             (qkv[:, :hq * d].view(t, hq, d), qkv[:, hq * d:(hq + hkv) * d].view(t, hkv, d)),
+             (rnd(hq, t, d).transpose(0, 1), rnd(hkv, t, d).transpose(0, 1)),
+             (odd[:, 1:].view(t, hq, d), rnd(t, hkv, d + 4)[..., :d]),
+             (rnd(t, hq, 2 * d)[..., ::2], rnd(t, 1, d).expand(t, hkv, d))]
+    wide = torch.randn(t, 2 * d + 2, generator=g).to(cs).to(DEV)
+    rows = [(torch.randn(t, d, generator=g).to(cs).to(DEV), torch.randn(t, d, generator=g).to(cs).to(DEV)),
+            (wide[:, :d], wide[:, 1:d + 1]), (wide[:1, :d].expand(t, d), wide[:1, d:2 * d].expand(t, d))]
+    for n, (q, k) in enumerate(pairs):
+        for m, (cos, sin) in enumerate(rows):
+            print(f"rope rows q/k {n} cos/sin {m} {cs}", flush=True)
+            for rows_fn, fn in ((R.rope_rows_fwd, R.rope_fwd), (R.rope_rows_bwd, R.rope_bwd)):
+                a, b = rows_fn(q, k, cos, sin), fn(q[None], k[None], cos[None], sin[None])
+                assert same(a[0], b[0][0]) and same(a[1], b[1][0])
+            assert same(R.rotate_k_backward(k, cos, sin), R.rope_bwd(q[None], k[None], cos[None], sin[None])[1][0])
+    q, k = pairs[0]
+    cos, sin = rows[0]
+    a = R.rope_rows_fwd(q[:0], k[:0], cos[:0], sin[:0])
+    assert a[0].shape == (0, hq, d) and a[1].shape == (0, hkv, d)
+    for bad in ((q.float(), k, cos, sin), (q, k[:-1], cos, sin), (q, k, cos[:-1], sin[:-1]), (q, k, cos, sin.half()),
+                (q, k[..., :32], cos, sin), (q[0], k, cos, sin), (q.cpu(), k, cos, sin)):
+        with pytest.raises(ValueError):
+            R.rope_rows_fwd(*bad)
