@@ -121,6 +121,25 @@ struct GatherNKC {
   __device__ __forceinline__ void issue_tail(int hf, int64_t k0, int, bf16* lds, int wu, int) { issue(hf, k0, lds, wu); }
 };
 
+// Work of a launch whose reduction is split: unit = (split, tile), dealt to the
+// XCDs in contiguous runs of (split, J tile, I tile), I fastest (block b runs on
+// XCD b % 8).  Every XCD gets the same number of units, whatever the number of
+// tiles -- tiles dealt out alone left XCDs idle while others ran two rounds of
+// 32 workgroups (4 tiles of 40 splits: 40 workgroups on four XCDs) -- and the
+// tiles of one k range meet in one L2.  Measured: those 160 workgroups (one
+// 27 x 27 image) 25 -> 16 us; 96 tiles of 2 splits 60 us either way.
+__device__ __forceinline__ bool unit_of(int nI, int nJ, int splits, int& ti, int& tj, int& split) {
+  const int tiles = nI * nJ, total = tiles * splits;
+  const int per = (total + kXcds - 1) / kXcds;
+  const int k = (int)(blockIdx.x / kXcds), lin = (int)(blockIdx.x % kXcds) * per + k;
+  if (k >= per || lin >= total) return false;
+  split = lin / tiles;
+  const int tile = lin - split * tiles;
+  tj = tile / nI;
+  ti = tile - tj * nI;
+  return true;
+}
+
 struct FwdArgs {
   GOp W;            // [n, k]
   const bf16* x;
@@ -133,9 +152,8 @@ struct FwdArgs {
 
 __global__ __launch_bounds__(NT) void proj_fwd_kernel(const FwdArgs p) {
   __shared__ __align__(16) bf16 smem[SMEM];
-  int ti, tj;
-  if (!tile_of(p.nI, p.nJ, p.nI, ti, tj)) return;
-  const int split = blockIdx.y;
+  int ti, tj, split;
+  if (!unit_of(p.nI, p.nJ, p.splits, ti, tj, split)) return;
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
   const int64_t kb = split * p.kper, ke = min((int64_t)p.sh.k, kb + p.kper);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
@@ -224,9 +242,8 @@ struct DwArgs {
 
 __global__ __launch_bounds__(NT) void proj_dw_kernel(const DwArgs p) {
   __shared__ __align__(16) bf16 smem[SMEM];
-  int ti, tj;
-  if (!tile_of(p.nI, p.nJ, p.nI, ti, tj)) return;
-  const int split = blockIdx.y;
+  int ti, tj, split;
+  if (!unit_of(p.nI, p.nJ, p.splits, ti, tj, split)) return;
   const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
   const int64_t kb = split * p.kper, ke = min((int64_t)p.sh.m, kb + p.kper);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
@@ -337,7 +354,7 @@ Shuffle shuffle_of(const ProjArgs& a) {
 // Split-K factor: enough workgroups to cover the CUs once, each keeping at
 // least 4 k-steps, at most 48 splits.  A call of few tiles is bound by the
 // length of a workgroup's k loop (one 27 x 27 image, 4 tiles of 162 k-steps:
-// forward 32 us at 8 splits, 25 at 40); a call of many tiles has few splits
+// forward 32 us at 8 splits, 16 at 40); a call of many tiles has few splits
 // either way.  kMaxSplits bounds the partial sums (48 m n fp32 for at most 5
 // tiles).
 constexpr int kMaxSplits = 48;
@@ -354,7 +371,9 @@ int64_t kper_for(int64_t kdim, int splits) {
   return ((ksteps + splits - 1) / splits) * BK;
 }
 
-unsigned grid_of(int nI, int nJ) { return (unsigned)(((nI * nJ + kXcds - 1) / kXcds) * kXcds); }
+unsigned grid_of(int nI, int nJ, int splits) {
+  return (unsigned)((((int64_t)nI * nJ * splits + kXcds - 1) / kXcds) * kXcds);
+}
 
 void launch_sum(const float* part, bf16* out, int64_t elems, int splits, hipStream_t stream) {
   const int64_t nvec = elems / 8;
@@ -388,7 +407,7 @@ hipError_t proj_fwd(const ProjArgs& a, hipStream_t stream) {
   p.nJ = (int)((sh.m + BJ - 1) / BJ);
   p.splits = splits_for((int64_t)p.nI * p.nJ, sh.k, cu_count());
   p.kper = kper_for(sh.k, p.splits);
-  hipLaunchKernelGGL(proj_fwd_kernel, dim3(grid_of(p.nI, p.nJ), (unsigned)p.splits), dim3(NT), 0, stream, p);
+  hipLaunchKernelGGL(proj_fwd_kernel, dim3(grid_of(p.nI, p.nJ, p.splits)), dim3(NT), 0, stream, p);
   if (p.splits > 1) launch_sum(a.part, a.y, (int64_t)sh.m * a.n, p.splits, stream);
   return hipGetLastError();
 }
@@ -413,7 +432,7 @@ hipError_t proj_bwd(const ProjArgs& a, hipStream_t stream) {
     p.dx = a.dx;
     p.nI = (int)((sh.k + BI - 1) / BI);
     p.nJ = (int)((sh.m + BJ - 1) / BJ);
-    hipLaunchKernelGGL(proj_dx_kernel, dim3(grid_of(p.nI, p.nJ)), dim3(NT), 0, stream, p);
+    hipLaunchKernelGGL(proj_dx_kernel, dim3(grid_of(p.nI, p.nJ, 1)), dim3(NT), 0, stream, p);
   }
   if (a.dweight != nullptr) {
     DwArgs p{};
@@ -427,7 +446,7 @@ hipError_t proj_bwd(const ProjArgs& a, hipStream_t stream) {
     p.nJ = (int)((a.n + BJ - 1) / BJ);
     p.splits = splits_for((int64_t)p.nI * p.nJ, sh.m, cu_count());
     p.kper = kper_for(sh.m, p.splits);
-    hipLaunchKernelGGL(proj_dw_kernel, dim3(grid_of(p.nI, p.nJ), (unsigned)p.splits), dim3(NT), 0, stream, p);
+    hipLaunchKernelGGL(proj_dw_kernel, dim3(grid_of(p.nI, p.nJ, p.splits)), dim3(NT), 0, stream, p);
     if (p.splits > 1) launch_sum(a.part, a.dweight, a.n * sh.k, p.splits, stream);
   }
   return hipGetLastError();
