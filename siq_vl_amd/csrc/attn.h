@@ -87,7 +87,7 @@ struct AttnParams {
   bf16* dq;
   bf16* dk;
   bf16* dv;
-  float* delta;      // [hq, lse_head] rowsum(dO * O) (backward workspace)
+  float* delta;      // [hq, lse_head] -rowsum(dO * O) (backward workspace)
   float* lse2;       // [hq, lse_head] LSE * log2(e) (backward workspace)
   float* dq_acc;     // [total_q, hq, D] fp32 dQ sums of the atomic backward; nullptr: deterministic
   const SeqInfo* seq;

@@ -13,7 +13,7 @@
 //    the forward); wave g owns q rows 32 g .. 32 g + 31 with Q and dO in
 //    registers as B operands of S^T = K Q^T and dP^T = V dO^T.  Each lane
 //    also reads its row's O to form Delta = rowsum(dO o O), and the kernel
-//    publishes Delta and LSE * log2(e) for the dK/dV kernel.  K and V tiles
+//    publishes -Delta and LSE * log2(e) for the dK/dV kernel.  K and V tiles
 //    of 64 rows are double-buffered row-major in LDS and taken 32 rows at a
 //    time (operand reads one k-step ahead of the MFMAs); dQ^T += K^T dS^T reads
 //    K^T with ds_read_b64_tr_b16.
@@ -23,7 +23,7 @@
 //    every SIMD runs two waves, half a step apart.  K of the tile in LDS and V
 //    in registers are the B operands of S = Q K^T and dP = dO V^T.  A work item
 //    walks steps (q block, q-head of the GQA group) of its kv tile, with Q / dO
-//    / LSE2 / Delta in a ring of three LDS stages by direct global->LDS loads
+//    / LSE2 / -Delta in a ring of three LDS stages by direct global->LDS loads
 //    and the operand reads two k-steps ahead of the MFMAs; dV^T += dO^T P and
 //    dK^T += Q^T dS read dO^T / Q^T with ds_read_b64_tr_b16.  The two q-group
 //    waves' partial dK/dV of each kv quarter are summed through LDS.  Tiles
@@ -31,7 +31,7 @@
 //    writing fp32 sums to workspace slots,
 //  * which the partial-sum kernel adds in piece order afterwards.
 // At D = 64 the deterministic backward's dK/dV kernel is
-// attn_bwd_dkdv_w4_kernel (one wave per SIMD, K and V in registers); the
+// attn_bwd_dkdv_w4_kernel (four waves, K and V in registers); the
 // atomic backward replaces the dQ kernel with a Delta / LSE2 pass, dQ formed
 // in a dK/dV kernel of its own (attn_bwd_dkdv_atomic_kernel, all waves in
 // step), and a conversion of the fp32 sums.
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_atomic_kernel(const Attn
   constexpr int NDT = D / 32;
   constexpr int SMEM = NS * STAGE + 2 * KVTile::ELEMS;  // stages, K, V
   __shared__ __align__(16) bf16 smem[SMEM];
-  __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | delta][q] (raw, as loaded)
+  __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | -delta][q] (raw, as loaded)
   __shared__ __align__(16) bf16 dsx[BM * kDsxLd];  // dS exchange (atomic dQ)
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_atomic_kernel(const Attn
     const bf16* Qs = smem + buf * STAGE;
     const bf16* Gs = Qs + TE;
     const float* lse2 = rowv[buf][0];
-    const float* dlt = rowv[buf][1];
+    const float* ndelta = rowv[buf][1];
     const int q0 = (qb_last - step / p.n_rep) * BM;
     const int qvalid = si.q_len - q0;  // rows of this block that exist
     const bool pf = i + 1 < ns;
@@ -336,12 +336,12 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_atomic_kernel(const Attn
         const int qo = 32 * g + 16 * j + 4 * h;
         const f32x4 l0 = *reinterpret_cast<const f32x4*>(lse2 + qo);
         const f32x4 l1 = *reinterpret_cast<const f32x4*>(lse2 + qo + 8);
-        const f32x4 d0 = *reinterpret_cast<const f32x4*>(dlt + qo);
-        const f32x4 d1 = *reinterpret_cast<const f32x4*>(dlt + qo + 8);
+        const f32x4 d0 = *reinterpret_cast<const f32x4*>(ndelta + qo);
+        const f32x4 d1 = *reinterpret_cast<const f32x4*>(ndelta + qo + 8);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           s[8 * j + e] = __builtin_fmaf(s[8 * j + e], c, -(e < 4 ? l0[e] : l1[e - 4]));
-          dp[8 * j + e] -= e < 4 ? d0[e] : d1[e - 4];
+          dp[8 * j + e] += e < 4 ? d0[e] : d1[e - 4];
         }
       }
       if (32 * g + 32 > qvalid || (CAUSAL && wq0 + off < kb + 31)) {
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
   constexpr int SMEM = NS * STAGE + KTile::ELEMS;  // stages, K
   static_assert(8 * 2 * (NDT / 2) * 16 * 64 * 4 <= SMEM * 2, "dkdv_finish's exchange fits the LDS");
   __shared__ __align__(256) bf16 smem[SMEM];  // (whole rows aligned: operand addresses are formed by XOR)
-  __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | delta][q] (raw, as loaded)
+  __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | -delta][q] (raw, as loaded)
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
   const int wu = wave_uniform(tid >> 6);
@@ -634,18 +634,18 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
     // end of the sequence the exponent is -inf (P = 0, hence dS = 0)
     {
       const float* lse2 = &rowv[buf][0][32 * g + 4 * h];
-      const float* delta = lse2 + BM;
+      const float* ndelta = lse2 + BM;
       f32x4 lv[4], dl[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         lv[u] = *reinterpret_cast<const f32x4*>(lse2 + 8 * u);
-        dl[u] = *reinterpret_cast<const f32x4*>(delta + 8 * u);
+        dl[u] = *reinterpret_cast<const f32x4*>(ndelta + 8 * u);
       }
       if (late) load_k(0);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         s[r] = __builtin_fmaf(s[r], c, -lv[r >> 2][r & 3]);
-        dp[r] -= dl[r >> 2][r & 3];
+        dp[r] += dl[r >> 2][r & 3];
       }
     }
     pin_vgpr(s);
@@ -710,19 +710,25 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
   dkdv_finish<D>(p, it, hk, g, kq, lane, smem, dk, dv);
 }
 
-// dK/dV with one wave per SIMD (the deterministic backward's kernel at D =
-// 64; measured 15% faster than attn_bwd_dkdv_kernel on the SigLIP shape): one
-// workgroup = 4 waves = 128 kv rows of one kv-head, wave w owning kv rows
-// 32 w .. 32 w + 31 of the tile for the whole work item.  K and V of those
-// rows stay in registers as the B operands of S = Q K^T and dP = dO V^T (a
-// wave has the SIMD's 512 registers), and each wave accumulates dK^T / dV^T
-// over both 32-row q groups of every 64-row step, so no partial sums cross
-// waves.  The products of the two groups are interleaved (four independent
-// accumulator chains).  Q / dO / LSE2 / Delta of each step are
-// double-buffered in LDS by direct global->LDS loads, spread over the
-// previous step's S / dP products; dV^T += dO^T P and dK^T += Q^T dS read
-// dO^T / Q^T with ds_read_b64_tr_b16.  Work items, steps and split-tile slots
-// are those of attn_bwd_dkdv_kernel.
+// dK/dV at D = 64 (the deterministic backward): one workgroup = 4 waves = 128
+// kv rows of one kv-head, wave w owning kv rows 32 w .. 32 w + 31 of the tile
+// for the whole work item; two workgroups run on a CU.  K and V of those rows
+// stay in registers as the B operands of S = Q K^T and dP = dO V^T, and each
+// wave accumulates dK^T / dV^T over both 32-row q groups of every 64-row step,
+// so no partial sums cross waves.  Q / dO / LSE2 / -Delta of each step are
+// double-buffered in LDS by direct global->LDS loads, issued between the
+// previous step's products; dV^T += dO^T P and dK^T += Q^T dS read dO^T / Q^T
+// with ds_read_b64_tr_b16.  Work items, steps and split-tile slots are those
+// of attn_bwd_dkdv_kernel.
+//
+// A step is 32 products (1024 cycles of the matrix unit) and about as many
+// cycles of vector work, and what bounds it is how much of the two overlaps
+// (matrix units busy 40% of the time at 2.0 GHz).  So the order is written out:
+// one product, then two entries of the other q group's vector work, each part
+// held in place by scheduling barriers; and what a step does besides was taken
+// out of the loop (load addresses and the division of the step number into
+// block and head: 563 -> 375 instructions a step).  16 images x 1024 x 16 heads:
+// 163 -> 148 us (the address arithmetic alone gave 163 -> 159).
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_w4_kernel(const AttnParams p) {
   constexpr int BN = kBwdBN, BM = kBwdBM, NT = 256, NW = NT / 64, NS = 2;
@@ -732,7 +738,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_w4_kernel(const AttnPara
   constexpr int STAGE = 2 * TE;  // Q, dO (bf16 elements)
   constexpr int NDT = D / 32, KS = D / 16;
   __shared__ __align__(16) bf16 smem[NS * STAGE];
-  __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | delta][q] (raw, as loaded)
+  __shared__ __align__(16) float rowv[NS][2][BM];  // [stage][lse2 | -delta][q] (raw, as loaded)
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
   const int wu = wave_uniform(tid >> 6);
@@ -781,163 +787,205 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_w4_kernel(const AttnPara
     dv[i] = zero16();
   }
 
-  // steps (q block qb, q-head j of the GQA group): q blocks from the last one
+  // steps (q block, q-head j of the GQA group): q blocks from the last one
   // down, the n_rep heads inside; this item runs steps [s0, s1)
   const int qb_last = (si.q_len - 1) / BM;
   const int s0 = it.s0, ns = it.s1 - it.s0;
-  int64_t qtok = p.q_tok, qhead = p.q_head, gtok = p.do_tok, ghead = p.do_head, lhead = p.lse_head;
-  pin_sgpr(qtok);
-  pin_sgpr(qhead);
-  pin_sgpr(gtok);
-  pin_sgpr(ghead);
-  pin_sgpr(lhead);
-  struct StepLoad {
-    const bf16* q;
-    const bf16* g;
-    const float* rsrc;  // LSE2 (wave 0) or Delta (wave 1) of the step's rows
-    int nrows, buf;
+  int q0 = (qb_last - s0 / p.n_rep) * BM, j = s0 % p.n_rep;  // the step's first q row and head
+
+  // Loads, untracked: step ln into its stage, PERW instructions a wave of Q and
+  // of dO, spread over the previous step's products; waves 0 / 1 also LSE2 /
+  // -Delta.  Their offsets are computed once, and again around the q block that
+  // is not whole; sources step by precomputed strides.
+  const bf16* qsrc = p.q + ((int64_t)si.q_start + q0) * p.q_tok + (int64_t)(hk * p.n_rep + j) * p.q_head;
+  const bf16* gsrc = p.dout + ((int64_t)si.q_start + q0) * p.do_tok + (int64_t)(hk * p.n_rep + j) * p.do_head;
+  const float* rsrc = (wu == 0 ? p.lse2 : p.delta) + (int64_t)(hk * p.n_rep + j) * p.lse_head + si.q_start + q0;
+  // to the next head; to the next block's first head
+  int64_t qstep = p.q_head, qwrap = -(p.n_rep - 1) * p.q_head - BM * p.q_tok;
+  int64_t gstep = p.do_head, gwrap = -(p.n_rep - 1) * p.do_head - BM * p.do_tok;
+  int64_t rstep = p.lse_head, rwrap = -(p.n_rep - 1) * p.lse_head - BM;
+  int n_rep = p.n_rep;
+  pin_sgpr(qstep);
+  pin_sgpr(qwrap);
+  pin_sgpr(gstep);
+  pin_sgpr(gwrap);
+  pin_sgpr(rstep);
+  pin_sgpr(rwrap);
+  pin_sgpr(n_rep);
+  uint32_t qoff[StTile::PERW], goff[StTile::PERW];
+  int nrows = si.q_len - q0, lj = j, ln = 0;
+  bool whole = false;  // the offsets are those of a whole block
+  auto load_offsets = [&]() {  // before a step's loads
+    if (whole && nrows >= BM) return;
+    st.clamped_offsets(p.q_tok, min(nrows, BM), wu, qoff);
+    st.clamped_offsets(p.do_tok, min(nrows, BM), wu, goff);
+    whole = nrows >= BM;
   };
-  auto describe = [&](int step, int buf) {
-    const int j = step % p.n_rep, qb = qb_last - step / p.n_rep;
-    const int hq = hk * p.n_rep + j;
-    const int q0 = qb * BM;
-    const int64_t r0 = si.q_start + q0;
-    const float* rb = (wu == 0 ? p.lse2 : p.delta) + (int64_t)hq * lhead + r0;
-    return StepLoad{p.q + r0 * qtok + (int64_t)hq * qhead, p.dout + r0 * gtok + (int64_t)hq * ghead, rb, si.q_len - q0,
-                    buf};
-  };
-  // instruction k < PERW: Q, PERW .. 2 PERW - 1: dO; waves 0 / 1 also stage LSE2 / Delta with k == 0
-  auto issue_k = [&](const StepLoad& l, int k) {
-    bf16* dst = smem + l.buf * STAGE;
+  auto load_k = [&](int k) {
+    bf16* dst = smem + (ln % NS) * STAGE;
     if (k < StTile::PERW)
-      st.template issue_one<true>(k, l.q, qtok, l.nrows, dst, wu);
+      dma16(qsrc, qoff[k], dst + (wu * StTile::PERW + k) * 512);
     else
-      st.template issue_one<true>(k - StTile::PERW, l.g, gtok, l.nrows, dst + TE, wu);
-    if (k == 0 && wu < 2) dma4_untracked(l.rsrc + min(lane, l.nrows - 1), &rowv[l.buf][wu][0]);
+      dma16(gsrc, goff[k - StTile::PERW], dst + TE + (wu * StTile::PERW + k - StTile::PERW) * 512);
+    if (k == 0 && wu < 2) dma4_untracked(rsrc + min(lane, nrows - 1), &rowv[ln % NS][wu][0]);
   };
   constexpr int NLD = 2 * StTile::PERW;
-  static_assert(KS % NLD == 0, "loads spread evenly over the k-steps");
-  constexpr int KPI = KS / NLD;  // S / dP k-steps per spread load instruction
+  static_assert(NLD == KS && KS == 4 && NDT == 2, "one load a k-step; eight products a phase");
+  auto loads_on = [&]() {  // after a step's loads; after the last step's, which then come once more, unread
+    if (++ln >= ns) return;
+    const bool wrap = lj + 1 == n_rep;
+    lj = wrap ? 0 : lj + 1;
+    qsrc += wrap ? qwrap : qstep;
+    gsrc += wrap ? gwrap : gstep;
+    rsrc += wrap ? rwrap : rstep;
+    nrows += wrap ? BM : 0;
+  };
 
   if (ns > 0) {
-    const StepLoad l = describe(s0, 0);
+    load_offsets();
 #pragma unroll
-    for (int k = 0; k < NLD; ++k) issue_k(l, k);
+    for (int k = 0; k < NLD; ++k) load_k(k);
+    loads_on();
   }
   wait_vmem();
   __syncthreads();
 
-  for (int i = 0; i < ns; ++i) {
-    const int step = s0 + i;
-    const int buf = i % NS;
-    const bf16* Qs = smem + buf * STAGE;
-    const bf16* Gs = Qs + TE;
-    const float* lse2 = rowv[buf][0];
-    const float* dlt = rowv[buf][1];
-    const int q0 = (qb_last - step / p.n_rep) * BM;
-    const int qvalid = si.q_len - q0;  // rows of this block that exist
-    const bool pf = i + 1 < ns;
-    const StepLoad nl = describe(step + 1, buf ^ 1);
-    // a q group contributes when it has rows and, causally, some row sees this wave's kv rows
-    auto group_active = [&](int g) {
-      return 32 * g < qvalid && kb < si.k_len && (!CAUSAL || q0 + 32 * g + 31 + off >= kb);
-    };
-    const bool act0 = group_active(0), act1 = group_active(1);
-    if (!act0 && !act1) {
-      if (pf) {
-#pragma unroll
-        for (int k = 0; k < NLD; ++k) issue_k(nl, k);
-      }
-    } else {
-      // S_g = Q_g K^T, dP_g = dO_g V^T for both q groups, interleaved; accumulator r (= 8j + i)
-      // holds q = q0 + 32 g + 16 j + 8 (i / 4) + 4 h + i % 4, kv = kvrow.  Q / dO fragments one
-      // k-step ahead of the MFMAs.
-      f32x16 s[2], dp[2];
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        s[g] = zero16();
-        dp[g] = zero16();
-      }
-      bf16x8 fq[2][2], fg[2][2];  // [buffer][group]
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        fq[0][g] = rr.read(Qs, 32 * g, 0);
-        fg[0][g] = rr.read(Gs, 32 * g, 0);
-      }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int cur = ks & 1;
-        if (pf && ks % KPI == 0) issue_k(nl, ks / KPI);
-        if (ks + 1 < KS) {
-#pragma unroll
-          for (int g = 0; g < 2; ++g) {
-            fq[cur ^ 1][g] = rr.read(Qs, 32 * g, ks + 1);
-            fg[cur ^ 1][g] = rr.read(Gs, 32 * g, ks + 1);
-          }
-        }
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          s[g] = mfma32(fq[cur][g], kreg[ks], s[g]);
-          dp[g] = mfma32(fg[cur][g], vreg[ks], dp[g]);
-        }
-      }
-      // P = exp2(S scale log2e - LSE2), dS = P (dP - Delta); masked entries (causal, past the
-      // end of the sequence) get P = 0, hence dS = 0
-      bf16x8 pb[2][2], db[2][2];  // [group][j]
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int qo = 32 * g + 16 * j + 4 * h;
-          const f32x4 l0 = *reinterpret_cast<const f32x4*>(lse2 + qo);
-          const f32x4 l1 = *reinterpret_cast<const f32x4*>(lse2 + qo + 8);
-          const f32x4 d0 = *reinterpret_cast<const f32x4*>(dlt + qo);
-          const f32x4 d1 = *reinterpret_cast<const f32x4*>(dlt + qo + 8);
-#pragma unroll
-          for (int e2 = 0; e2 < 8; ++e2) {
-            s[g][8 * j + e2] = __builtin_fmaf(s[g][8 * j + e2], c, -(e2 < 4 ? l0[e2] : l1[e2 - 4]));
-            dp[g][8 * j + e2] -= e2 < 4 ? d0[e2] : d1[e2 - 4];
-          }
-        }
-        const int wq0 = q0 + 32 * g;
-        if (32 * g + 32 > qvalid || (CAUSAL && wq0 + off < kb + 31)) {
-          const int rel = CAUSAL ? kvrow - off - wq0 - 4 * h : -(1 << 30);  // keep q offsets >= rel
-          const int lim = qvalid - 32 * g - 4 * h;                            // keep q offsets < lim
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int qoff = 8 * (r >> 2) + (r & 3);
-            s[g][r] = (qoff >= rel && qoff < lim) ? s[g][r] : -INFINITY;
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          s[g][r] = exp2f_fast(s[g][r]);
-          dp[g][r] *= s[g][r];
-        }
-        pb[g][0] = pack8(s[g], 0);
-        pb[g][1] = pack8(s[g], 8);
-        db[g][0] = pack8(dp[g], 0);
-        db[g][1] = pack8(dp[g], 8);
-      }
-      // dV^T += dO^T P, dK^T += Q^T dS over the step's 64 q rows (transposed reads one ahead)
-      constexpr int NU = 4 * NDT;  // (group, j, d-tile)
-      bf16x8 tg[2], tq[2];
-      tg[0] = tr.read(Gs, 0, 0);
-      tq[0] = tr.read(Qs, 0, 0);
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const int gj = u / NDT, dt = u % NDT, cur = u & 1;
-        if (u + 1 < NU) {
-          const int gj1 = (u + 1) / NDT, dt1 = (u + 1) % NDT;
-          tg[cur ^ 1] = tr.read(Gs, 16 * gj1, dt1);
-          tq[cur ^ 1] = tr.read(Qs, 16 * gj1, dt1);
-        }
-        dv[dt] = mfma32(tg[cur], pb[gj >> 1][gj & 1], dv[dt]);
-        dk[dt] = mfma32(tq[cur], db[gj >> 1][gj & 1], dk[dt]);
-      }
-    }
+  int i = 0;
+  // a q group contributes when it has rows and, causally, some row sees this
+  // wave's kv rows; once both do not, no later step (of earlier rows) has one
+  auto group_active = [&](int g) {
+    return 32 * g < si.q_len - q0 && kb < si.k_len && (!CAUSAL || q0 + 32 * g + 31 + off >= kb);
+  };
+  auto active = [&]() { return group_active(0) || group_active(1); };
+  auto needs_mask = [&]() { return si.q_len - q0 < BM || (CAUSAL && q0 + off < kb + 31); };
+  auto finish_step = [&]() {
+    loads_on();
+    const bool wrap = j + 1 == n_rep;
+    j = wrap ? 0 : j + 1;
+    q0 -= wrap ? BM : 0;
+    ++i;
     wait_vmem();
     __syncthreads();
+  };
+  auto step = [&](auto masked) {
+    constexpr bool MASK = decltype(masked)::value;
+    const bf16* Qs = smem + (i % NS) * STAGE;
+    const bf16* Gs = Qs + TE;
+    const float* lse2 = rowv[i % NS][0];
+    const float* ndelta = rowv[i % NS][1];
+    // S_g = Q_g K^T, dP_g = dO_g V^T - Delta for both q groups, then
+    // P = exp2(S scale log2e - LSE2), dS = P (dP - Delta) (masked entries --
+    // causal, past the end of the sequence -- get P = 0, hence dS = 0), then
+    // dV^T += dO_g^T P, dK^T += Q_g^T dS; accumulator r (= 8j + i) holds
+    // q = q0 + 32 g + 16 j + 8 (i / 4) + 4 h + i % 4, kv = kvrow.  Group 1's
+    // S / dP products are issued one by one between the parts of group 0's
+    // vector work, and group 0's dK / dV products between those of group 1's.
+    f32x16 s[2], dp[2];
+    f32x4 lv[2][4];
+    bf16x8 pb[2][2], db[2][2];  // [group][j]
+    bf16x8 fa[4], fb[4];        // operands of the products at hand
+    auto order = []() { __builtin_amdgcn_sched_barrier(0); };
+    auto start = [&](int g) {
+      s[g] = zero16();
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        lv[g][u] = *reinterpret_cast<const f32x4*>(lse2 + 32 * g + 8 * u + 4 * h);
+        const f32x4 d = *reinterpret_cast<const f32x4*>(ndelta + 32 * g + 8 * u + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dp[g][4 * u + e] = d[e];
+      }
+    };
+    auto fetch1 = [&](int g, int ks) {
+      fa[ks] = rr.read(Qs, 32 * g, ks);
+      fb[ks] = rr.read(Gs, 32 * g, ks);
+    };
+    auto fetch2 = [&](int g, int u) {
+      fa[u] = tr.read(Gs, 32 * g + 16 * (u / NDT), u % NDT);
+      fb[u] = tr.read(Qs, 32 * g + 16 * (u / NDT), u % NDT);
+    };
+    // part n (0 .. 8) of a group's vector work: two entries' exponentials, and the previous two's dS
+    auto values = [&](int g, int n) {
+      if (n < 8) {
+#pragma unroll
+        for (int r = 2 * n; r < 2 * n + 2; ++r) {
+          s[g][r] = __builtin_fmaf(s[g][r], c, -lv[g][r >> 2][r & 3]);
+          if constexpr (MASK) {
+            const int qo = q0 + 32 * g + 8 * (r >> 2) + 4 * h + (r & 3);
+            s[g][r] = (qo < si.q_len && (!CAUSAL || qo + off >= kvrow)) ? s[g][r] : -INFINITY;
+          }
+          s[g][r] = exp2f_fast(s[g][r]);
+        }
+      }
+      if (n > 0) {
+        dp[g][2 * n - 2] *= s[g][2 * n - 2];
+        dp[g][2 * n - 1] *= s[g][2 * n - 1];
+      }
+      if (n == 4 || n == 8) {
+        pb[g][n / 4 - 1] = pack8(s[g], 2 * n - 8);
+        db[g][n / 4 - 1] = pack8(dp[g], 2 * n - 8);
+      }
+    };
+    load_offsets();
+    start(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) fetch1(0, ks);
+    order();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      s[0] = mfma32(fa[ks], kreg[ks], s[0]);
+      dp[0] = mfma32(fb[ks], vreg[ks], dp[0]);
+      load_k(ks);
+      fetch1(1, ks);
+      order();
+    }
+    start(1);
+    order();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      s[1] = mfma32(fa[ks], kreg[ks], s[1]);
+      order();
+      values(0, 2 * ks);
+      order();
+      dp[1] = mfma32(fb[ks], vreg[ks], dp[1]);
+      order();
+      values(0, 2 * ks + 1);
+      fetch2(0, ks);
+      order();
+    }
+    values(0, 8);
+    order();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      dv[u % NDT] = mfma32(fa[u], pb[0][u / NDT], dv[u % NDT]);
+      order();
+      values(1, 2 * u);
+      order();
+      dk[u % NDT] = mfma32(fb[u], db[0][u / NDT], dk[u % NDT]);
+      order();
+      values(1, 2 * u + 1);
+      fetch2(1, u);
+      order();
+    }
+    values(1, 8);
+    order();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      dv[u % NDT] = mfma32(fa[u], pb[1][u / NDT], dv[u % NDT]);
+      dk[u % NDT] = mfma32(fb[u], db[1][u / NDT], dk[u % NDT]);
+    }
+    finish_step();
+  };
+  // the block that is not whole, whole blocks, the causal diagonal, and what
+  // is left to load for the other waves: loops of their own, so that no
+  // accumulator crosses a branch
+  while (i < ns && active() && needs_mask()) step(std::true_type{});
+  while (i < ns && active() && !needs_mask()) step(std::false_type{});
+  while (i < ns && active()) step(std::true_type{});
+  while (i < ns) {
+    load_offsets();
+#pragma unroll
+    for (int k = 0; k < NLD; ++k) load_k(k);
+    finish_step();
   }
 
   // A whole tile (np == 1): dK (scaled) and dV of this wave's rows as bf16; a
@@ -1141,7 +1189,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnParams p)
     gf[ks] = qvalid ? b : zero_bf16x8();
   }
   const float lse2 = qvalid ? l2 : INFINITY;
-  const float dlt = qvalid ? dsh[32 * g + l32] : 0.f;
+  const float ndlt = qvalid ? -dsh[32 * g + l32] : 0.f;
   // every wave's staged rows read: the first K / V block may overwrite them
   __syncthreads();
   if (nblk > 0) issue(0, 0);
@@ -1149,6 +1197,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnParams p)
   f32x16 dq[NDT];
 #pragma unroll
   for (int i = 0; i < NDT; ++i) dq[i] = zero16();
+  // load offsets of a whole block, computed once; the last block's (the last
+  // loaded) are replaced when it is not whole.  (Four multiplies and four
+  // selects per load before: 116 -> 113 us at 16 x 1024 x 16 x 64, 103 -> 101
+  // at 16384 packed tokens x 12 x 128.  -Delta as the initial dP accumulator,
+  // which saves the addition, gave nothing more and cost a wave per SIMD at
+  // D = 64.)
+  uint32_t koff[Tile::PERW], voff[Tile::PERW];
+  kt.clamped_offsets(p.k_tok, BN, g, koff);
+  vt.clamped_offsets(p.v_tok, BN, g, voff);
 
   wait_vmem();
   __syncthreads();
@@ -1165,12 +1222,17 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnParams p)
     const bool pf = kb + 1 < nblk;
     const int nb = (kb + 1) * BN;  // first kv row of the next block
     bf16* nx = smem + ((kb + 1) & 1) * STAGE;
+    if (pf && si.k_len - nb < BN) {
+      kt.clamped_offsets(p.k_tok, si.k_len - nb, g, koff);
+      vt.clamped_offsets(p.v_tok, si.k_len - nb, g, voff);
+    }
+    const bf16* kn = kbase + (int64_t)nb * p.k_tok;
+    const bf16* vn = vbase + (int64_t)nb * p.v_tok;
     auto issue_k = [&](int idx) {
       if (idx < Tile::PERW)
-        kt.template issue_one<true>(idx, kbase + (int64_t)nb * p.k_tok, p.k_tok, si.k_len - nb, nx, g);
+        dma16(kn, koff[idx], nx + (g * Tile::PERW + idx) * 512);
       else
-        vt.template issue_one<true>(idx - Tile::PERW, vbase + (int64_t)nb * p.v_tok, p.v_tok, si.k_len - nb, nx + TE,
-                                    g);
+        dma16(vn, voff[idx - Tile::PERW], nx + TE + (g * Tile::PERW + idx - Tile::PERW) * 512);
     };
     // the step's two 32-row kv halves in turn
 #pragma unroll
@@ -1201,7 +1263,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnParams p)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         s[r] = __builtin_fmaf(s[r], c, -lse2);
-        dp[r] -= dlt;
+        dp[r] += ndlt;
       }
       if (kw + 31 > si.k_len - 1 || (CAUSAL && kw + 31 > wq0 + off)) {
         // kv rows past the end of the sequence or after the causal limit of some row
@@ -1229,7 +1291,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnParams p)
   }
 
   if (qvalid && h == 0) {
-    p.delta[lidx] = dlt;
+    p.delta[lidx] = ndlt;
     p.lse2[lidx] = lse2;
   }
   // dq through LDS, so that it leaves as whole 256-byte rows: after the
@@ -1304,7 +1366,7 @@ __global__ __launch_bounds__(256) void attn_bwd_prep_kernel(const AttnParams p) 
     *reinterpret_cast<f32x4*>(z + 4) = f32x4{0.f, 0.f, 0.f, 0.f};
     if (c == 0) {
       const int64_t idx = (int64_t)hq * p.lse_head + row;
-      p.delta[idx] = acc;
+      p.delta[idx] = -acc;
       p.lse2[idx] = p.lse[idx] * kLog2e;
     }
   }

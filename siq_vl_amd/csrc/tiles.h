@@ -85,6 +85,13 @@ struct LdsTile {
     for (int k = 0; k < PERW; ++k) o[k] = (uint32_t)((wu * PERW + k) * RPI + lrow) * (uint32_t)stride + coff[k % PAT];
   }
 
+  // Byte offsets for a tile of nrows rows (rows past them repeat the last one).
+  __device__ __forceinline__ void clamped_offsets(int64_t stride, int nrows, int wu, uint32_t (&o)[PERW]) const {
+#pragma unroll
+    for (int k = 0; k < PERW; ++k)
+      o[k] = 2 * ((uint32_t)min((wu * PERW + k) * RPI + lrow, nrows - 1) * (uint32_t)stride + coff[k % PAT]);
+  }
+
   // A whole tile from the offsets of full_offsets, untracked (as issue<true>).
   __device__ __forceinline__ void issue_full(const bf16* gbase, const uint32_t (&o)[PERW], bf16* lds, int wu) const {
 #pragma unroll

@@ -154,3 +154,32 @@ def test_dkdv_stage_ring_at_few_steps(heads, causal):
     for name, a, b, r in zip(("dk", "dv"), got[1:], atomic[1:], ref[1:]):
         assert torch.equal(a, b), name
         assert rel(a.float().cpu().numpy(), r) <= TOL, name
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("heads", [(1, 1), (3, 1), (4, 2)])
+def test_d64_backward_at_partial_blocks(heads, causal):
+    """The D = 64 dK/dV kernel runs the q block that is not whole, the whole
+    ones, the causal diagonal and the idle steps in loops of their own, and the
+    dQ kernel replaces its load offsets for a kv block that is not whole:
+    sequences around 32, 64 and 128 rows, fewer and more queries than keys,
+    and one long enough to be cut into pieces, each against the oracle (three
+    bf16 roundings: of P or dS, of the operands, of the result)."""
+    print(f"d64 backward heads={heads} causal={causal}", flush=True)
+    hq, hkv = heads
+    lens_k = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 193, 255, 256, 257, 1500, 130, 70, 200]
+    lens_q = lens_k[:16] + [40, 190, 64]
+    g = torch.Generator().manual_seed(hq + 10)
+    tq, tk, cu_q, cu_k = sum(lens_q), sum(lens_k), offsets(lens_q), offsets(lens_k)
+    q, do = (torch.randn(tq, hq, 64, generator=g).to(torch.bfloat16) for _ in range(2))
+    k, v = (torch.randn(tk, hkv, 64, generator=g).to(torch.bfloat16) for _ in range(2))
+    ref = oa.attention_bwd(do, q, k, v, cu_q, cu_k, 0.125, causal)
+    q, k, v, do, dcu_q, dcu_k = (x.to(DEV) for x in (q, k, v, do, cu_q, cu_k))
+    out, lse = A.varlen_attn_fwd(q, k, v, dcu_q, dcu_k, 1500, 1500, 0.125, causal)
+    got = A.varlen_attn_bwd(do, q, k, v, out, lse, dcu_q, dcu_k, 1500, 1500, 0.125, causal, deterministic=True)
+    for name, a, r, cu in zip(("dq", "dk", "dv"), got, ref, (cu_q, cu_k, cu_k)):
+        a, r = a.double().cpu().numpy(), np.asarray(r, dtype=np.float64)
+        assert rel(a, r) <= TOL, name
+        for b in range(len(lens_k)):
+            x, y = a[cu[b]:cu[b + 1]], r[cu[b]:cu[b + 1]]
+            assert np.linalg.norm(x - y) <= 2 * TOL * np.linalg.norm(y) + 2**-8 * y.size**0.5, (name, b)
