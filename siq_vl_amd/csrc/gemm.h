@@ -164,6 +164,9 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt(N | (0x7 << 4) | (0xF << 8));
 }
 
+// Wait until this wave's LDS reads have returned.
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
+
 // A workgroup barrier that waits for no memory: the compiler neither moves
 // code across it nor drains the load queue at it.
 __device__ __forceinline__ void phase_barrier() {
@@ -228,7 +231,9 @@ __device__ __forceinline__ bool tile_of(int nI, int nJ, int GI, int& ti, int& tj
 //
 // Loads: a half is read in one phase (p) only; its buffer is loaded again, for
 // two steps later, in phase p + 2 (by then every wave, also one a barrier
-// behind, has passed the compute part that waits for its reads), and read six
+// behind, has passed the compute part of phase p, which ends with a wait for
+// the wave's LDS reads: those of B lower, read a phase before it is multiplied,
+// have no other; they are back by then, so it costs nothing), and read six
 // phases after that.  A wave waits, at the end of each memory part, for the
 // half that the next phase reads (all but the ten newest load instructions),
 // so the queue is never drained before the last two steps.
@@ -287,6 +292,7 @@ __device__ __forceinline__ void gemm_core_l(bf16* smem, LA& la, LB& lb, int64_t 
     }
     phase_barrier();
     read_b(b0, 0, 0);
+    wait_lds();
     if (wu >= NW / 2) phase_barrier();
     // one k-step from buffer `buf`; bl holds its lower B half on entry, bu the next step's on exit
     auto step = [&](int s, int buf, bf16x8 (&bl)[4], bf16x8 (&bu)[4]) {
@@ -297,6 +303,7 @@ __device__ __forceinline__ void gemm_core_l(bf16* smem, LA& la, LB& lb, int64_t 
         __builtin_amdgcn_s_setprio(1);
         multiply(bf, a, b);
         __builtin_amdgcn_s_setprio(0);
+        wait_lds();
         phase_barrier();
       };
       read_a(0, buf);
