@@ -673,7 +673,7 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
   const bool two = nvt_all <= 2 * p.chunk;
   const int mode = p.c0 == 0 ? (last || two ? 0 : 1) : (two ? 4 : (last ? 3 : 2));
   // tokens past the last 64-row step with a valid row are skipped (those up to
-  // it are zero padding)
+  // it are zero rows: flce_gather_kernel)
   const int64_t nv = nvt_all - p.c0;
   const int64_t ke = min(p.Ht.rows, nv > 0 ? ((nv + BK - 1) / BK) * BK : (int64_t)0);
   f32x16 acc[4][2];
@@ -817,8 +817,10 @@ __global__ __launch_bounds__(1024) void flce_compact_kernel(const int64_t* __res
 
 // The compacted operands: Hc[k] = H[rows[k]], yc[k] = y[rows[k]] and the row's
 // reference, its label logit in log2 units, for k < nvalid; zero rows,
-// ignore_index and 0 up to the next multiple of 256 (the padding the GEMM
-// tiles read); and dH = 0 on every row whose label does not count.  One wave
+// ignore_index and 0 after them, up to the next multiple of 256 and at least
+// BK - 1 of them: dW reduces over whole k-steps counted from the chunk's first
+// row, wherever that lies, so its last one reads up to BK - 1 rows past the
+// valid ones.  And dH = 0 on every row whose label does not count.  One wave
 // per row, 16 bytes per lane per step.
 __global__ __launch_bounds__(256) void flce_gather_kernel(const bf16* __restrict__ H, const bf16* __restrict__ W,
                                                           const int64_t* __restrict__ y,
@@ -828,7 +830,8 @@ __global__ __launch_bounds__(256) void flce_gather_kernel(const bf16* __restrict
                                                           int64_t* __restrict__ yc, float* __restrict__ ref,
                                                           bf16* __restrict__ dh) {
   const int lane = threadIdx.x & 63;
-  const int64_t nvec = hdim / 8, nv = *nvalid, npad = ((nv + 255) / 256) * 256;
+  const int64_t nvec = hdim / 8, nv = *nvalid;
+  const int64_t npad = min(((n + 255) / 256) * 256, max(((nv + 255) / 256) * 256, nv + BK - 1));
   const int64_t wstep = (int64_t)gridDim.x * 4;
   for (int64_t k = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); k < npad; k += wstep) {
     const bool real = k < nv;

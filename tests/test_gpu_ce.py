@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from oracle import cross_entropy as oc
+from siq_vl_amd import _lib
 from siq_vl_amd import cross_entropy as C
 from siq_vl_amd import workloads as W
 
@@ -316,3 +317,32 @@ def test_dh_ranges_and_parts(n, hdim, vocab):
         err = (dh[r0:r0 + 4096].double() - ref).abs()
         assert bool((err <= 2.0**-8 * ref.abs() + slack * mag + 1e-30)[vb].all())
     assert abs(float(loss) - total / int(count)) <= 1e-5 * abs(total / int(count))
+
+
+@pytest.mark.parametrize("n,chunk,valid", [(300, 100, 250), (600, 300, 505), (700, 300, 500), (2000, 1000, 96),
+                                           (700, 300, 600), (512, 512, 512), (90, 1, 70)])
+def test_dw_reads_no_row_that_the_call_did_not_write(n, chunk, valid):
+    """Chunks that start off the 64-row grid: dW's last k-step reaches past the
+    valid rows, there to zero rows only, whatever the workspace held before
+    (large finite values here)."""
+    hdim, vocab = 128, 520
+    h, w, y = make(n, hdim, vocab, seed=valid, ignore_frac=0.0)
+    g = torch.Generator().manual_seed(n)
+    y[torch.randperm(n, generator=g)[valid:]] = -100
+    print(f"flce workspace contents n={n} chunk={chunk} valid={valid}", flush=True)
+    L = _lib.lib()
+    hd, wd, yd = h.to(DEV), w.to(DEV), y.to(DEV)
+    dh, dw = torch.empty_like(hd), torch.empty_like(wd)
+    loss, count, bad = (torch.empty((), dtype=t, device=DEV) for t in (torch.float32, torch.int64, torch.int64))
+    nbytes = L.siq_flce_workspace_bytes(n, hdim, vocab, chunk, 1)
+    ws = torch.full((nbytes // 2,), 3.0, dtype=torch.bfloat16, device=DEV)
+    rc = L.siq_flce_fwd_bwd(hd.data_ptr(), wd.data_ptr(), yd.data_ptr(), n, hdim, vocab, -100, 0, None,
+                            loss.data_ptr(), count.data_ptr(), bad.data_ptr(), dh.data_ptr(), dw.data_ptr(), chunk,
+                            ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "siq_flce_fwd_bwd")
+    ref = oc.linear_ce(h, w, y)
+    assert int(count) == ref["count"] == valid
+    assert abs(float(loss) - ref["loss"]) <= 1e-5 * abs(ref["loss"])
+    # bf16 operands, a few roundings each; over two chunks the first one's sum is rounded besides
+    assert rel(dh.float().cpu().numpy(), ref["dh"]) <= 2.0**-7
+    assert rel(dw.float().cpu().numpy(), ref["dw"]) <= 2.0**-7
