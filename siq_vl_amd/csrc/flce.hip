@@ -486,14 +486,14 @@ struct DhArgs {
   GOp Wt;        // W [V, hdim] read as A[i = h][k = v]
   GOp E;         // [nc, V] read as B[j = tok][k = v]
   bf16* dh;      // dhidden [n, hdim]
-  float* part;   // [slots][prow][hdim] partial sums (dh_layout; none when splits == 1)
+  float* part;   // [slots][prow][hdim] partial sums (DhTiles; none when splits == 1)
   const float* f;         // [nc] row factors, label weights, labels
   const float* wt;
   const int64_t* y;
   const int32_t* rows;    // compacted row -> original row (whole batch)
   const int64_t* nvalid;
   int64_t hdim, nc, c0;
-  int nI, splits, prow;  // hdim tiles; vocab ranges; rows of a slot
+  int nI, splits, prow, run;  // hdim tiles; vocab ranges; rows of a slot; dh_run
 };
 
 // dH work: a unit is one (token tile, vocab range); its nI hdim tiles share
@@ -503,12 +503,17 @@ struct DhArgs {
 // token tile, and a last round of a few of its workgroups (32 run at a time)
 // would leave the others idle: 27 token tiles x 6 hdim tiles are 5 rounds and
 // 2 workgroups.  So the token tiles past the last whole round have their ranges
-// cut into kDhSub parts.  The cut is made on the device, from the valid rows;
-// partial sums lie in slots, splits of them for a token tile with whole ranges,
-// then kDhSub times 8 for each of the others.  With fewer ranges (more than 292
-// tiles: eight rounds or more) nothing is cut.  Measured, whole calls on one
-// card: loss, dH and dW of 16384 rows, 11455 valid, x 1536 13.31 -> 13.05 ms;
-// loss and dH of 4099 rows, 2870 valid, x 896 1.57 -> 1.50 ms.
+// cut into kDhSub parts.  With fewer ranges (more than 292 tiles: eight rounds
+// or more) nothing is cut.  Measured, whole calls on one card: loss, dH and dW
+// of 16384 rows, 11455 valid, x 1536 13.31 -> 13.05 ms; loss and dH of 4099
+// rows, 2870 valid, x 896 1.57 -> 1.50 ms.
+//
+// A row's partial sums, and with them its last bits, must not depend on the
+// caller's chunk.  So token tiles are those of the batch's counted rows, not of
+// the chunk's (a chunk that starts inside one has the rest of it), and the
+// "rounds" are those of runs of dh_run tiles, the default chunk: a tile is cut
+// or not by its place in its run and by the batch's valid-row count, on the
+// device.
 constexpr int kDhSub = 4, kXcdSlots = 32;
 // Splits of the dH vocab reduction: enough WGs to fill the chip several
 // rounds over, bounded by the size of the fp32 partial sums.
@@ -519,45 +524,80 @@ int dh_splits(int64_t hdim, int64_t chunk) {
   if (s > kXcds) s = kXcds;
   return (int)s;
 }
-struct DhLayout {
-  int nj, nfull;  // token tiles with a valid row, those with whole ranges
+// Token tiles whose E takes 2 GiB (the Python entry's default chunk).
+int dh_run(int64_t V) { return (int)std::max<int64_t>((int64_t(1) << 31) / (2 * BJ * V), 1); }
+
+// The token tiles of the rows [c0, c0 + nv), and where their partial sums lie:
+// splits slots for a tile with whole ranges, kDhSub times 8 for one with cut
+// ranges, in tile order.
+struct DhTiles {
+  int t0, t1;       // first tile, and past the last one
+  int run, nj;      // tiles of a run; of the batch
+  int full, last;   // cut tiles of a whole run, of the last one
+  __device__ __forceinline__ int cut_before(int t) const {
+    const int g = t / run, i = t - g * run, whole = nj / run;
+    return g * full + max(0, g < whole ? i - (run - full) : i - (nj - whole * run - last));
+  }
+  // units of 8 slots before tile t (8 ranges)
+  __device__ __forceinline__ int at(int t) const { return t - t0 + (kDhSub - 1) * (cut_before(t) - cut_before(t0)); }
+  __device__ __forceinline__ bool cut(int t) const { return cut_before(t + 1) > cut_before(t); }
 };
-__device__ __forceinline__ DhLayout dh_layout(int64_t nv, int nI, int splits) {
-  DhLayout L;
-  L.nj = nv > 0 ? (int)((nv + BJ - 1) / BJ) : 0;
-  const int rem = (int)(((int64_t)L.nj * nI) % kXcdSlots);
-  L.nfull = splits == kXcds ? L.nj - min(L.nj, (rem + nI - 1) / nI) : L.nj;
-  return L;
+__device__ __forceinline__ DhTiles dh_tiles(int64_t nvalid, int64_t c0, int64_t nv, int nI, int splits, int run) {
+  DhTiles T;
+  T.t0 = (int)(c0 / BJ);
+  T.t1 = nv > 0 ? (int)((c0 + nv + BJ - 1) / BJ) : T.t0;
+  T.run = run;
+  T.nj = (int)((nvalid + BJ - 1) / BJ);
+  auto cut = [&](int n) {  // the tiles past the last whole round
+    return splits == kXcds ? min(n, (int)(((int64_t)n * nI % kXcdSlots + nI - 1) / nI)) : 0;
+  };
+  T.full = cut(run);
+  T.last = cut(T.nj % run);
+  return T;
 }
-// Slots, also units, for any number of valid rows in nj token tiles.
-int64_t dh_slots(int nj, int nI, int splits) {
-  if (splits < kXcds) return (int64_t)nj * splits;
-  return (int64_t)kXcds * (nj + (int64_t)(kDhSub - 1) * std::min(nj, (kXcdSlots - 1 + nI - 1) / nI));
+// Slots, also units, that the rows [c0, c0 + nc) can need.
+int64_t dh_slots(int64_t c0, int64_t nc, int nI, int splits, int run) {
+  const int64_t t0 = c0 / BJ, t1 = (c0 + nc + BJ - 1) / BJ, tiles = t1 - t0;
+  if (splits < kXcds) return tiles * splits;
+  const int64_t cut = std::min<int64_t>(run, (kXcdSlots - 1 + nI - 1) / nI) * ((t1 - 1) / run - t0 / run + 1);
+  return kXcds * (tiles + (kDhSub - 1) * std::min(tiles, cut));
 }
 
 __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
   __shared__ __align__(16) bf16 smem[SMEM];
   const int64_t nv = min(p.nc, *p.nvalid - p.c0);
-  const DhLayout L = dh_layout(nv, p.nI, p.splits);
+  const DhTiles T = dh_tiles(*p.nvalid, p.c0, nv, p.nI, p.splits, p.run);
   const int x = (int)(blockIdx.x % kXcds), k = (int)(blockIdx.x / kXcds);
-  const int ti = k % p.nI, unit = x + kXcds * (k / p.nI), slot = unit;
+  const int ti = k % p.nI, u = k / p.nI, unit = x + kXcds * u, slot = unit;
   // k-steps of the unit's range, or part of one
   const int64_t S = (p.E.cols + BK - 1) / BK, per = (S + p.splits - 1) / p.splits;
-  int tj;
+  int t;
   int64_t sb, se;
-  if (unit < L.nfull * p.splits) {
-    tj = unit / p.splits;
-    sb = (unit - tj * p.splits) * per;
+  if (p.splits < kXcds) {
+    t = T.t0 + unit / p.splits;
+    if (t >= T.t1) return;
+    sb = (unit % p.splits) * per;
     se = min(S, sb + per);
   } else {
-    const int q = k / p.nI - L.nfull;
-    tj = L.nfull + q / kDhSub;
-    if (p.splits < kXcds || tj >= L.nj) return;
-    const int64_t sub = (per + kDhSub - 1) / kDhSub, s0 = x * per;
-    sb = s0 + (q % kDhSub) * sub;
-    se = min(min(S, s0 + per), sb + sub);
+    if (T.t1 == T.t0 || u >= T.at(T.t1)) return;
+    t = T.t0;  // the tile whose units u is among
+    for (int end = T.t1; end - t > 1;) {
+      const int mid = (t + end) / 2;
+      if (T.at(mid) <= u)
+        t = mid;
+      else
+        end = mid;
+    }
+    sb = x * per;
+    se = min(S, sb + per);
+    if (T.cut(t)) {
+      const int64_t sub = (per + kDhSub - 1) / kDhSub;
+      sb += (u - T.at(t)) * sub;
+      se = min(se, sb + sub);
+    }
   }
-  const int64_t i0 = (int64_t)ti * BI, j0 = (int64_t)tj * BJ;
+  const int64_t i0 = (int64_t)ti * BI, j0 = max((int64_t)t * BJ - p.c0, (int64_t)0);
+  const int64_t j1 = min((int64_t)(t + 1) * BJ - p.c0, nv);  // the tile's rows of the chunk: j0 .. j1 - 1
   f32x16 acc[4][2];
   // (an empty range, of a vocabulary of few steps, leaves zeros)
   gemm_core<false, true, true>(smem, p.Wt, p.E, i0, j0, sb * BK, min(p.E.cols, se * BK), acc);
@@ -567,7 +607,7 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
   for (int b = 0; b < 2; ++b) {
     const int r = wave_col(b, wj) + l32;
     const int64_t tok = j0 + r;
-    if (tok >= nv) continue;
+    if (tok >= j1) continue;
     const int64_t orow = p.splits == 1 ? p.rows[p.c0 + tok] : 0;
     const float f = p.splits == 1 ? p.f[tok] : 0.f, wt = p.splits == 1 ? p.wt[tok] : 0.f;
     const bf16* wy = p.Wt.base + (p.splits == 1 ? p.y[tok] : 0) * p.hdim;
@@ -604,14 +644,15 @@ __global__ __launch_bounds__(NT) void flce_dh_kernel(const DhArgs p) {
 __global__ __launch_bounds__(256) void flce_dh_sum_kernel(const DhArgs p) {
   constexpr int U = 4;  // partial sums in flight
   const int64_t nv = min(p.nc, *p.nvalid - p.c0);
-  const DhLayout L = dh_layout(nv, p.nI, p.splits);
+  const DhTiles T = dh_tiles(*p.nvalid, p.c0, nv, p.nI, p.splits, p.run);
   const int64_t gpr = p.hdim / 8, stride = p.prow * p.hdim;  // groups of 8 elements, hdim / 8 per row
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nv * gpr; i += (int64_t)gridDim.x * 256) {
     const int64_t r = i / gpr, col = 8 * (i - r * gpr);
-    const int tj = (int)(r / BJ), tail = tj - L.nfull;
-    const int nslots = tail < 0 ? p.splits : kDhSub * kXcds;
-    const float* src = p.part + (r - (int64_t)tj * BJ) * p.hdim + col +
-                       stride * (tail < 0 ? tj * p.splits : kXcds * (L.nfull + kDhSub * tail));
+    const int t = (int)((p.c0 + r) / BJ);
+    const int64_t j0 = max((int64_t)t * BJ - p.c0, (int64_t)0);
+    const int nslots = T.cut(t) ? kDhSub * kXcds : p.splits;
+    const int64_t slot0 = p.splits < kXcds ? (t - T.t0) * p.splits : kXcds * T.at(t);
+    const float* src = p.part + (r - j0) * p.hdim + col + stride * slot0;
     const bf16x8 l = ld_bf16x8(p.Wt.base + p.y[r] * p.hdim + col);
     f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
     for (int s = 0; s < nslots; s += U, src += U * stride) {
@@ -905,7 +946,7 @@ __global__ __launch_bounds__(256) void zero_bf16_kernel(bf16* __restrict__ x, in
 struct Layout {
   size_t invden, loss_row, mpart, spart, zy, f, wt, E, part, acc32, rows, hc, yc, ref, keys, slot, lsum, total;
   int64_t chunk, nvt;
-  int splits, prow;  // of dH: vocab ranges, rows of a slot
+  int splits, prow, run;  // of dH: vocab ranges, rows of a slot, dh_run
   int nsort;  // sorted runs of a chunk's labels (dW only)
 };
 
@@ -944,9 +985,13 @@ Layout layout(int64_t n, int64_t hdim, int64_t V, int64_t chunk, bool need_dh, b
   L.part = off;
   L.splits = dh_splits(hdim, L.chunk);
   L.prow = (int)std::min<int64_t>(L.chunk, BJ);
-  if (need_dh && L.splits > 1)
-    off += al(sizeof(float) * (size_t)(dh_slots((int)((L.chunk + BJ - 1) / BJ), (int)((hdim + BI - 1) / BI), L.splits) *
-                                       L.prow * hdim));
+  L.run = dh_run(V);
+  if (need_dh && L.splits > 1) {
+    int64_t slots = 0;
+    for (int64_t c0 = 0; c0 < nchunks * L.chunk; c0 += L.chunk)
+      slots = std::max(slots, dh_slots(c0, std::min(L.chunk, n - c0), (int)((hdim + BI - 1) / BI), L.splits, L.run));
+    off += al(sizeof(float) * (size_t)(slots * L.prow * hdim));
+  }
   L.acc32 = off;
   // the fp32 dW sum: only when the valid rows may span more than two chunks
   // (over two, the first chunk's sum is kept in dW itself)
@@ -1089,8 +1134,9 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
     dh.nI = (int)((Hd + BI - 1) / BI);
     dh.splits = L.splits;
     dh.prow = L.prow;
+    dh.run = L.run;
     {
-      const int64_t units = dh_slots((int)((nc + BJ - 1) / BJ), dh.nI, L.splits);
+      const int64_t units = dh_slots(c0, nc, dh.nI, L.splits, L.run);
       const int64_t grid = kXcds * dh.nI * ((units + kXcds - 1) / kXcds);
       hipLaunchKernelGGL(flce_dh_kernel, dim3((unsigned)grid), dim3(NT), 0, stream, dh);
     }

@@ -346,3 +346,23 @@ def test_dw_reads_no_row_that_the_call_did_not_write(n, chunk, valid):
     # bf16 operands, a few roundings each; over two chunks the first one's sum is rounded besides
     assert rel(dh.float().cpu().numpy(), ref["dh"]) <= 2.0**-7
     assert rel(dw.float().cpu().numpy(), ref["dw"]) <= 2.0**-7
+
+
+@pytest.mark.parametrize("n,hdim,vocab,chunks", [(8192, 1536, 151936, (None, 8192, 4096, 1000)),
+                                                 (3000, 896, 1032, (None, 1500, 1024, 700, 100))])
+def test_loss_and_dh_do_not_depend_on_the_chunk(n, hdim, vocab, chunks):
+    """Bitwise: the cut of dH's vocab ranges goes by the batch's token tiles,
+    also in chunks that start inside one or hold more than one run of them
+    (151936 columns: runs of 27 tiles; all chunks have 8 ranges)."""
+    g = torch.Generator(device=DEV).manual_seed(hdim)
+    h = torch.randn(n, hdim, device=DEV, generator=g).to(torch.bfloat16)
+    w = (0.05 * torch.randn(vocab, hdim, device=DEV, generator=g)).to(torch.bfloat16)
+    y = torch.randint(0, vocab, (n,), device=DEV, generator=g)
+    y[torch.rand(n, device=DEV, generator=g) < 0.1] = -100
+    want = None
+    for chunk in chunks:
+        print(f"flce chunk n={n} hdim={hdim} V={vocab} chunk={chunk}", flush=True)
+        loss, _, _, dh, _ = C.flce_fwd_bwd(h, w, y, -100, None, False, chunk)
+        want = want or (loss, dh)
+        assert torch.equal(loss, want[0])
+        assert torch.equal(dh.view(torch.int16), want[1].view(torch.int16))
