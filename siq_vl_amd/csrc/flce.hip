@@ -231,25 +231,35 @@ struct RowArgs {
   const int64_t* nvalid;
   uint64_t* keys;        // [nsort, kIdChunk] rows sorted by label
   int32_t* slot;         // [V] cleared
-  int64_t nc, nvt, V, hdim, ignore_index, c0, ldp;
+  int64_t nc, nvt, V, hdim, c0, ldp;
   int nsort;             // sorting workgroups (0 without dW)
+  int parts;             // workgroups per 64 rows
   int grads;             // 0: loss only (E was never stored)
 };
 
-// Workgroups [0, nsort) sort the chunk's labels; each of the others takes 64
-// rows.  Sixteen waves read the rows' tile sums (lane = row, so each read is
-// 256 contiguous bytes), added in a fixed order; the rest of the work is per
-// row.
-constexpr int kRowThreads = 1024, kRowRows = 64;
+// Workgroups [0, nsort) sort the chunk's labels; the others take 64 rows each,
+// `parts` workgroups the same ones.  Sixteen waves read the rows' tile sums
+// (lane = row, so each read is 256 contiguous bytes), added in a fixed order;
+// that, and what is per row, every part does for itself.  What is per element
+// (E of the rows with redone tiles, H scaled by f) is divided over the parts:
+// few rows would otherwise leave it to a few CUs.  About as many workgroups as
+// CUs (twice as many: up to 5% slower where rows are redone).  Measured, loss
+// and dH, all rows redone, against one workgroup per 64 rows that took a row's
+// tiles and its E one after the other: 512 x 1536 over 151936 columns 1.87 ->
+// 0.58 ms, 2048 x 896 2.48 -> 1.17 ms, 16384 x 1536 13.5 -> 10.6 ms; no row
+// redone: 0.52, 0.92 and 9.4 ms either way.
+constexpr int kRowThreads = 1024, kRowRows = 64, kRowGroups = 256, kRowSeg = 64;
 __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) {
-  constexpr int NWR = kRowThreads / 64;
+  constexpr int NWR = kRowThreads / 64, U = 8;
   __shared__ union {
     uint64_t sk[kIdChunk];
     struct {
-      float sum[NWR][kRowRows], mx[NWR][kRowRows], f[kRowRows], top[kRowRows];
+      float sum[NWR][kRowRows], mx[NWR][kRowRows], redone[NWR][kRowRows], f[kRowRows], top[kRowRows];
+      int list[kRowRows], n;  // the rows with redone tiles
+      float fac[kRowSeg][kRowRows];
     } r;
   } sh;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t nv = min(p.nc, *p.nvalid - p.c0);  // valid rows of the chunk
   if ((int)blockIdx.x < p.nsort) {
     const int64_t base = (int64_t)blockIdx.x * kIdChunk;
@@ -263,85 +273,129 @@ __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) 
     for (int i = tid; i < kIdChunk; i += kRowThreads) p.keys[base + i] = i < np2 ? sh.sk[i] : kNoKey;
     return;
   }
-  const int blk = (int)blockIdx.x - p.nsort, nblk = (int)gridDim.x - p.nsort;
+  const int blk = (int)blockIdx.x - p.nsort, groups = ((int)gridDim.x - p.nsort) / p.parts;
+  const int part = blk / groups;
   if (p.nsort > 0)
-    for (int64_t v = (int64_t)blk * kRowThreads + tid; v < p.V; v += (int64_t)nblk * kRowThreads) p.slot[v] = 0;
-  const int64_t r0 = (int64_t)blk * kRowRows;
+    for (int64_t v = (int64_t)blk * kRowThreads + tid; v < p.V; v += (int64_t)groups * p.parts * kRowThreads)
+      p.slot[v] = 0;
+  const int64_t r0 = (int64_t)(blk - part * groups) * kRowRows;
   if (r0 >= nv) return;
-  {
-    const int64_t row = min(r0 + lane, nv - 1);
-    const float rf = p.ref[row];
-    float sum = 0.f, mx = -INFINITY;  // of the tiles relative to ref; the redone tiles' largest reference
-    constexpr int U = 8;
-    for (int64_t t0 = w; t0 < p.nvt; t0 += NWR * U) {
-      float s[U];
+  const int64_t row = min(r0 + lane, nv - 1);
+  const float rf = p.ref[row];
+  float sum = 0.f;  // of the tiles relative to ref
+  bool redone = false;
+  for (int64_t t0 = w; t0 < p.nvt; t0 += NWR * U) {
+    float s[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) s[u] = t0 + NWR * u < p.nvt ? p.spart[(t0 + NWR * u) * p.ldp + row] : 0.f;
+    for (int u = 0; u < U; ++u) s[u] = t0 + NWR * u < p.nvt ? p.spart[(t0 + NWR * u) * p.ldp + row] : 0.f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      redone |= s[u] < 0.f;
+      sum += s[u] < 0.f ? 0.f : s[u];  // (a NaN too)
+    }
+  }
+  sh.r.sum[w][lane] = sum;
+  float top = rf;  // the reference that E has after this pass
+  if (__syncthreads_or(redone)) {
+    // redone tiles: this wave's relative to their largest reference, then everything relative to the row's
+    float mx = -INFINITY, s2 = 0.f;
+    for (int64_t t0 = w; t0 < p.nvt; t0 += NWR * U) {
+      float s[U], m[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (s[u] < 0.f)
-          mx = fmaxf(mx, p.mpart[(t0 + NWR * u) * p.ldp + row]);
-        else
-          sum += s[u];  // (a NaN too)
+        const int64_t at = min(t0 + NWR * u, p.nvt - 1) * p.ldp + row;
+        s[u] = p.spart[at];
+        m[u] = p.mpart[at];
       }
+      float top2 = mx;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        s[u] = t0 + NWR * u < p.nvt && s[u] < 0.f ? s[u] : 0.f;
+        top2 = s[u] < 0.f ? fmaxf(top2, m[u]) : top2;
+      }
+      s2 = s2 > 0.f ? s2 * exp2f_fast(mx - top2) : 0.f;
+      mx = top2;
+#pragma unroll
+      for (int u = 0; u < U; ++u) s2 -= s[u] < 0.f ? s[u] * exp2f_fast(m[u] - mx) : 0.f;
     }
-    sh.r.sum[w][lane] = sum;
     sh.r.mx[w][lane] = mx;
+    sh.r.redone[w][lane] = s2;
     __syncthreads();
-    if (w == 0) {
-      sum = sh.r.sum[0][lane];
-      mx = sh.r.mx[0][lane];
-      for (int i = 1; i < NWR; ++i) {
-        sum += sh.r.sum[i][lane];
-        mx = fmaxf(mx, sh.r.mx[i][lane]);
+    mx = sh.r.mx[0][lane];
+    for (int i = 1; i < NWR; ++i) mx = fmaxf(mx, sh.r.mx[i][lane]);
+    redone = mx > -INFINITY;
+    if (redone) top = fmaxf(rf, mx);
+  }
+  if (w == 0) {
+    sum = sh.r.sum[0][lane];
+    for (int i = 1; i < NWR; ++i) sum += sh.r.sum[i][lane];
+    if (redone) {
+      sum *= exp2f_fast(rf - top);
+      for (int i = 0; i < NWR; ++i)
+        if (sh.r.redone[i][lane] > 0.f) sum += sh.r.redone[i][lane] * exp2f_fast(sh.r.mx[i][lane] - top);
+    }
+    const float lse2 = top + __log2f(sum);
+    const bool mine = r0 + lane < nv && part == 0;
+    if (mine) p.loss_row[row] = lse2 * kLn2 - p.zy[row];
+    if (p.grads) {
+      const float g = *p.invden, f = exp2f_fast(top - lse2) * g;
+      if (mine) {
+        p.f[row] = f;
+        p.wt[row] = (exp2f_fast(__builtin_fmaf(p.zy[row], kLog2e, -lse2)) - 1.f) * g;
+        if (!redone) p.E[row * p.V + p.y[row]] = (bf16)0.f;
       }
-      float top = rf;  // the reference that E has after this pass
-      if (mx > -INFINITY) {
-        // redone tiles: everything relative to the largest reference
-        top = fmaxf(rf, mx);
-        sum *= exp2f_fast(rf - top);
-        for (int64_t t = 0; t < p.nvt; ++t) {
-          const float s = p.spart[t * p.ldp + row];
-          if (s < 0.f) sum -= s * exp2f_fast(p.mpart[t * p.ldp + row] - top);
-        }
-      }
-      const float lse2 = top + __log2f(sum);
-      const bool mine = r0 + lane < nv;
-      const int64_t y = p.y[row];
-      if (mine) p.loss_row[row] = lse2 * kLn2 - p.zy[row];
-      if (p.grads) {
-        const float g = *p.invden, f = exp2f_fast(top - lse2) * g;
-        if (mine) {
-          p.f[row] = f;
-          p.wt[row] = (exp2f_fast(__builtin_fmaf(p.zy[row], kLog2e, -lse2)) - 1.f) * g;
-          if (!(mx > -INFINITY)) p.E[row * p.V + y] = (bf16)0.f;
-        }
-        sh.r.f[lane] = f;
-        sh.r.top[lane] = mx > -INFINITY ? top : INFINITY;  // INFINITY: E is already relative to one reference
-      }
+      sh.r.f[lane] = f;
+      sh.r.top[lane] = top;
+      const uint64_t m = __ballot(redone && r0 + lane < nv);
+      if ((m >> lane) & 1) sh.r.list[__popcll(m & ((1ull << lane) - 1))] = lane;
+      if (lane == 0) sh.r.n = __popcll(m);
     }
   }
   if (!p.grads) return;
   __syncthreads();
-  const int rows = (int)min((int64_t)kRowRows, nv - r0);
-  // rows with redone tiles: E of every tile brought to the common reference (8 columns never straddle a tile)
-  for (int r = 0; r < rows; ++r) {
-    const float top = sh.r.top[r];
-    if (top == INFINITY) continue;
-    const int64_t row = r0 + r, y = p.y[row];
-    const float rf = p.ref[row];
-    for (int64_t c = tid; c < p.V / 8; c += kRowThreads) {
-      const int64_t t = c / (kVT / 8);
-      const float fv = exp2f_fast((p.spart[t * p.ldp + row] < 0.f ? p.mpart[t * p.ldp + row] : rf) - top);
-      bf16x8 x = ld_bf16x8(p.E + row * p.V + 8 * c);
+  // rows with redone tiles: E of every tile brought to the common reference (8 columns never straddle a tile);
+  // this part's tiles, kRowSeg of them at a time, four rows at once
+  constexpr int CT = 256, UE = 4;
+  const int64_t tper = (p.nvt + p.parts - 1) / p.parts, te = min(p.nvt, (part + 1) * tper);
+  for (int64_t tb = part * tper; sh.r.n > 0 && tb < te; tb += kRowSeg) {
+    const int nt = (int)min((int64_t)kRowSeg, te - tb);
+    float m[kRowSeg / NWR];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = 8 * c + i == y ? (bf16)0.f : (bf16)((float)x[i] * fv);
-      st_bf16x8(p.E + row * p.V + 8 * c, x);
+    for (int u = 0; u < kRowSeg / NWR; ++u) {
+      const int64_t at = (tb + min(w + NWR * u, nt - 1)) * p.ldp + row;
+      m[u] = p.mpart[at];
+      m[u] = p.spart[at] < 0.f ? m[u] : rf;
     }
+#pragma unroll
+    for (int u = 0; u < kRowSeg / NWR; ++u) sh.r.fac[w + NWR * u][lane] = exp2f_fast(m[u] - top);
+    __syncthreads();
+    const int64_t c0 = tb * (kVT / 8);
+    const int ne = (int)(min(p.V / 8, (tb + nt) * (kVT / 8)) - c0);
+    for (int i = tid / CT; i < sh.r.n; i += kRowThreads / CT) {
+      const int r = sh.r.list[i];
+      const int64_t y = p.y[r0 + r] - 8 * c0;
+      const int ych = y >= 0 && y < 8 * ne ? (int)y / 8 : -1, yq = (int)(y & 7);  // the label's place in the segment
+      bf16* e = p.E + (r0 + r) * p.V + 8 * c0;
+      for (int cc = tid % CT; cc < ne; cc += CT * UE) {
+        bf16x8 x[UE];
+#pragma unroll
+        for (int u = 0; u < UE; ++u) x[u] = ld_bf16x8(e + 8 * min(cc + CT * u, ne - 1));
+#pragma unroll
+        for (int u = 0; u < UE; ++u) {
+          const int c = cc + CT * u;
+          if (c >= ne) break;
+          const float k = sh.r.fac[c / (kVT / 8)][r];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) x[u][q] = c == ych && q == yq ? (bf16)0.f : (bf16)((float)x[u][q] * k);
+          st_bf16x8(e + 8 * c, x[u]);
+        }
+      }
+    }
+    __syncthreads();
   }
   if (p.nsort == 0) return;
-  const int gpr = (int)(p.hdim / 8);
-  for (int i = tid; i < rows * gpr; i += kRowThreads) {
+  const int rows = (int)min((int64_t)kRowRows, nv - r0), gpr = (int)(p.hdim / 8);
+  for (int i = part * kRowThreads + tid; i < rows * gpr; i += p.parts * kRowThreads) {
     const float f = sh.r.f[i / gpr];
     bf16* hp = p.H + r0 * p.hdim + 8 * (int64_t)i;
     bf16x8 x = ld_bf16x8(hp);
@@ -1111,11 +1165,11 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
     rw.V = V;
     rw.hdim = Hd;
     rw.ldp = L.chunk;
-    rw.ignore_index = a.ignore_index;
     rw.nsort = L.nsort;
     rw.grads = grads ? 1 : 0;
-    hipLaunchKernelGGL(flce_row_kernel, dim3((unsigned)(L.nsort + (nc + kRowRows - 1) / kRowRows)), dim3(kRowThreads), 0,
-                       stream, rw);
+    const int64_t groups = (nc + kRowRows - 1) / kRowRows;
+    rw.parts = grads ? (int)std::max<int64_t>(kRowGroups / groups, 1) : 1;
+    hipLaunchKernelGGL(flce_row_kernel, dim3((unsigned)(L.nsort + groups * rw.parts)), dim3(kRowThreads), 0, stream, rw);
     if (!grads) continue;
 
     DhArgs dh{};

@@ -251,7 +251,8 @@ def test_full_size_vs_torch_fp32():
     assert bool((dh[~valid] == 0).all())
 
 
-@pytest.mark.parametrize("n,hdim,vocab,chunk", [(70, 64, 1032, 4096), (4500, 128, 1032, 4096), (700, 192, 520, 300)])
+@pytest.mark.parametrize("n,hdim,vocab,chunk", [(70, 64, 1032, 4096), (4500, 128, 1032, 4096), (700, 192, 520, 300),
+                                                (200, 64, 20008, 4096)])
 def test_row_references_and_label_terms(n, hdim, vocab, chunk):
     """Rows whose label logit is near the maximum, 2^60 below it in every tile
     or in some (their tiles are redone relative to their own maximum), labels
