@@ -34,8 +34,8 @@
 //     factor f = 2^(ref - lse) inv_den and its label weight w = (p_y - 1)
 //     inv_den; E at the label is set to zero (the label's term is added in
 //     fp32 instead); rows with redone tiles have their E brought to one
-//     reference; for dW, H's rows are scaled by f and the rows sorted by
-//     label.
+//     reference, the one that makes f a power of two; for dW, H's rows are
+//     scaled by f and the rows sorted by label.
 //  3. dH GEMM  dH_c^T = W^T E_c^T (split over the vocab), dH = f (sum over the
 //     splits) + w W[y], and
 //  4. dW GEMM  dW^T = (f H_c)^T E_c, plus the sums of w H over the rows of
@@ -44,7 +44,8 @@
 // twice, where a pass between the products read it and wrote dZ (1.5 of 14.8
 // ms at 16384 rows x 1536, V = 151936, 340 of 1970 us at 4099 x 896).  E is
 // rounded once on its way into dH (dZ was twice); in dW one rounding of E and
-// one of f H replace E's two; the label terms, which dominate both gradients,
+// one of f H replace E's two (in rows with redone tiles E is
+// rounded twice and f H not at all, as dZ was); the label terms, which dominate both gradients,
 // are exact.
 // With several chunks dW accumulates over them: in dW itself (bf16) when the
 // valid rows span two chunks, in an fp32 workspace when they span more;
@@ -254,7 +255,7 @@ __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) 
   __shared__ union {
     uint64_t sk[kIdChunk];
     struct {
-      float sum[NWR][kRowRows], mx[NWR][kRowRows], redone[NWR][kRowRows], f[kRowRows], top[kRowRows];
+      float sum[NWR][kRowRows], mx[NWR][kRowRows], redone[NWR][kRowRows], f[kRowRows], lse[kRowRows];
       int list[kRowRows], n;  // the rows with redone tiles
       float fac[kRowSeg][kRowRows];
     } r;
@@ -295,7 +296,7 @@ __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) 
     }
   }
   sh.r.sum[w][lane] = sum;
-  float top = rf;  // the reference that E has after this pass
+  float top = rf;  // the reference of the sum
   if (__syncthreads_or(redone)) {
     // redone tiles: this wave's relative to their largest reference, then everything relative to the row's
     float mx = -INFINITY, s2 = 0.f;
@@ -338,14 +339,16 @@ __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) 
     const bool mine = r0 + lane < nv && part == 0;
     if (mine) p.loss_row[row] = lse2 * kLn2 - p.zy[row];
     if (p.grads) {
-      const float g = *p.invden, f = exp2f_fast(top - lse2) * g;
+      // (a power of two in rows whose E is rounded once more below: then f H is exact)
+      const float g = *p.invden;
+      const float f = redone ? __builtin_ldexpf(1.f, __builtin_amdgcn_frexp_expf(g)) : exp2f_fast(top - lse2) * g;
       if (mine) {
         p.f[row] = f;
         p.wt[row] = (exp2f_fast(__builtin_fmaf(p.zy[row], kLog2e, -lse2)) - 1.f) * g;
         if (!redone) p.E[row * p.V + p.y[row]] = (bf16)0.f;
       }
       sh.r.f[lane] = f;
-      sh.r.top[lane] = top;
+      sh.r.lse[lane] = lse2;
       const uint64_t m = __ballot(redone && r0 + lane < nv);
       if ((m >> lane) & 1) sh.r.list[__popcll(m & ((1ull << lane) - 1))] = lane;
       if (lane == 0) sh.r.n = __popcll(m);
@@ -353,9 +356,10 @@ __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) 
   }
   if (!p.grads) return;
   __syncthreads();
-  // rows with redone tiles: E of every tile brought to the common reference (8 columns never straddle a tile);
-  // this part's tiles, kRowSeg of them at a time, four rows at once
+  // rows with redone tiles: E of every tile times what makes it the gradient over f (8 columns never straddle a
+  // tile); this part's tiles, kRowSeg of them at a time, four rows at once
   constexpr int CT = 256, UE = 4;
+  const float lse2 = sh.r.lse[lane], gm = __builtin_amdgcn_frexp_mantf(*p.invden);
   const int64_t tper = (p.nvt + p.parts - 1) / p.parts, te = min(p.nvt, (part + 1) * tper);
   for (int64_t tb = part * tper; sh.r.n > 0 && tb < te; tb += kRowSeg) {
     const int nt = (int)min((int64_t)kRowSeg, te - tb);
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) 
       m[u] = p.spart[at] < 0.f ? m[u] : rf;
     }
 #pragma unroll
-    for (int u = 0; u < kRowSeg / NWR; ++u) sh.r.fac[w + NWR * u][lane] = exp2f_fast(m[u] - top);
+    for (int u = 0; u < kRowSeg / NWR; ++u) sh.r.fac[w + NWR * u][lane] = exp2f_fast(m[u] - lse2) * gm;
     __syncthreads();
     const int64_t c0 = tb * (kVT / 8);
     const int ne = (int)(min(p.V / 8, (tb + nt) * (kVT / 8)) - c0);
