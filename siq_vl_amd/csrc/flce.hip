@@ -409,13 +409,17 @@ __global__ __launch_bounds__(kRowThreads) void flce_row_kernel(const RowArgs p) 
   }
 }
 
-// Label terms of dW: for each label of the chunk, the sum of w H over its
-// rows in fp32, in the slot of the label's first sorted key (lsum[slot],
-// slot[label] = that slot + 1).  One workgroup per key; the keys of a label
-// but its first one return at once.  Rounds of kLabelRound rows, listed one
-// per thread: wave k adds rows k, k + 4, ... of the round, eight in flight; the
-// waves' sums are added in order at the end.  Bound by the commonest label
-// (400 of 6912 rows where labels are Zipf-distributed): 77 us for 6912 rows x 1536.
+// Label terms of dW: for each label of the chunk, the sums of w H over its
+// rows in fp32, up to kLabelRound rows of one sorted run to a sum.  A sum lies
+// in the slot of its first sorted key; a label's first one is in slot[label],
+// the next one in next[its slot] (slots + 1; 0: none), so dW adds them in a
+// fixed order.  One workgroup per key, of which those that start no sum return
+// at once: a label that holds many rows has as many workgroups as sums.  (With
+// one workgroup a label, loss, dH and dW of 16384 x 320 over 32008 columns, 11455
+// rows of one label: 2.99 ms, 1.37 now; this kernel, labels Zipf-distributed,
+// 6912 of 16384 rows x 1536 a call: 54 and 38 us.)  The sum's rows are listed
+// one per thread; wave k adds rows k, k + 4, ..., eight in flight, and the
+// waves' sums are added in order at the end.
 constexpr int kLabelRound = 256;
 struct LabelArgs {
   const uint64_t* keys;  // [nsort, kIdChunk]
@@ -424,6 +428,7 @@ struct LabelArgs {
   const float* wt;       // [nc]
   float* lsum;           // [nsort * kIdChunk (rows that exist), hdim]
   int32_t* slot;         // [V]
+  int32_t* next;         // [nsort * kIdChunk]
   int64_t hdim;
   int nsort;
 };
@@ -436,33 +441,45 @@ __global__ __launch_bounds__(256) void flce_label_kernel(const LabelArgs p) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t item = blockIdx.x;
   const int c = (int)(item / kIdChunk), i = (int)(item % kIdChunk);
-  const uint64_t key = p.keys[item];
+  const uint64_t* kc = p.keys + (int64_t)c * kIdChunk;
+  const uint64_t key = kc[i];
   if (key == kNoKey) return;
   const uint32_t v = (uint32_t)(key >> 32);
-  if (i > 0 && (uint32_t)(p.keys[item - 1] >> 32) == v) return;  // not the label's first key in this chunk
-  // lane l: the label's run [first, first + len) in chunk g0 + l
-  int first = 0, incl = 0, total = 0;
-  auto runs = [&](int g0) {
-    int len = 0;
-    if (g0 + lane < p.nsort) {
-      const int2 r = id_run(p.keys + (int64_t)(g0 + lane) * kIdChunk, v);
-      first = r.x;
-      len = r.y - r.x;
+  auto same = [&](int at) { return (uint32_t)(kc[at] >> 32) == v; };
+  if (i > 0 && same(i - 1) && (i < kLabelRound || !same(i - kLabelRound))) return;  // inside the run's first round
+  // the label's runs: this one, whether an earlier one exists, and the first key of the next later one
+  int first = 0, end = 0;
+  bool earlier = false;
+  int32_t later = 0;
+  for (int g0 = 0; g0 < p.nsort && later == 0; g0 += 64) {
+    int2 r = make_int2(0, 0);
+    if (g0 + lane < p.nsort) r = id_run(p.keys + (int64_t)(g0 + lane) * kIdChunk, v);
+    const uint64_t has = __ballot(r.y > r.x);
+    const int q = c - g0;  // this run's lane
+    if (q >= 0 && q < 64) {
+      first = __builtin_amdgcn_readlane(r.x, q);
+      end = __builtin_amdgcn_readlane(r.y, q);
     }
-    incl = len;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o);
-      if (lane >= o) incl += y;
+    const uint64_t before = q >= 64 ? ~0ull : q > 0 ? (1ull << q) - 1 : 0ull;
+    earlier |= (has & before) != 0;
+    const uint64_t after = q < 0 ? has : q >= 63 ? 0ull : has & (~0ull << (q + 1));
+    if (after != 0) {
+      const int l = (int)__builtin_ctzll(after);
+      later = (int32_t)((g0 + l) * kIdChunk + __builtin_amdgcn_readlane(r.x, l)) + 1;
     }
-    total = __shfl(incl, 63);
-    return len;
-  };
-  for (int g0 = 0; g0 < c; g0 += 64) {
-    const int len = runs(g0);
-    if (__ballot(len > 0 && g0 + lane < c)) return;  // an earlier chunk holds the label
   }
-  if (tid == 0) p.slot[v] = (int32_t)item + 1;
+  if ((i - first) % kLabelRound != 0) return;
+  const int have = min(kLabelRound, end - i);
+  if (tid == 0) {
+    p.next[item] = i + kLabelRound < end ? (int32_t)item + kLabelRound + 1 : later;
+    if (i == first && !earlier) p.slot[v] = (int32_t)item + 1;
+  }
+  if (tid < have) {
+    const uint32_t k = (uint32_t)(c * kIdChunk) + (uint32_t)kc[i + tid];
+    row_sh[tid] = p.rows[k];
+    wt_sh[tid] = p.wt[k];
+  }
+  __syncthreads();
   const int64_t nvec = p.hdim / 8;
   for (int64_t p0 = 0; p0 < nvec; p0 += 64 * U) {
     float acc[U][8];
@@ -470,51 +487,32 @@ __global__ __launch_bounds__(256) void flce_label_kernel(const LabelArgs p) {
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[u][e] = 0.f;
-    for (int g0 = c; g0 < p.nsort; g0 += 64) {
-      runs(g0);
-      for (int rank0 = 0; rank0 < total; rank0 += kLabelRound) {
-        const int have = min(kLabelRound, total - rank0);
-        __syncthreads();  // the last round's list is read no more
-        // row rank0 + tid of the group's runs: in the first chunk whose inclusive count exceeds it
-        int q = 0, base = 0;
-        for (int j = 0; j < 64 && g0 + j < p.nsort; ++j) {
-          const int upto = __builtin_amdgcn_readlane(incl, j);
-          q = upto <= rank0 + tid ? j + 1 : q;
-          base = upto <= rank0 + tid ? upto : base;
+    for (int t0 = w; t0 < have; t0 += NWL * R) {
+      bf16x8 x[R][U];
+      float wr[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int t = min(t0 + NWL * r, have - 1);
+        wr[r] = wt_sh[t];
+        const bf16* src = p.H + (int64_t)row_sh[t] * p.hdim;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (p0 + 64 * u >= nvec) break;
+          const int64_t ch = min(p0 + 64 * u + lane, nvec - 1);
+          x[r][u] = ld_bf16x8(src + 8 * ch);
         }
-        const int at = __shfl(first, q & 63) + rank0 + tid - base;
-        if (tid < have) {
-          const uint32_t k = (uint32_t)((g0 + q) * kIdChunk) + (uint32_t)p.keys[(int64_t)(g0 + q) * kIdChunk + at];
-          row_sh[tid] = p.rows[k];
-          wt_sh[tid] = p.wt[k];
-        }
-        __syncthreads();
-        for (int t0 = w; t0 < have; t0 += NWL * R) {
-          bf16x8 x[R][U];
-          float wr[R];
+      }
 #pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const int t = min(t0 + NWL * r, have - 1);
-            wr[r] = wt_sh[t];
-            const bf16* src = p.H + (int64_t)row_sh[t] * p.hdim;
+      for (int r = 0; r < R; ++r) {
+        if (t0 + NWL * r >= have) break;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-              const int64_t ch = min(p0 + 64 * u + lane, nvec - 1);
-              x[r][u] = ld_bf16x8(src + 8 * ch);
-            }
-          }
+        for (int u = 0; u < U; ++u) {
+          if (p0 + 64 * u >= nvec) break;
 #pragma unroll
-          for (int r = 0; r < R; ++r) {
-            if (t0 + NWL * r >= have) break;
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-              for (int e = 0; e < 8; ++e) acc[u][e] = __builtin_fmaf(wr[r], (float)x[r][u][e], acc[u][e]);
-          }
+          for (int e = 0; e < 8; ++e) acc[u][e] = __builtin_fmaf(wr[r], (float)x[r][u][e], acc[u][e]);
         }
       }
     }
-    __syncthreads();
     if (w > 0) {
 #pragma unroll
       for (int u = 0; u < U; ++u)
@@ -536,6 +534,7 @@ __global__ __launch_bounds__(256) void flce_label_kernel(const LabelArgs p) {
         *reinterpret_cast<f32x4*>(dst + 4) = f32x4{acc[u][4], acc[u][5], acc[u][6], acc[u][7]};
       }
     }
+    __syncthreads();  // part_sh is read no more
   }
 }
 
@@ -744,6 +743,7 @@ struct DwArgs {
   GOp Ht;        // hidden rows of the chunk [nc, hdim], scaled by f, read as A[i = h][k = tok]
   GOp Et;        // E [nc, V] read as B[j = v][k = tok]
   const int32_t* slot;   // [V] label terms: row of lsum + 1, or 0
+  const int32_t* next;   // [rows] the label's next row of lsum + 1, or 0
   const float* lsum;     // [rows, hdim]
   bf16* dw;      // [V, hdim]
   float* acc32;  // [V, hdim] fp32 accumulator across chunks
@@ -783,8 +783,22 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
   for (int b = 0; b < 2; ++b) {
     const int64_t v = j0 + wave_col(b, wj) + l32;
     if (v >= p.V) continue;
-    const int sl = nv > 0 ? p.slot[v] : 0;
-    const float* lt = p.lsum + (int64_t)(sl - 1) * p.hdim;
+    for (int sl = nv > 0 ? p.slot[v] : 0; sl > 0; sl = p.next[sl - 1]) {
+      const float* lt = p.lsum + (int64_t)(sl - 1) * p.hdim + i0 + 8 * h;
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj) {
+          const int64_t ho = wave_row(a, wi) + 16 * jj;
+          if (i0 + 8 * h + ho >= p.hdim) continue;
+          const f32x4 lo = *reinterpret_cast<const f32x4*>(lt + ho), hi = *reinterpret_cast<const f32x4*>(lt + ho + 4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            acc[a][b][8 * jj + i] += lo[i];
+            acc[a][b][8 * jj + 4 + i] += hi[i];
+          }
+        }
+    }
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -796,10 +810,6 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
         for (int i = 0; i < 4; ++i) {
           lo[i] = acc[a][b][8 * jj + i];
           hi[i] = acc[a][b][8 * jj + 4 + i];
-        }
-        if (sl > 0) {
-          lo += *reinterpret_cast<const f32x4*>(lt + hh);
-          hi += *reinterpret_cast<const f32x4*>(lt + hh + 4);
         }
         float* a32 = p.acc32 + v * p.hdim + hh;
         if (mode == 2 || mode == 3) {
@@ -1002,7 +1012,7 @@ __global__ __launch_bounds__(256) void zero_bf16_kernel(bf16* __restrict__ x, in
 
 // ---------------------------------------------------------------- workspace
 struct Layout {
-  size_t invden, loss_row, mpart, spart, zy, f, wt, E, part, acc32, rows, hc, yc, ref, keys, slot, lsum, total;
+  size_t invden, loss_row, mpart, spart, zy, f, wt, E, part, acc32, rows, hc, yc, ref, keys, slot, next, lsum, total;
   int64_t chunk, nvt;
   int splits, prow, run;  // of dH: vocab ranges, rows of a slot, dh_run
   int nsort;  // sorted runs of a chunk's labels (dW only)
@@ -1068,6 +1078,8 @@ Layout layout(int64_t n, int64_t hdim, int64_t V, int64_t chunk, bool need_dh, b
   off += al(sizeof(uint64_t) * (size_t)L.nsort * kIdChunk);
   L.slot = off;
   if (need_dw) off += al(sizeof(int32_t) * (size_t)V);
+  L.next = off;
+  off += al(sizeof(int32_t) * (size_t)L.nsort * kIdChunk);
   // the label terms' sums, one row for each row of the chunk: in dH's partial sums, which are read by then
   L.lsum = L.splits > 1 ? L.part : off;
   if (need_dw && L.splits <= 1) off += al(sizeof(float) * (size_t)(L.chunk * hdim));
@@ -1103,6 +1115,7 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
   float* wrow = reinterpret_cast<float*>(ws + L.wt);
   uint64_t* keys = reinterpret_cast<uint64_t*>(ws + L.keys);
   int32_t* slot = reinterpret_cast<int32_t*>(ws + L.slot);
+  int32_t* next = reinterpret_cast<int32_t*>(ws + L.next);
   float* lsum = reinterpret_cast<float*>(ws + L.lsum);
   const int64_t V = a.vocab, Hd = a.hdim;
 
@@ -1213,6 +1226,7 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
       la.wt = wrow;
       la.lsum = lsum;
       la.slot = slot;
+      la.next = next;
       la.hdim = Hd;
       la.nsort = L.nsort;
       hipLaunchKernelGGL(flce_label_kernel, dim3((unsigned)nc), dim3(256), 0, stream, la);
@@ -1221,6 +1235,7 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
       dw.Ht = GOp{Hc, Hd, nc, Hd};
       dw.Et = GOp{E, V, nc, V};
       dw.slot = slot;
+      dw.next = next;
       dw.lsum = lsum;
       dw.dw = a.dweight;
       dw.acc32 = acc32;

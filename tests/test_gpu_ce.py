@@ -398,3 +398,36 @@ def test_redone_rows_are_rounded_no_more_often_than_others(n, peaked):
         err = float((got.double() - ref).norm() / ref.norm())
         print(f"  rel {err:.3e}", flush=True)
         assert err <= (2 if peaked else 3) ** 0.5 * 2.0**-9.2
+
+
+@pytest.mark.parametrize("n,hdim,counts", [(1500, 64, (255, 256, 257, 512, 1)), (6000, 832, (5000, 600)),
+                                           (2048, 1600, (2048,)), (140000, 64, ())])
+def test_label_terms_of_frequent_labels(n, hdim, counts):
+    """dW's label terms: labels with a sum's 256 rows and a few more or less,
+    labels that hold nearly all rows over three sorted runs, and labels spread
+    over more runs than a wave searches at once (69).  Where the softmax part is
+    small (p = 1 / 8192) a missing row shows: the error is that of bf16 operands."""
+    vocab = 8192 if n < 100000 else 520
+    g = torch.Generator(device=DEV).manual_seed(n)
+    h = torch.randn(n, hdim, device=DEV, generator=g).to(torch.bfloat16)
+    w = (0.2 / hdim**0.5 * torch.randn(vocab, hdim, device=DEV, generator=g)).to(torch.bfloat16)
+    y = torch.randint(0, vocab, (n,), device=DEV, generator=g)
+    order, at = torch.randperm(n, device=DEV, generator=g), 0
+    for i, c in enumerate(counts):
+        y[y == 9 + i] = 0
+        y[order[at:at + c]] = 9 + i
+        at += c
+    print(f"flce frequent labels n={n} hdim={hdim}", flush=True)
+    _, count, bad, _, dw = C.flce_fwd_bwd(h, w, y, -100, None, True)
+    assert int(count) == n and int(bad) == 0
+    ref = torch.zeros(vocab, hdim, dtype=torch.float64, device=DEV)
+    for r0 in range(0, n, 4096):
+        hb = h[r0:r0 + 4096].double()
+        p = torch.softmax(hb @ w.double().t(), 1)
+        p[torch.arange(hb.shape[0], device=DEV), y[r0:r0 + 4096]] -= 1.0
+        ref += (p / n).t() @ hb
+    err = (dw.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    print(f"  largest relative error of a row {float(err.max()):.2e}", flush=True)
+    assert float(err.max()) <= 2.0**-6  # (sums that nearly cancel: bf16 errors of the terms over the result)
+    again = C.flce_fwd_bwd(h, w, y, -100, None, True)[4]
+    assert torch.equal(dw.view(torch.int16), again.view(torch.int16))
