@@ -840,47 +840,25 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
 }
 
 // ---------------------------------------------------------------- scalars
-__global__ __launch_bounds__(1024) void flce_count_kernel(const int64_t* __restrict__ y, int64_t n, int64_t V,
-                                                          int64_t ignore_index, int reduction,
-                                                          const float* __restrict__ divisor, int64_t* count,
-                                                          int64_t* bad, float* invden) {
-  __shared__ long long sc[1024], sb[1024];
-  long long c = 0, b = 0;
-  for (int64_t i = threadIdx.x; i < n; i += 1024) {
-    const int64_t v = y[i];
-    if (v == ignore_index) continue;
-    if (v >= 0 && v < V) ++c;
-    else ++b;
-  }
-  sc[threadIdx.x] = c;
-  sb[threadIdx.x] = b;
-  __syncthreads();
-  for (int s = 512; s >= 1; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      sc[threadIdx.x] += sc[threadIdx.x + s];
-      sb[threadIdx.x] += sb[threadIdx.x + s];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    *count = sc[0];
-    *bad = sb[0];
-    *invden = reduction == 0 ? 1.f / (float)sc[0] : 1.f / *divisor;
-  }
-}
-
 // Valid rows in order, compacted: rows[k] = the k-th row whose label counts,
-// *nvalid = their number.  One workgroup; per round 16 chunks of 1024 labels
-// are loaded at once, each wave ballots its valid lanes, and one prefix over
-// the 256 (chunk, wave) counts places every valid row.
+// *nvalid = *count = their number; *bad = the labels out of range; *invden =
+// what the loss is multiplied by.  One workgroup; per round 16 chunks of 1024
+// labels are loaded at once, each wave ballots its valid lanes, and one prefix
+// over the 256 (chunk, wave) counts places every valid row.  (The counts had a
+// kernel of their own: one launch of a small call's ten, 5 us, and 12 us of
+// kernel time at 16384 rows.)
 __global__ __launch_bounds__(1024) void flce_compact_kernel(const int64_t* __restrict__ y, int64_t n, int64_t V,
-                                                            int64_t ignore_index, int32_t* __restrict__ rows,
-                                                            int64_t* __restrict__ nvalid) {
+                                                            int64_t ignore_index, int reduction,
+                                                            const float* __restrict__ divisor,
+                                                            int32_t* __restrict__ rows, int64_t* __restrict__ nvalid,
+                                                            int64_t* __restrict__ count, int64_t* __restrict__ bad,
+                                                            float* __restrict__ invden) {
   constexpr int CT = 1024, NWV = CT / 64, PER = 16;
   static_assert(PER * NWV == 256, "one (chunk, wave) count per lane quarter");
   __shared__ int cnt_sh[PER * NWV];  // valid rows of (chunk i, wave w) at i * NWV + w, in row order
-  __shared__ long long carry_sh;
+  __shared__ long long carry_sh, bad_sh[NWV];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  long long nbad = 0;  // of this wave
   const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;  // lanes before this one
   if (tid == 0) carry_sh = 0;
   __syncthreads();
@@ -895,6 +873,7 @@ __global__ __launch_bounds__(1024) void flce_compact_kernel(const int64_t* __res
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       m[i] = __ballot(v[i] != ignore_index && v[i] >= 0 && v[i] < V);
+      nbad += __popcll(__ballot(v[i] != ignore_index && !(v[i] >= 0 && v[i] < V)));
       if (lane == 0) cnt_sh[i * NWV + wv] = __popcll(m[i]);
     }
     __syncthreads();
@@ -921,7 +900,14 @@ __global__ __launch_bounds__(1024) void flce_compact_kernel(const int64_t* __res
     if (tid == 0) carry_sh += total;
     __syncthreads();
   }
-  if (tid == 0) *nvalid = carry_sh;
+  if (lane == 0) bad_sh[wv] = nbad;
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 1; i < NWV; ++i) nbad += bad_sh[i];
+    *nvalid = *count = carry_sh;
+    *bad = nbad;
+    *invden = reduction == 0 ? 1.f / (float)carry_sh : 1.f / *divisor;
+  }
 }
 
 // The compacted operands: Hc[k] = H[rows[k]], yc[k] = y[rows[k]] and the row's
@@ -1119,10 +1105,8 @@ hipError_t flce_run(const FlceArgs& a, hipStream_t stream) {
   float* lsum = reinterpret_cast<float*>(ws + L.lsum);
   const int64_t V = a.vocab, Hd = a.hdim;
 
-  hipLaunchKernelGGL(flce_count_kernel, dim3(1), dim3(1024), 0, stream, a.labels, a.n, V, a.ignore_index,
-                     a.reduction, a.divisor, a.count, a.bad_labels, invden);
-  hipLaunchKernelGGL(flce_compact_kernel, dim3(1), dim3(1024), 0, stream, a.labels, a.n, V, a.ignore_index, rows,
-                     nvalid);
+  hipLaunchKernelGGL(flce_compact_kernel, dim3(1), dim3(1024), 0, stream, a.labels, a.n, V, a.ignore_index,
+                     a.reduction, a.divisor, rows, nvalid, a.count, a.bad_labels, invden);
   if (a.n > 0) {
     int64_t blocks = (a.n + 3) / 4;
     if (blocks > 4096) blocks = 4096;
