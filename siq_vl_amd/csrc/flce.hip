@@ -775,15 +775,18 @@ __global__ __launch_bounds__(NT) void flce_dw_kernel(const DwArgs p) {
   // it are zero rows: flce_gather_kernel)
   const int64_t nv = nvt_all - p.c0;
   const int64_t ke = min(p.Ht.rows, nv > 0 ? ((nv + BK - 1) / BK) * BK : (int64_t)0);
-  f32x16 acc[4][2];
-  gemm_core<false, false, true>(smem, p.Ht, p.Et, i0, j0, 0, ke, acc);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5, l32 = lane & 31;
   const int wi = w & 1, wj = w >> 1;
+  int slot[2];  // of the columns' first label sum (loaded while there is a product to wait for)
+#pragma unroll
+  for (int b = 0; b < 2; ++b) slot[b] = nv > 0 ? p.slot[min(j0 + wave_col(b, wj) + l32, p.V - 1)] : 0;
+  f32x16 acc[4][2];
+  gemm_core<false, false, true>(smem, p.Ht, p.Et, i0, j0, 0, ke, acc);
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     const int64_t v = j0 + wave_col(b, wj) + l32;
     if (v >= p.V) continue;
-    for (int sl = nv > 0 ? p.slot[v] : 0; sl > 0; sl = p.next[sl - 1]) {
+    for (int sl = slot[b]; sl > 0; sl = p.next[sl - 1]) {
       const float* lt = p.lsum + (int64_t)(sl - 1) * p.hdim + i0 + 8 * h;
 #pragma unroll
       for (int a = 0; a < 4; ++a)
