@@ -289,17 +289,25 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const bf16* __restrict
 //    chunk and the later ones (chunks are in position order, so the
 //    concatenation is the stable order) and writes the row, if they are one
 //    partial sum (at most kRowsPerPartial tokens); every other wave returns at
-//    once, and the wave of an id with more tokens puts it on the hot list;
-//  * emb_hot_kernel: the ids of the hot list, a workgroup per (id, column
-//    block).  The partial sums of an id are independent, so the sixteen waves
+//    once, and the wave of an id with more tokens puts it on a list;
+//  * emb_hot_kernel: the ids of the lists, a workgroup (or, for those of few
+//    partial sums, some of its waves) per (id, column block).  The partial sums of an id are independent, so the sixteen waves
 //    form one each, all its rows in flight, and the workgroup adds them in
 //    order.  Token ids are Zipf-distributed (the commonest id of 12288 text
 //    tokens comes about 700 times), and one wave adding those rows one after
 //    the other waited for memory at each of them: 1065 us of the 1.24 ms that
 //    the splice's forward and backward took at 16384 tokens x 1536; with the
-//    hot list emb_sum takes 27 us and emb_hot 36 us.
+//    lists emb_sum takes 27 us and emb_hot 36 us.
 constexpr int kEmbChunk = kIdChunk;
 constexpr int kRowsPerPartial = 10;
+// Ids with more than one partial sum, by how many: up to 2, 4, 6 (tiers 0 to 2:
+// as many waves) or more (tier 3: a workgroup).  A tier's list holds at most
+// n / (tokens that its ids have at least) ids.
+constexpr int kTiers = 4;
+__host__ __device__ constexpr int tier_waves(int t) { return 2 * t + 2; }
+__host__ __device__ constexpr int tier_tokens(int t) { return (t == 0 ? 1 : tier_waves(t - 1)) * kRowsPerPartial + 1; }
+constexpr int kWarmTokens = tier_tokens(kTiers - 1) - 1;
+static_assert(kWarmTokens <= 64, "a lane per token");
 
 // Blocks [0, nch) sort one chunk each (after clearing that chunk's run
 // table); the other blocks zero the table gradient meanwhile, so that the
@@ -309,7 +317,7 @@ __global__ __launch_bounds__(1024) void emb_prep_kernel(const int64_t* __restric
                                                         int2* __restrict__ seg, int nch, u32x4* __restrict__ dw,
                                                         int64_t dw16, int* __restrict__ nhot) {
   __shared__ uint64_t sk[kEmbChunk];
-  if (blockIdx.x == 0 && threadIdx.x == 0) *nhot = 0;
+  if (blockIdx.x == 0 && threadIdx.x < kTiers) nhot[threadIdx.x] = 0;
   const u32x4 z = {0u, 0u, 0u, 0u};
   if ((int)blockIdx.x >= nch) {
     const int64_t stride = (int64_t)(gridDim.x - nch) * 1024;
@@ -379,14 +387,17 @@ struct HotId {
   uint32_t v;
   int c;
 };
+struct HotLists {
+  HotId* ids[kTiers];
+  int* n;  // [kTiers]
+};
 
 // The id's runs in chunks c .. c + 63 are read one per lane.  R rows x U
 // 16-byte chunks per lane are in flight together.
 template <typename T>
 __global__ __launch_bounds__(256) void emb_sum_kernel(const T* __restrict__ grad, const uint64_t* __restrict__ keys,
                                                       const int2* __restrict__ seg, int nchunks, int64_t vocab,
-                                                      int64_t hidden, T* __restrict__ dw, HotId* __restrict__ hot,
-                                                      int* __restrict__ nhot) {
+                                                      int64_t hidden, T* __restrict__ dw, HotLists hot) {
   using V = Vec16<T>;
   constexpr int E = V::E, U = 4, R = 4;
   __shared__ uint32_t tok_sh[4][kRowsPerPartial];
@@ -407,7 +418,7 @@ __global__ __launch_bounds__(256) void emb_sum_kernel(const T* __restrict__ grad
   }
   // the id's tokens (a wave's own LDS row: its writes and reads run in order)
   int cnt = 0;
-  for (int g0 = c; g0 < nchunks && cnt <= kRowsPerPartial; g0 += 64) {
+  for (int g0 = c; g0 < nchunks && cnt <= kWarmTokens; g0 += 64) {
     int2 mine = make_int2(0, 0);
     if (g0 + lane < nchunks) mine = seg[(int64_t)(g0 + lane) * vocab + v];
     const int len = mine.y - mine.x;
@@ -423,7 +434,10 @@ __global__ __launch_bounds__(256) void emb_sum_kernel(const T* __restrict__ grad
     cnt += __shfl(incl, 63);
   }
   if (cnt > kRowsPerPartial) {
-    if (lane == 0) hot[atomicAdd(nhot, 1)] = HotId{v, c};
+#pragma unroll
+    for (int t = 0; t < kTiers; ++t)
+      if (lane == 0 && cnt >= tier_tokens(t) && (t == kTiers - 1 || cnt < tier_tokens(t + 1)))
+        hot.ids[t][atomicAdd(hot.n + t, 1)] = HotId{v, c};
     return;
   }
   __builtin_amdgcn_wave_barrier();
@@ -468,27 +482,112 @@ __global__ __launch_bounds__(256) void emb_sum_kernel(const T* __restrict__ grad
 // gridDim.x).  Rounds of kHotWaves partial sums: the workgroup lists the
 // round's tokens in LDS (one thread per token), wave w sums rows
 // kRowsPerPartial w .. of the round in order, and thread j adds the round's
-// partial sums of column j in order to its running total.
+// partial sums of column j in order to its running total.  Then the ids of few
+// partial sums, as many to a workgroup as its waves are enough for, from the
+// workgroups on that the lists before left without one.  (A workgroup to each of
+// them: every id 11 times, 16384 tokens x 1536 230 us, where one wave had added
+// the rows one by one in 146; 153 now; 40000 x 2048 553, 235 and 255.  In
+// emb_sum's wave, one partial sum after the other, up to 40 rows held up the ids
+// behind them: Zipf-distributed ids 163 -> 193 us.)
 constexpr int kHotWaves = 16, kHotRound = kHotWaves * kRowsPerPartial;
+struct HotShared {
+  uint32_t* tok;  // [kHotRound]
+  float* part;    // [kHotWaves][COLS]
+  int* cnt;       // [kHotWaves]
+};
+
+// The ids of tier `t`, W = tier_waves(t) waves each; unit0: workgroups that the
+// lists before took.
+template <typename T, int TIER>
+__device__ __forceinline__ void emb_warm(const T* __restrict__ grad, const uint64_t* __restrict__ keys,
+                                         const int2* __restrict__ seg, int nchunks, int64_t vocab, int64_t hidden,
+                                         T* __restrict__ dw, const HotId* __restrict__ ids, int n,
+                                         const HotShared& sh, int& unit0) {
+  if (n == 0) return;
+  using V = Vec16<T>;
+  constexpr int E = V::E, COLS = 64 * E, W = tier_waves(TIER), IDS = kHotWaves / W, NTOK = W * kRowsPerPartial;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, group = wv / W, wq = wv % W;
+  const int64_t nvec = hidden / E, ch = (int64_t)blockIdx.y * 64 + lane, col0 = (int64_t)blockIdx.y * COLS;
+  const int units = (n + IDS - 1) / IDS, G = (int)gridDim.x;
+  for (int unit = ((int)blockIdx.x + G - unit0 % G) % G; unit < units; unit += G) {
+    const bool mine = group < IDS && unit * IDS + group < n;
+    const HotId id = ids[min(unit * IDS + group, n - 1)];
+    if (mine && wq == 0) {
+      int cnt = 0;
+      for (int g0 = id.c; g0 < nchunks; g0 += 64) {
+        int2 r = make_int2(0, 0);
+        if (g0 + lane < nchunks) r = seg[(int64_t)(g0 + lane) * vocab + id.v];
+        const int len = r.y - r.x;
+        // lane cnt + rank: token `rank` of the chunks' runs, in the first chunk whose inclusive count exceeds it
+        int q = -1, base = 0, upto = 0;
+        for (uint64_t m = __ballot(len > 0); m != 0; m &= m - 1) {
+          const int j = (int)__builtin_ctzll(m), l = __builtin_amdgcn_readlane(len, j);
+          if (q < 0 && lane >= cnt && lane - cnt < upto + l) {
+            q = j;
+            base = upto;
+          }
+          upto += l;
+        }
+        const int at = __shfl(r.x, q & 63) + lane - cnt - base;
+        if (q >= 0)
+          sh.tok[group * NTOK + lane] =
+              (uint32_t)((g0 + q) * kEmbChunk) + (uint32_t)keys[(int64_t)(g0 + q) * kEmbChunk + at];
+        cnt += upto;
+      }
+      if (lane == 0) sh.cnt[group] = cnt;
+    }
+    __syncthreads();
+    const int have = mine ? sh.cnt[group] : 0, r0 = wq * kRowsPerPartial, nr = min(kRowsPerPartial, have - r0);
+    if (nr > 0 && ch < nvec) {
+      typename V::Raw x[kRowsPerPartial];
+      float part[E];
+#pragma unroll
+      for (int r = 0; r < kRowsPerPartial; ++r)  // rows past the last one re-read it
+        x[r] = *reinterpret_cast<const typename V::Raw*>(
+            grad + (int64_t)sh.tok[group * NTOK + r0 + min(r, nr - 1)] * hidden + ch * E);
+#pragma unroll
+      for (int e = 0; e < E; ++e) part[e] = 0.f;
+#pragma unroll
+      for (int r = 0; r < kRowsPerPartial; ++r)
+        if (r < nr) V::add(part, x[r]);
+#pragma unroll
+      for (int e = 0; e < E; ++e) sh.part[wv * COLS + lane * E + e] = part[e];
+    }
+    __syncthreads();
+    const int np = (have + kRowsPerPartial - 1) / kRowsPerPartial;
+    if (mine) {
+      for (int j = tid - group * W * 64; j < COLS && col0 + j < hidden; j += 64 * W) {
+        float tot = 0.f;
+        for (int w = 0; w < np; ++w) tot += sh.part[(group * W + w) * COLS + j];
+        dw[(int64_t)id.v * hidden + col0 + j] = (T)tot;
+      }
+    }
+    __syncthreads();  // the lists and sums are read no more
+  }
+  unit0 += units;
+}
+
 template <typename T>
 __global__ __launch_bounds__(64 * kHotWaves) void emb_hot_kernel(const T* __restrict__ grad,
                                                                  const uint64_t* __restrict__ keys,
                                                                  const int2* __restrict__ seg, int nchunks,
                                                                  int64_t vocab, int64_t hidden, T* __restrict__ dw,
-                                                                 const HotId* __restrict__ hot,
-                                                                 const int* __restrict__ nhot) {
+                                                                 HotLists hot) {
   using V = Vec16<T>;
   constexpr int E = V::E, COLS = 64 * E;
   static_assert(COLS <= 64 * kHotWaves, "a thread per column");
   __shared__ uint32_t tok_sh[kHotRound];
+  __shared__ int cnt_sh[kHotWaves];
   __shared__ float part_sh[kHotWaves][COLS];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t nvec = hidden / E, ch = (int64_t)blockIdx.y * 64 + lane;
   const int64_t col = (int64_t)blockIdx.y * COLS + tid;
-  const int n = *nhot;
+  static_assert(kTiers == 4, "the lists' lengths in one load");
+  const int4 len = *reinterpret_cast<const int4*>(hot.n);
+  const int n = len.w;
   for (int k = blockIdx.x; k < n; k += gridDim.x) {
-    const uint32_t v = hot[k].v;
-    int g0 = hot[k].c;  // chunks g0 .. g0 + 63: lane l holds chunk g0 + l's run, every wave alike
+    const uint32_t v = hot.ids[kTiers - 1][k].v;
+    int g0 = hot.ids[kTiers - 1][k].c;  // chunks g0 .. g0 + 63: lane l holds chunk g0 + l's run, every wave alike
     int rank0 = 0;      // tokens of the group's runs listed so far
     int first, incl, total;
     auto group = [&]() {
@@ -553,6 +652,11 @@ __global__ __launch_bounds__(64 * kHotWaves) void emb_hot_kernel(const T* __rest
     if (tid < COLS && col < hidden) dw[(int64_t)v * hidden + col] = (T)tot;
     __syncthreads();  // part_sh and tok_sh are read no more
   }
+  const HotShared sh{tok_sh, &part_sh[0][0], cnt_sh};
+  int unit0 = n;
+  emb_warm<T, 2>(grad, keys, seg, nchunks, vocab, hidden, dw, hot.ids[2], len.z, sh, unit0);
+  emb_warm<T, 1>(grad, keys, seg, nchunks, vocab, hidden, dw, hot.ids[1], len.y, sh, unit0);
+  emb_warm<T, 0>(grad, keys, seg, nchunks, vocab, hidden, dw, hot.ids[0], len.x, sh, unit0);
 }
 
 unsigned row_blocks(int64_t n) {
@@ -579,36 +683,39 @@ hipError_t splice_fwd(const SpliceArgs& a, int32_t* image_pos, int64_t* counts, 
 }
 
 namespace {
-// workspace of the table gradient: sorted keys, run table, hot list (ids with
-// more than kRowsPerPartial tokens: at most n / (kRowsPerPartial + 1)) and its length
+// workspace of the table gradient: sorted keys, run table, the tiers' id lists and their lengths
 struct EmbLayout {
   int64_t nch;
-  size_t runs, hot, nhot, total;
+  size_t runs, hot[kTiers], nhot, total;
 };
 EmbLayout emb_layout(int64_t n, int64_t vocab) {
   EmbLayout L;
   L.nch = n > 0 ? (n + kEmbChunk - 1) / kEmbChunk : 0;
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
   L.runs = al((size_t)L.nch * kEmbChunk * sizeof(uint64_t));
-  L.hot = L.runs + al((size_t)L.nch * (size_t)vocab * sizeof(int2));
-  L.nhot = L.hot + al((size_t)(n > 0 ? n / (kRowsPerPartial + 1) + 1 : 1) * sizeof(HotId));
-  L.total = L.nhot + 256;
+  size_t off = L.runs + al((size_t)L.nch * (size_t)vocab * sizeof(int2));
+  for (int t = 0; t < kTiers; ++t) {
+    L.hot[t] = off;
+    off += al((size_t)((n > 0 ? n / tier_tokens(t) : 0) + 1) * sizeof(HotId));
+  }
+  L.nhot = off;
+  L.total = off + 256;
   return L;
 }
 
 template <typename T>
-void launch_emb_sums(const void* grad, const uint64_t* keys, const int2* seg, int nch, int64_t vocab, int64_t hidden,
-                     void* dw, HotId* hot, int* nhot, hipStream_t stream) {
+void launch_emb_sums(const void* grad, const uint64_t* keys, const int2* seg, int64_t n, int nch, int64_t vocab,
+                     int64_t hidden, void* dw, const HotLists& hot, hipStream_t stream) {
   const T* g = static_cast<const T*>(grad);
   T* out = static_cast<T*>(dw);
   const unsigned blocks = (unsigned)(((int64_t)nch * kEmbChunk + 3) / 4);
-  hipLaunchKernelGGL(emb_sum_kernel<T>, dim3(blocks), dim3(256), 0, stream, g, keys, seg, nch, vocab, hidden, out, hot,
-                     nhot);
-  // an id needs more than kRowsPerPartial tokens to be hot
-  const unsigned ids = (unsigned)std::min<int64_t>((int64_t)nch * kEmbChunk / (kRowsPerPartial + 1), 128);
+  hipLaunchKernelGGL(emb_sum_kernel<T>, dim3(blocks), dim3(256), 0, stream, g, keys, seg, nch, vocab, hidden, out, hot);
+  // no more than one workgroup for every id that can be listed
+  const unsigned ids = (unsigned)std::min<int64_t>(n / tier_tokens(0), 128);
+  if (ids == 0) return;
   const unsigned cols = (unsigned)((hidden / Vec16<T>::E + 63) / 64);
   hipLaunchKernelGGL(emb_hot_kernel<T>, dim3(ids, cols), dim3(64 * kHotWaves), 0, stream, g, keys, seg, nch, vocab, hidden,
-                     out, hot, nhot);
+                     out, hot);
 }
 }  // namespace
 
@@ -621,17 +728,18 @@ hipError_t embedding_bwd(const void* grad, const int64_t* ids, int64_t n, int64_
   char* base = static_cast<char*>(ws);
   uint64_t* keys = reinterpret_cast<uint64_t*>(base);
   int2* seg = reinterpret_cast<int2*>(base + L.runs);
-  HotId* hot = reinterpret_cast<HotId*>(base + L.hot);
-  int* nhot = reinterpret_cast<int*>(base + L.nhot);
+  HotLists hot;
+  for (int t = 0; t < kTiers; ++t) hot.ids[t] = reinterpret_cast<HotId*>(base + L.hot[t]);
+  hot.n = reinterpret_cast<int*>(base + L.nhot);
   const int64_t dw16 = vocab * hidden * (fp32 ? 4 : 2) / 16;  // hidden % 8 == 0
   const int clear_blocks = (int)std::min<int64_t>((dw16 + 1023) / 1024, 512);
   hipLaunchKernelGGL(emb_prep_kernel, dim3((unsigned)(nch + std::max(clear_blocks, 1))), dim3(1024), 0, stream, ids, n,
-                     vocab, skip0, skip1, keys, seg, nch, static_cast<u32x4*>(dw), dw16, nhot);
+                     vocab, skip0, skip1, keys, seg, nch, static_cast<u32x4*>(dw), dw16, hot.n);
   if (nch > 0) {
     if (fp32)
-      launch_emb_sums<float>(grad, keys, seg, nch, vocab, hidden, dw, hot, nhot, stream);
+      launch_emb_sums<float>(grad, keys, seg, n, nch, vocab, hidden, dw, hot, stream);
     else
-      launch_emb_sums<bf16>(grad, keys, seg, nch, vocab, hidden, dw, hot, nhot, stream);
+      launch_emb_sums<bf16>(grad, keys, seg, n, nch, vocab, hidden, dw, hot, stream);
   }
   return hipGetLastError();
 }

@@ -333,3 +333,32 @@ def test_table_gradient_of_frequent_ids_keeps_the_stated_order(hidden, dtype):
                 part = part + r
             tot = tot + part
         assert torch.equal(got[v], tot.to(dtype)), f"id {v}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden,filler", [(8, 0), (520, 0), (1032, 140000)])
+def test_table_gradient_at_the_tiers_of_frequent_ids(hidden, filler, dtype):
+    """Ids of as many tokens as each tier holds at least and at most, more ids
+    of a tier than a workgroup takes, and runs over more chunks than a wave reads
+    at once (69): bitwise the fp32 sums in the stated order."""
+    print(f"table gradient, tiers, hidden={hidden} filler={filler} {dtype}", flush=True)
+    counts = [10, 11, 12, 20, 21, 39, 40, 41, 60, 61, 62, 161] + [15] * 9 + [33] * 5 + [50] * 3
+    skip = len(counts)  # tokens of no id of interest, between the others
+    g = torch.Generator().manual_seed(hidden)
+    ids = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)] + [torch.full((max(filler, 50),), skip)])
+    ids = ids[torch.randperm(ids.numel(), generator=g)]
+    wanted = (ids != skip).nonzero().flatten()
+    rows = torch.randn(wanted.numel(), hidden, generator=g).to(dtype)
+    grad = torch.zeros(ids.numel(), hidden, dtype=dtype, device=DEV)
+    grad[wanted.to(DEV)] = rows.to(DEV)
+    got = S.embedding_bwd(grad, ids.to(DEV), skip + 2, (skip,)).cpu()
+    for v in range(skip):
+        tot = torch.zeros(hidden)
+        mine = rows[ids[wanted] == v].float()
+        for a in range(0, mine.shape[0], 10):
+            part = torch.zeros(hidden)
+            for r in mine[a:a + 10]:
+                part = part + r
+            tot = tot + part
+        assert torch.equal(got[v], tot.to(dtype)), f"id {v} ({counts[v]} tokens)"
+    assert not got[skip:].any()
