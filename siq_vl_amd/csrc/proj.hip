@@ -21,9 +21,11 @@
 //   dX       dXs^T [k][m] = W^T . dY^T (A = W read k-major, B = dY rows)
 //   dW       dW^T [k][n]  = Xs^T . dY  (A = gathered Xs read k-major, B = dY read k-major)
 // The forward and dW have few tiles at projector sizes (96 at m = 4096,
-// n = 1536, k = 4096), so their reduction is split over up to 48 workgroups
+// n = 1536, k = 4096), so their reduction may be split over up to 48 workgroups
 // per tile with fp32 partial sums added afterwards in split order
 // (deterministic).
+#include <algorithm>
+
 #include "gemm.h"
 #include "proj.h"
 
@@ -351,19 +353,36 @@ Shuffle shuffle_of(const ProjArgs& a) {
   return s;
 }
 
-// Split-K factor: enough workgroups to cover the CUs once, each keeping at
-// least 4 k-steps, at most 48 splits.  A call of few tiles is bound by the
-// length of a workgroup's k loop (one 27 x 27 image, 4 tiles of 162 k-steps:
-// forward 32 us at 8 splits, 16 at 40); a call of many tiles has few splits
-// either way.  kMaxSplits bounds the partial sums (48 m n fp32 for at most 5
-// tiles).
+// Split-K factor: the one with the least estimated time, of at most as many
+// splits as give every CU one workgroup, at least 4 k-steps each (fewer gained
+// nothing) and at most kMaxSplits (which bounds the partial sums: 48 m n fp32
+// for at most 5 tiles).  The estimate, in us: the k loop of one workgroup, its
+// measured step times its steps; with splits also the launch of the sum and its
+// ends (5), the partial sums' writing, by one CU (4 for a whole tile) or by all
+// (1.5 elements a ps), and their reading (4).  Fitted to 56 products of 16 to
+// 6144 tokens, k 768 to 10368, n 896 to 2048, each timed at up to 15 split
+// counts: 1% above the best count on average.  Both sides of the line: 3072 x
+// 768 x 896 (48 tiles of 12 steps) 22 us whole, 30 in 3 splits; dW of 512
+// tokens, 4096 x 1536 (96 tiles of 8 steps) 21 whole, 31 in 2; dW of 2048
+// tokens 53 whole, 49 in 2; one 27 x 27 image (4 tiles of 162 steps) 186 whole,
+// 34 in 8, 23 in 32.
 constexpr int kMaxSplits = 48;
-int splits_for(int64_t tiles, int64_t kdim, int cus) {
-  int64_t s = tiles > 0 ? cus / tiles : 1;
+constexpr double kFwdStep = 1.1, kDwStep = 1.35;  // us a k-step (dW reads both operands transposed)
+int splits_for(int64_t tiles, int64_t kdim, int64_t elems, double step, int cus) {
   const int64_t ksteps = (kdim + BK - 1) / BK;
-  if (s > ksteps / 4) s = ksteps / 4;
-  if (s > kMaxSplits) s = kMaxSplits;
-  return s < 1 ? 1 : (int)s;
+  const int64_t most = std::min<int64_t>(std::min<int64_t>(tiles > 0 ? cus / tiles : 1, ksteps / 4), kMaxSplits);
+  const double fill = tiles > 0 ? (double)elems / ((double)tiles * BI * BJ) : 0.0;
+  int best = 1;
+  double least = step * (double)ksteps;
+  for (int64_t s = 2; s <= most; ++s) {
+    const double sums = (double)(s * elems);
+    const double t = step * (double)((ksteps + s - 1) / s) + 5.0 + std::max(4.0 * fill, sums / 1.5e6) + sums / 4e6;
+    if (t < least) {
+      least = t;
+      best = (int)s;
+    }
+  }
+  return best;
 }
 
 int64_t kper_for(int64_t kdim, int splits) {
@@ -389,7 +408,7 @@ size_t proj_workspace_bytes(int64_t batch, int64_t side, int64_t dv, int r, int6
   const int cus = cu_count();
   const int64_t tiles_f = ((n + BI - 1) / BI) * ((m + BJ - 1) / BJ);
   const int64_t tiles_w = ((k + BI - 1) / BI) * ((n + BJ - 1) / BJ);
-  const int sf = splits_for(tiles_f, k, cus), sw = splits_for(tiles_w, m, cus);
+  const int sf = splits_for(tiles_f, k, m * n, kFwdStep, cus), sw = splits_for(tiles_w, m, n * k, kDwStep, cus);
   const int64_t f = sf > 1 ? (int64_t)sf * m * n : 0, w = sw > 1 ? (int64_t)sw * n * k : 0;
   return (size_t)((f > w ? f : w) * 4);
 }
@@ -405,7 +424,7 @@ hipError_t proj_fwd(const ProjArgs& a, hipStream_t stream) {
   p.n = a.n;
   p.nI = (int)((a.n + BI - 1) / BI);
   p.nJ = (int)((sh.m + BJ - 1) / BJ);
-  p.splits = splits_for((int64_t)p.nI * p.nJ, sh.k, cu_count());
+  p.splits = splits_for((int64_t)p.nI * p.nJ, sh.k, (int64_t)sh.m * a.n, kFwdStep, cu_count());
   p.kper = kper_for(sh.k, p.splits);
   hipLaunchKernelGGL(proj_fwd_kernel, dim3(grid_of(p.nI, p.nJ, p.splits)), dim3(NT), 0, stream, p);
   if (p.splits > 1) launch_sum(a.part, a.y, (int64_t)sh.m * a.n, p.splits, stream);
@@ -444,7 +463,7 @@ hipError_t proj_bwd(const ProjArgs& a, hipStream_t stream) {
     p.n = a.n;
     p.nI = (int)((sh.k + BI - 1) / BI);
     p.nJ = (int)((a.n + BJ - 1) / BJ);
-    p.splits = splits_for((int64_t)p.nI * p.nJ, sh.m, cu_count());
+    p.splits = splits_for((int64_t)p.nI * p.nJ, sh.m, a.n * sh.k, kDwStep, cu_count());
     p.kper = kper_for(sh.m, p.splits);
     hipLaunchKernelGGL(proj_dw_kernel, dim3(grid_of(p.nI, p.nJ, p.splits)), dim3(NT), 0, stream, p);
     if (p.splits > 1) launch_sum(a.part, a.dweight, a.n * sh.k, p.splits, stream);

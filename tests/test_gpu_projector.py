@@ -84,11 +84,11 @@ def test_gemm_core_at_few_k_steps(steps, tail):
         assert bool(((got - exact).abs() <= 2**-8 * exact.abs() + a.shape[1] * 2**-23 * mag).all())
 
 
-@pytest.mark.parametrize("side,dv,n", [(6, 1152, 40), (6, 448, 264), (30, 64, 8)])
+@pytest.mark.parametrize("side,dv,n", [(6, 1152, 40), (6, 448, 264), (30, 64, 8), (30, 192, 8), (48, 448, 264)])
 def test_many_splits_of_few_tiles(side, dv, n):
     """Few tiles, long k: the forward's reduction over up to 48 workgroups
-    (40, 15 and 2 here), dweight's over tokens likewise.  One bf16 rounding of
-    fp32 sums, as in test_gemm_core_at_few_k_steps."""
+    (33, 13, 1, 6 and 13 here), dweight's over tokens likewise (1, and none to 2
+    at 256 tokens).  One bf16 rounding of fp32 sums, as in test_gemm_core_at_few_k_steps."""
     print(f"projector splits side={side} dv={dv} n={n}", flush=True)
     x, w, dy = make(1, side, dv, 3, n, seed=n)
     y = P.proj_fwd(x.to(DEV), w.to(DEV), 3).double().cpu()[0]
