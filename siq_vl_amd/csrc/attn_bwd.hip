@@ -443,6 +443,11 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_atomic_kernel(const Attn
 // the end of their M1 of step i + 1.  V of the kv rows stays in registers (a
 // third of M1's LDS reads, which one wave per SIMD could not otherwise take at
 // the products' pace), K in LDS.
+// Items of up to kApartSteps steps, which load nothing beyond their first two
+// stages, keep all waves in step: the half step that waves 4-7 end later is
+// then all that being apart does (700 sequences of 24 tokens x 8 heads: the
+// backward 230 -> 225 us, 218 with the kernel that kept every item in step).
+constexpr int kApartSteps = 2;
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams p) {
   constexpr int BN = kBwdBN, BM = kBwdBM, NT = 512, NW = NT / 64, NS = 3;
@@ -509,6 +514,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
   const int s0 = it.s0, ns = it.s1 - it.s0;
   int q0 = (qb_last - s0 / p.n_rep) * BM, j = s0 % p.n_rep;  // the step's first q row and head
   int i = 0, buf = 0;                                        // the step, its stage
+  const bool apart = ns > kApartSteps;  // waves 4-7 run half a step behind
 
   // Loads of waves 4-7: step ln into its stage (untracked; 4 + 4 instructions
   // a wave of 4 rows each, waves 4 / 5 also LSE2 / Delta).  Instructions k
@@ -606,7 +612,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
   }
   wait_vmem();
   __syncthreads();
-  if (late) phase_barrier();
+  if (late && apart) phase_barrier();
   for (; i < ns && !active();) idle_step();
   fetch(qa0 + 2 * STAGE * buf, 0);  // (in bounds, and unused, when there is no step left)
   fetch(qa0 + 2 * STAGE * buf, 1);
@@ -705,7 +711,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
     __builtin_amdgcn_s_setprio(0);
   }
   for (; i < ns;) idle_step();
-  if (!late) phase_barrier();  // both groups have met the same number of barriers
+  if (!late && apart) phase_barrier();  // both groups have met the same number of barriers
   __syncthreads();             // every wave's last stage reads are done
   dkdv_finish<D>(p, it, hk, g, kq, lane, smem, dk, dv);
 }
