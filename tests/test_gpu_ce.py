@@ -431,3 +431,26 @@ def test_label_terms_of_frequent_labels(n, hdim, counts):
     assert float(err.max()) <= 2.0**-6  # (sums that nearly cancel: bf16 errors of the terms over the result)
     again = C.flce_fwd_bwd(h, w, y, -100, None, True)[4]
     assert torch.equal(dw.view(torch.int16), again.view(torch.int16))
+
+
+@pytest.mark.parametrize("n,chunk", [(700, 4096), (700, 256)])
+def test_dhidden_in_the_place_of_hidden(n, chunk):
+    """The C ABI with dhidden == hidden: bitwise the results of separate buffers."""
+    hdim, vocab = 128, 1032
+    h, w, y = make(n, hdim, vocab, seed=77)
+    y[::3] = 5
+    print(f"flce dhidden in place chunk={chunk}", flush=True)
+    hd, wd, yd = h.to(DEV), w.to(DEV), y.to(DEV)
+    loss, _, _, dh, dw = C.flce_fwd_bwd(hd, wd, yd, -100, None, True, chunk)
+    L = _lib.lib()
+    nbytes = L.siq_flce_workspace_bytes(n, hdim, vocab, chunk, 1)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    dw2, loss2 = torch.empty_like(wd), torch.empty_like(loss)
+    count, bad = (torch.empty((), dtype=torch.int64, device=DEV) for _ in range(2))
+    rc = L.siq_flce_fwd_bwd(hd.data_ptr(), wd.data_ptr(), yd.data_ptr(), n, hdim, vocab, -100, 0, None,
+                            loss2.data_ptr(), count.data_ptr(), bad.data_ptr(), hd.data_ptr(), dw2.data_ptr(), chunk,
+                            ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "siq_flce_fwd_bwd")
+    assert torch.equal(loss, loss2)
+    assert torch.equal(hd.view(torch.int16), dh.view(torch.int16))
+    assert torch.equal(dw2.view(torch.int16), dw.view(torch.int16))
