@@ -5,7 +5,7 @@
 // of a SIMD take turns: while one multiplies, the other reads its next
 // operands and issues loads (gemm_core_l).
 #pragma once
-#include "common.h"
+#include "lds.h"
 
 namespace siq {
 namespace gemm {
@@ -15,9 +15,6 @@ constexpr int NW = NT / 64;         // 8 waves: 2 along I x 4 along J
 constexpr int HALF = 128 * BK;      // bf16 elements of one staged operand half (16 KB)
 constexpr int SMEM = 8 * HALF;      // A lo / hi, B lo / hi, two k-steps each (128 KB)
 constexpr int kXcds = 8;
-
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
 struct GOp {
   const bf16* base;
@@ -45,22 +42,6 @@ __device__ __forceinline__ int wave_col(int b, int wj) { return 128 * b + 32 * w
 __device__ __forceinline__ int swz_kc(int r) { return (((r >> 1) & 3) << 1) | ((r >> 3) & 1); }
 __device__ __forceinline__ int swz_nkc(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
-// One wave instruction of direct global->LDS loading: lane l's 16 bytes land
-// at LDS byte lds + 16 l.  Written as inline asm so that the compiler's wait
-// insertion does not track these loads: it cannot tell the slab being read
-// from the one being loaded (both live in one LDS array) and would wait for
-// the prefetch before the first transposed read of every step.  The GEMM loop
-// orders them with the LDS reads itself (a vmcnt wait, then a barrier).  The LDS
-// address goes in m0 (one wait state after its write) and the uniform base in
-// SGPRs, which the compiler may have just written from a VALU instruction
-// (v_readfirstlane; an SGPR written by VALU and read by VMEM needs five wait
-// states): its hazard checks do not look inside the asm, so it starts with
-// s_nop 4.
-__device__ __forceinline__ void dma16(const bf16* gbase, uint32_t byte_off, const bf16* lds) {
-  const uint32_t la = (uint32_t)(uintptr_t)(lds_void*)lds;
-  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(byte_off), "s"(gbase), "{m0}"(la)
-               : "memory");
-}
 // Direct global->LDS staging of an operand half: 16 instructions of 1 KB, two
 // per wave (instruction 2 w + q; KC: rows 16 w + 8 q .. + 7, lane / 8 inside;
 // NKC: k rows 8 w + 4 q .. + 3, lane / 16 inside).  A row-major operand whose
@@ -155,27 +136,6 @@ struct HalfRead {
     return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   }
 };
-
-// Wait until at most N of this wave's loads are outstanding (they complete in
-// issue order).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 16, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt(N | (0x7 << 4) | (0xF << 8));
-}
-
-// Wait until this wave's LDS reads have returned.
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-
-// A workgroup barrier that waits for no memory: the compiler neither moves
-// code across it nor drains the load queue at it.
-__device__ __forceinline__ void phase_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-}
 
 // Zeroes the k tail of a staged B half (k >= kval) once it has landed: the
 // loader filled it by re-reading the last valid k, and the product must not

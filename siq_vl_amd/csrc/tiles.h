@@ -19,12 +19,9 @@
 // D = 128: swz(r) = 4 (r mod 4) + (r / 4 mod 4)   (bits 2-3 separate the rows)
 // D = 64:  swz(r) = 4 (r / 2 mod 2) + (r / 4 mod 4) (rows alternate bank halves)
 #pragma once
-#include "common.h"
+#include "lds.h"
 
 namespace siq {
-
-typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-typedef __attribute__((address_space(3))) void lds_void;
 
 template <int D>
 __device__ __forceinline__ int swz(int r) {
@@ -95,11 +92,7 @@ struct LdsTile {
   // A whole tile from the offsets of full_offsets, untracked (as issue<true>).
   __device__ __forceinline__ void issue_full(const bf16* gbase, const uint32_t (&o)[PERW], bf16* lds, int wu) const {
 #pragma unroll
-    for (int k = 0; k < PERW; ++k) {
-      const uint32_t la = (uint32_t)(uintptr_t)(lds_void*)(lds + (wu * PERW + k) * 512);
-      asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(o[k] << 1), "s"(gbase), "{m0}"(la)
-                   : "memory");
-    }
+    for (int k = 0; k < PERW; ++k) dma16(gbase, o[k] << 1, lds + (wu * PERW + k) * 512);
   }
 
   // Instruction k (< PERW) of this wave's share, so that a caller can spread
@@ -113,12 +106,7 @@ struct LdsTile {
     if (nrows < ROWS) r = min(r, nrows - 1);
     const uint32_t o = (uint32_t)r * st + coff[k % PAT];
     if constexpr (UNTRACKED) {
-      // lane l's 16 bytes land at LDS byte m0 + 16 l.  s_nop 4: m0 needs one wait state after its
-      // write, and the base SGPRs may have been written by a VALU instruction (an SGPR written by
-      // VALU and read by VMEM needs five), which the compiler's hazard checks do not see in asm.
-      const uint32_t la = (uint32_t)(uintptr_t)(lds_void*)(lds + i * 512);
-      asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(o << 1), "s"(gbase), "{m0}"(la)
-                   : "memory");
+      dma16(gbase, o << 1, lds + i * 512);
     } else {
       // uniform base + 32-bit byte offset: the saddr + voffset form
       __builtin_amdgcn_global_load_lds(reinterpret_cast<const char*>(gbase) + (o << 1), (lds_void*)(lds + i * 512),
@@ -232,22 +220,6 @@ struct TrRead {
   }
 };
 
-// One wave instruction of direct loading from a uniform base and this lane's
-// byte offset, untracked (as LdsTile::issue<true>, whose s_nop it shares).
-__device__ __forceinline__ void dma16(const bf16* gbase, uint32_t byte_off, const bf16* lds) {
-  const uint32_t la = (uint32_t)(uintptr_t)(lds_void*)lds;
-  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(byte_off), "s"(gbase), "{m0}"(la) : "memory");
-}
-
-// One dword per lane from gptr straight into LDS (lane l's 4 bytes land at LDS
-// byte lds + 4 l), untracked like LdsTile::issue<true>: the caller orders it
-// with wait_vmem and a barrier.  s_nop 0: m0 needs one wait state after its
-// write; the address is a VGPR pair.
-__device__ __forceinline__ void dma4_untracked(const void* gptr, const void* lds) {
-  const uint32_t la = (uint32_t)(uintptr_t)(lds_void*)lds;
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(gptr), "{m0}"(la) : "memory");
-}
-
 // Makes a wave-uniform value opaque, so the compiler keeps it in SGPRs rather
 // than re-reading it from the kernel arguments on every trip of a loop.
 template <typename T>
@@ -261,30 +233,6 @@ __device__ __forceinline__ void pin_sgpr(T& x) {
 template <typename T>
 __device__ __forceinline__ void pin_vgpr(T& x) {
   asm volatile("" : "+v"(x));
-}
-
-// Wait for this wave's outstanding global (and direct-to-LDS) loads.
-__device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-// Wait for this wave's outstanding LDS reads (lgkmcnt(0), vmcnt untouched).
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-
-// Wait until at most N of this wave's global loads are outstanding (loads
-// complete in issue order, so everything but the newest N has landed).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
-}
-
-// A workgroup barrier that waits for no memory: the compiler neither moves
-// code across it nor drains the load queue at it.
-__device__ __forceinline__ void phase_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
 }
 
 // Per-sequence extents, clamped on the device to [0, total).
