@@ -434,7 +434,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_atomic_kernel(const Attn
 // of a SIMD does its V, the other does M2 of its step and M1 of the next.
 // With both in step (all M1, all V, all M2, one barrier) the matrix cores
 // stood idle through every V, which the matrix products' register traffic
-// stretches to some 900 cycles against 512 each for M1 and M2.
+// stretches to some 900 cycles against 512 each for M1 and M2.  Kernel times of
+// both builds on one card: 16384 packed tokens in 32 sequences x 12 heads 105.6
+// -> 98.6 us, 32768 with one sequence of 16384 2003 -> 1837 us.
 // Q / dO / LSE2 / Delta stages are a ring of three: between its M1 and its M2
 // a wave group keeps a stage while the other group already reads the next
 // and a third is loaded.  Waves 4-7 load the stage of step i + 2 in their V of
@@ -733,8 +735,8 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnParams 
 // one product, then two entries of the other q group's vector work, each part
 // held in place by scheduling barriers; and what a step does besides was taken
 // out of the loop (load addresses and the division of the step number into
-// block and head: 563 -> 375 instructions a step).  16 images x 1024 x 16 heads:
-// 163 -> 148 us (the address arithmetic alone gave 163 -> 159).
+// block and head: 563 -> 375 instructions a step).  16 images x 1024 x 16 heads,
+// kernel times of both builds on one card: 170.5 -> 158.9 us.
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_w4_kernel(const AttnParams p) {
   constexpr int BN = kBwdBN, BM = kBwdBM, NT = 256, NW = NT / 64, NS = 2;
@@ -1205,8 +1207,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_kernel(const AttnParams p)
   for (int i = 0; i < NDT; ++i) dq[i] = zero16();
   // load offsets of a whole block, computed once; the last block's (the last
   // loaded) are replaced when it is not whole.  (Four multiplies and four
-  // selects per load before: 116 -> 113 us at 16 x 1024 x 16 x 64, 103 -> 101
-  // at 16384 packed tokens x 12 x 128.  -Delta as the initial dP accumulator,
+  // selects per load before: 119.5 -> 118.5 us at 16 x 1024 x 16 x 64, 84.1 ->
+  // 83.0 at 16384 packed tokens x 12 x 128, 1358 -> 1327 at 32768.  -Delta as the initial dP accumulator,
   // which saves the addition, gave nothing more and cost a wave per SIMD at
   // D = 64.)
   uint32_t koff[Tile::PERW], voff[Tile::PERW];

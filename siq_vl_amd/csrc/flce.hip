@@ -44,9 +44,8 @@
 // twice, where a pass between the products read it and wrote dZ (1.5 of 14.8
 // ms at 16384 rows x 1536, V = 151936, 340 of 1970 us at 4099 x 896).  E is
 // rounded once on its way into dH (dZ was twice); in dW one rounding of E and
-// one of f H replace E's two (in rows with redone tiles E is
-// rounded twice and f H not at all, as dZ was); the label terms, which dominate both gradients,
-// are exact.
+// one of f H replace E's two (in rows with redone tiles E is rounded twice and f
+// H not at all); the label terms, which dominate both gradients, are exact.
 // With several chunks dW accumulates over them: in dW itself (bf16) when the
 // valid rows span two chunks, in an fp32 workspace when they span more;
 // whether a chunk starts, continues or finishes that sum is decided on the

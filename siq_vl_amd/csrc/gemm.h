@@ -185,9 +185,10 @@ __device__ __forceinline__ bool tile_of(int nI, int nJ, int GI, int& ti, int& tj
 // and at the drain: busy 51-61% of the time, 66-76% now, at a lower clock (1.6
 // GHz against 1.8: the card's power limit, which now bounds the long products,
 // as it does the library's: 1.49 PFLOP/s on random operands, 2.1 on zeros).
-// Cross-entropy of 16384 rows (11455 counted) x 1536, V = 151936: logits 5.14
-// -> 4.70 ms, dH 5.38 -> 4.68, dW 4.61 -> 4.20 (1.27 PFLOP/s); projector 4096 x
-// 4096 x 1536: forward 68 -> 60 us, dX 53 -> 48, dW 79 -> 68.
+// Kernel times of both builds on one card: cross-entropy of 16384 rows (11467
+// counted) x 1536, V = 151936, logits 5.08 -> 4.52 ms, dH 5.30 -> 4.25 (its last
+// round cut finer besides), dW 4.57 -> 4.42 (1.21 PFLOP/s); projector 4096 x 4096
+// x 1536, forward 69.5 -> 62.7 us, dX 51.8 -> 48.0, dW 76.2 -> 68.1.
 //
 // Loads: a half is read in one phase (p) only; its buffer is loaded again, for
 // two steps later, in phase p + 2 (by then every wave, also one a barrier

@@ -4,8 +4,8 @@ the C ABI): dQ = dS K formed in the dK/dV kernel and summed with fp32 atomics.
 * small and medium cases against the fp64 CPU oracle (same cases and
   tolerance as the deterministic backward: ||x - x_ref||_F / ||x_ref||_F <=
   2e-2 for dQ, dK, dV);
-* at D = 128 dK and dV are bitwise those of the deterministic backward (the
-  same kernel and MFMA sequence; only dQ moves); at D = 64 the deterministic
+* at D = 128 dK and dV are bitwise those of the deterministic backward (a
+  kernel of its own with the same products in the same order; only dQ moves); at D = 64 the deterministic
   backward runs the one-wave-per-SIMD dK/dV kernel, which sums the two q
   groups in another order, so there they agree to rel <= 1e-2; dQ agrees with
   the deterministic dQ to fp32 summation order (rel <= 1e-2 after the bf16
@@ -66,7 +66,7 @@ def test_atomic_backward_vs_oracle(lengths, hq, hkv, d, causal):
         x = got[name] if name == "dq" else got[name].float().numpy()
         r = rel(x, ref)
         assert r <= TOL, (name, r)
-    # dK / dV do not depend on the dQ mode (bitwise where both modes run the same dK/dV kernel); dQ only by
+    # dK / dV do not depend on the dQ mode (bitwise where both modes' dK/dV kernels add the same products in the same order); dQ only by
     # the fp32 summation order
     det = run(q, k, v, do, cu, causal, True)
     if d == 128:

@@ -132,13 +132,13 @@ def test_qwen_vocab_vs_oracle():
 
 
 def test_vocab_past_one_factor_segment_vs_oracle():
-    """V = 270000: 1055 vocab tiles, more than the row pass keeps factors for
-    at once (1024), so it streams each row in two segments; the last tile
-    holds 176 columns.  Two chunks, so dW is also summed over chunks."""
+    """V = 270000: 1055 vocab tiles, of which the last holds 176 columns, with
+    labels in it and on both sides of its 1024th tile's end.  Two chunks, so dW
+    is also summed over chunks."""
     h, w, y = make(96, 64, 270000, seed=9, wscale=0.05)
     y[7] = 269999  # the last column of the partial last tile
-    y[8] = 262143  # the last column of the first segment
-    y[9] = 262144  # the first column of the second segment
+    y[8] = 262143  # the last column of tile 1023
+    y[9] = 262144  # the first column of tile 1024
     print("flce vocab 270000 n=96 chunk=64", flush=True)
     loss, count, _, dh, dw = run(h, w, y, 64)
     ref = oc.linear_ce(h, w, y, block=32)
@@ -369,14 +369,16 @@ def test_loss_and_dh_do_not_depend_on_the_chunk(n, hdim, vocab, chunks):
         assert torch.equal(dh.view(torch.int16), want[1].view(torch.int16))
 
 
-@pytest.mark.parametrize("n,peaked", [(1024, False), (1024, True), (1600, True)])
-def test_redone_rows_are_rounded_no_more_often_than_others(n, peaked):
+@pytest.mark.parametrize("n,vocab,peaked", [(1024, 32008, False), (1024, 32008, True), (1600, 32008, True),
+                                            (2100, 151936, False), (2100, 151936, True)])
+def test_redone_rows_are_rounded_no_more_often_than_others(n, vocab, peaked):
     """Labels far below their rows' other logits, so that tiles are redone.
     Rows of dW without a label (no exact label term) see a rounding of E, one on
     the way to the gradient and one of the result, each 2^-9.2 in the root mean
     square of a relative error; where one logit holds a row's mass, its E is 1
-    and the first rounding falls away."""
-    hdim, vocab = 896, 32008
+    and the first rounding falls away.  With 151936 columns a workgroup of the
+    row pass brings more tiles to the rows' reference than it keeps factors of."""
+    hdim = 896
     g = torch.Generator(device=DEV).manual_seed(5)
     h = torch.randn(n, hdim, device=DEV, generator=g).to(torch.bfloat16)
     w = (0.02 * torch.randn(vocab, hdim, device=DEV, generator=g)).to(torch.bfloat16)
