@@ -213,7 +213,7 @@ int siq_attn_rope_bwd_plan(const void* q_embed, const void* k, const void* v, co
  * Outputs (device): *loss fp32 scalar, *count int64 number of valid rows,
  * dhidden [n, hdim] bf16 = d loss / d hidden, dweight [vocab, hdim] bf16 =
  * d loss / d weight (may be NULL to skip it).  Ignored rows get dhidden
- * exactly 0.
+ * exactly 0.  dhidden may be the buffer of hidden.
  *
  * The logits are produced chunk_tokens rows at a time: only the softmax
  * numerators of one chunk (chunk_tokens x vocab bf16, each relative to its
@@ -222,7 +222,9 @@ int siq_attn_rope_bwd_plan(const void* q_embed, const void* k, const void* v, co
  * whose label counts (ignored rows are compacted away first).  Over two
  * chunks dweight is summed in dweight itself (the first chunk's sum rounded to
  * bf16 once); over more it is summed in an fp32 [vocab, hdim] workspace
- * buffer, which the workspace holds whenever n exceeds two chunks.
+ * buffer, which the workspace holds whenever n exceeds two chunks.  The loss
+ * does not depend on chunk_tokens, nor does dhidden between chunks of up to 292
+ * tiles of 256 rows x 256 features (bitwise).
  * ------------------------------------------------------------------------- */
 size_t siq_flce_workspace_bytes(int64_t n, int64_t hdim, int64_t vocab, int64_t chunk_tokens, int need_dweight);
 
